@@ -6,7 +6,8 @@
 //                                                          k_cell_keys, radix sort by super-cell
 //                                                          (physical order), k_gather
 //   table fill + kernel_build_hash_table                -> k_cell_keys (cell-table inserts)
-//   kernel_find_neighbours                              -> k_neighbours
+//   kernel_find_neighbours                              -> k_neighbours_wave (k_neighbours for very
+//                                                          long lists)
 //   kernel_calculate_densities + kernel_calculate_lambdas   -> k_density_lambda (one sweep)
 //   kernel_calculate_position_delta + kernel_correct_position -> k_delta_correct
 //   ... last iteration also kernel_update_position_and_velocity
@@ -382,8 +383,8 @@ __device__ __forceinline__ bool table_find(const uint4* __restrict__ table, cons
     return false;
 }
 
-// kernel_find_neighbours (NeighbourSearchCUDA.cu:72-130): stencil cells in (dx, dy, dz) order,
-// each bucket walked in logical order, self skipped, r^2 < h^2 kept, at most maxNeighbours.  A
+// kernel_find_neighbours (NeighbourSearchCUDA.cu:72-130), one thread per particle: for lists too long
+// for k_neighbours_wave's rows.  Stencil cells in (dx, dy, dz) order, each bucket walked in logical order, self skipped, r^2 < h^2 kept, at most maxNeighbours.  A
 // bucket reached from two stencil cells with equal hashes is walked twice, as in the reference.
 // The list stores physical slots.
 //
@@ -408,8 +409,8 @@ __device__ __forceinline__ void batch_slots(const DeviceState& d, bool run, uint
     }
 }
 
-__device__ __forceinline__ void neighbours_slot(const DeviceState& d, const SphParams& P,
-                                                uint32_t p) {
+__global__ __launch_bounds__(kBlock) void k_neighbours(DeviceState d, SphParams P) {
+    const uint32_t p = xcd_slot<kBlock>();
     uint32_t count = 0;
     if (p < d.nslots) {
         const SceneDev& sc = scene_of(d, p);
@@ -491,80 +492,331 @@ __device__ __forceinline__ void neighbours_slot(const DeviceState& d, const SphP
     }
 }
 
-template <int BS>
-__global__ __launch_bounds__(BS) void k_neighbours(DeviceState d, SphParams P) {
-    neighbours_slot(d, P, xcd_slot<BS>());
+// The same lists built by whole waves.  A wave owns S consecutive slots.  Neighbouring slots mostly
+// lie in the same search cell (the layout is cell ordered), so its particles fall into runs of at most
+// eight with one cell each, and kWaveRuns runs are taken at a time:
+//   1. their 27 buckets each are probed one per lane, all at once; a prefix over the bucket lengths
+//      makes them one stream of candidates, each run's in stencil order (a bucket reached from two
+//      cells appears twice);
+//   2. the stream passes 64 candidates at a time, one per lane (the next 64 are loaded meanwhile), and
+//      each particle of the run (its position in scalar registers) is tested against all 64 at once:
+//      the accepted lanes' ranks in the ballot are their positions behind the particle's entries so
+//      far, in stream order;
+//   3. entries gather in LDS, one row per particle, and leave as whole 16-byte chunks.
+// With one thread per particle a wave walks 27 buckets per lane, for as long as its lane with most
+// candidates, and appends under eight masks per batch; here probes and candidate loads are made once
+// per run, every lane of a test does work, and lists of uneven length cost no idle lanes.
+// Measured against one thread per particle (kernel time): 1M settled column 359 -> 222 us, 1M dam
+// break (sprayed: 29 cells per 64 particles) 448 -> 332, 64 scenes of 2.6M 892 -> 637, 27,000
+// particles 66 -> 17, 1,000 particles 62 -> 11.  The tests bound it (168 of the 222 us, 14 vector
+// instructions per 64 pairs); in sprayed scenes also the probes (129 of the 332 us).
+// Candidates find their bucket by rank: bit t of the bitmap says that a bucket begins at t + 1, so the
+// set bits below a lane count the non-empty buckets before its own, and those buckets' (slot offset,
+// contiguity) sit in LDS in that order.
+constexpr uint32_t kWaveRuns = 4;              // runs probed together
+constexpr uint32_t kWaveWindow = 2048;         // stream positions per bitmap
+constexpr int kWaveBuildBlock = 256;
+// Longest lists of which eight, or two, rows per wave fit in a workgroup's 64 KB of LDS.
+constexpr int kWaveBuildMaxN8 = 320, kWaveBuildMaxN2 = 1792;
+
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+
+// Words of a list row in LDS: a stride of 4 modulo 32 banks, so the chunk reads of the eight rows fall
+// on different banks.
+__host__ __device__ __forceinline__ uint32_t wave_row_words(int maxN) {
+    return (((uint32_t)maxN + 3u) / 4u * 4u + 27u) / 32u * 32u + 4u;
+}
+// Words per wave: the rows, the bitmap, the buckets' (offset, contiguity) and a spare word per lane.
+template <uint32_t kWaveRows>
+__host__ __device__ __forceinline__ uint32_t wave_build_words(int maxN) {
+    return kWaveRows * wave_row_words(maxN) + kWaveWindow / 32u + (2u * kWaveRuns * 27u + 3u) / 4u * 4u + 64u;
 }
 
-// The same lists with one lane per stencil cell, for scenes too small to fill the chip: 32 lanes
-// per particle (lanes 27-31 idle), lane c on stencil cell c.  Each lane walks its bucket twice:
-// first counting its accepted candidates, then, after an exclusive prefix of the 27 counts in
-// stencil order, storing them at their list positions; positions at or past maxN are dropped, as
-// the one-lane walk stops there.  A bucket reached from two stencil cells is walked by both lanes,
-// as in the reference.
-template <int BS>
-__global__ __launch_bounds__(BS) void k_neighbours_cells(DeviceState d, SphParams P) {
-    const uint32_t T = xcd_slot<BS>();
-    const uint32_t p = T >> 5, c = T & 31u;
-    if (p >= d.nslots) return;  // whole groups
-    const SceneDev& sc = scene_of(d, p);
-    if (p >= sc.end) return;
-    const f3 xi = make3(d.XsA[p]);
-    int cx, cy, cz;
-    discretize(xi, P.cellSearch, cx, cy, cz);
-    uint4 e = make_uint4(0u, 0u, 0u, 0u);
-    if (c < 27u) {
-        const uint32_t h = cell_hash((int)((uint32_t)cx + (c / 9u - 1u)), (int)((uint32_t)cy + ((c / 3u) % 3u - 1u)),
-                                     (int)((uint32_t)cz + (c % 3u - 1u)), sc);
-        if (!table_find(d.table, sc, h, e)) e = make_uint4(0u, 0u, 0u, 0u);
+// LDS written by some lanes of a wave and read by others: LDS instructions of one wave complete in
+// issue order, so only the compiler has to be kept from moving accesses across this point.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// Inclusive prefix sum over the wave's 64 lanes.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
+    int x = (int)v;
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)x;
+}
+
+__device__ __forceinline__ uint32_t lane_u(uint32_t v, uint32_t lane) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
+}
+__device__ __forceinline__ float lane_f(float v, uint32_t lane) {
+    return __uint_as_float(lane_u(__float_as_uint(v), lane));
+}
+
+// a in the lanes of m, b in the others.  Written out: as an expression it becomes a branch.
+__device__ __forceinline__ uint32_t select(uint64_t m, uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_cndmask_b32 %0, %1, %2, %3" : "=v"(r) : "v"(b), "v"(a), "s"(m));
+    return r;
+}
+
+// kWaveRows: list rows in LDS, and the longest run.
+template <int S, uint32_t kWaveRows>
+__global__ __launch_bounds__(kWaveBuildBlock) void k_neighbours_wave(DeviceState d, SphParams P) {
+    extern __shared__ uint4 waveLds[];
+    constexpr uint32_t kWaves = kWaveBuildBlock / 64;
+    const uint32_t lane = __lane_id();
+    const uint32_t nb = gridDim.x, b = blockIdx.x;
+    const uint32_t block = (b % kXcds) * (nb / kXcds) + b / kXcds;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t base = (block * kWaves + wave) * (uint32_t)S;  // the wave's first slot
+    if (base >= d.nslots) return;
+    const SceneDev& sc = d.scenes[d.chunkScene[base >> 8]];  // S divides 256: one scene per wave
+    const float4* __restrict__ const Xs = d.XsA;
+    const uint32_t maxN = (uint32_t)P.maxN, rowWords = wave_row_words(P.maxN);
+    const float h2 = P.h2;
+    uint32_t* const lds = reinterpret_cast<uint32_t*>(waveLds) + wave * wave_build_words<kWaveRows>(P.maxN);
+    const uint32_t ldsAt = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_u32*)lds);
+    uint32_t* const bitmap = lds + kWaveRows * rowWords;
+    uint2* const bucket = reinterpret_cast<uint2*>(bitmap + kWaveWindow / 32u);
+    const uint32_t spare = ldsAt + 4u * (wave_build_words<kWaveRows>(P.maxN) - 64u + lane);
+    uint4* const lists = d.nbr4 + (size_t)(base >> 6) * list_chunks(P.maxN) * 64u + (base & 63u);
+
+    const uint32_t slot = base + lane;
+    const bool mine = lane < (uint32_t)S && slot < d.nslots;
+    const bool valid = mine && slot < sc.end;  // a scene's slots are consecutive: the first lanes
+    const uint32_t nvalid = (uint32_t)__builtin_popcountll(__ballot(valid));
+    f3 xi{0.0f, 0.0f, 0.0f};
+    int cx = 0, cy = 0, cz = 0;
+    if (valid) {
+        xi = make3(Xs[slot]);
+        discretize(xi, P.cellSearch, cx, cy, cz);
     }
-    const uint32_t a = e.x, b = e.y;
-    const bool run = e.w != 0u;
-    const int32_t shift = (int32_t)e.z - (int32_t)a;  // physical - logical
-    // the accepted candidates of bucket positions [m0, m0 + kWalkBatch), one bit each
-    const auto batch = [&](uint32_t m0, uint32_t (&ph)[kWalkBatch]) {
-        float4 cand[kWalkBatch];
-        batch_slots<kWalkBatch>(d, run, m0, b, shift, ph);
-#pragma unroll
-        for (int u = 0; u < kWalkBatch; ++u) cand[u] = ld(d.XsA, ph[u]);
-        uint32_t acc = 0u;
-#pragma unroll
-        for (int u = 0; u < kWalkBatch; ++u) {
-            const f3 sep = xi - make3(cand[u]);
-            const bool ok = (dot3(sep, sep) < P.h2) & (ph[u] != p) & (m0 + u < b);
-            acc |= (uint32_t)ok << u;
-        }
-        return acc;
+    // first lanes of the runs: another cell than the lane before, or the ninth, 17th, ... of its cell
+    const int px = __builtin_amdgcn_update_dpp(0, cx, 0x138, 0xF, 0xF, false);  // wave_shr:1
+    const int py = __builtin_amdgcn_update_dpp(0, cy, 0x138, 0xF, 0xF, false);
+    const int pz = __builtin_amdgcn_update_dpp(0, cz, 0x138, 0xF, 0xF, false);
+    const uint64_t cells = __ballot(valid && (lane == 0u || px != cx || py != cy || pz != cz));
+    const uint64_t upTo = cells & (~0ull >> (63u - lane));
+    const uint32_t inCell = upTo ? lane - (63u - (uint32_t)__builtin_clzll(upTo)) : 1u;
+    uint64_t heads = __ballot(valid && (inCell & (kWaveRows - 1u)) == 0u);
+
+    uint32_t counts = 0;            // this lane's particle's list length
+    uint32_t row0 = 0, rowEnd = 0;  // the rows hold the lists of lanes [row0, rowEnd)
+    const auto flush = [&]() {
+        wave_lds_order();
+        const uint32_t r = lane & (kWaveRows - 1u), c0 = lane / kWaveRows;
+        const uint32_t held = (uint32_t)__shfl((int)counts, (int)((row0 + r) & 63u), 64);
+        const uint32_t n = row0 + r < rowEnd ? held : 0u;
+        for (uint32_t c = c0; __ballot(4u * c < n); c += 64u / kWaveRows)
+            if (4u * c < n)
+                lists[(size_t)c * 64u + row0 + r] = *reinterpret_cast<const uint4*>(&lds[r * rowWords + 4u * c]);
+        wave_lds_order();
+        row0 = rowEnd;
     };
-    uint32_t mine = 0;
-    for (uint32_t m0 = a; m0 < b; m0 += kWalkBatch) {
-        uint32_t ph[kWalkBatch];
-        mine += (uint32_t)__popc(batch(m0, ph));
-    }
-    uint32_t incl = mine;  // inclusive prefix over the group's 32 lanes (stencil order)
+
+    while (heads) {
+        // ---- the buckets of the next runs, entry 27 i + cell of run i in lane (entry % 64) ----
+        uint64_t h4 = heads;
+        uint32_t leader[kWaveRuns];
+        uint32_t nruns = 0;
 #pragma unroll
-    for (int off = 1; off < 32; off <<= 1) {
-        const uint32_t y = __shfl_up(incl, off, 32);
-        if ((int)c >= off) incl += y;
-    }
-    const uint32_t total = __shfl(incl, 31, 32);
-    const uint32_t maxN = (uint32_t)P.maxN;
-    uint32_t k = incl - mine;  // this cell's first list position
-    if (mine && k < maxN) {
-        uint32_t* out = reinterpret_cast<uint32_t*>(d.nbr4 + list_base(p, P.maxN));
-        for (uint32_t m0 = a; m0 < b && k < maxN; m0 += kWalkBatch) {
-            uint32_t ph[kWalkBatch];
-            const uint32_t acc = batch(m0, ph);
+        for (uint32_t i = 0; i < kWaveRuns; ++i) {
+            leader[i] = h4 ? (uint32_t)__builtin_ctzll(h4) : leader[i ? i - 1u : 0u];
+            nruns += h4 ? 1u : 0u;
+            h4 &= h4 - 1ull;
+        }
+        constexpr uint32_t kRounds = (kWaveRuns * 27u + 63u) / 64u;
+        uint32_t key[kRounds], at[kRounds], start[kRounds], len[kRounds], incl[kRounds];
 #pragma unroll
-            for (int u = 0; u < kWalkBatch; ++u) {
-                if ((acc >> u) & 1u) {
-                    if (k < maxN) out[((size_t)(k >> 2) * 64u) * 4u + (k & 3u)] = ph[u];
-                    ++k;
-                }
+        for (uint32_t u = 0; u < kRounds; ++u) {
+            const uint32_t entry = u * 64u + lane, i = entry / 27u, c = entry - 27u * i;
+            uint32_t from = leader[0];
+#pragma unroll
+            for (uint32_t k = 1; k < kWaveRuns; ++k) from = i == k ? leader[k] : from;
+            const uint32_t gx = (uint32_t)__shfl(cx, (int)from, 64), gy = (uint32_t)__shfl(cy, (int)from, 64),
+                           gz = (uint32_t)__shfl(cz, (int)from, 64);
+            const uint32_t h = cell_hash((int)(gx + (c / 9u - 1u)), (int)(gy + ((c / 3u) % 3u - 1u)),
+                                         (int)(gz + (c % 3u - 1u)), sc);
+            key[u] = i < nruns ? h : kEmptyKey;  // kEmptyKey: an idle lane
+            at[u] = table_slot(h, sc.tabLog2);
+        }
+        // every lane's first two table slots at once; the rare longer probes one slot at a time
+        const uint4* __restrict__ const table = d.table + sc.tabOffset;
+        const uint32_t mask = (1u << sc.tabLog2) - 1u;
+        uint4 e[kRounds], e1[kRounds];
+#pragma unroll
+        for (uint32_t u = 0; u < kRounds; ++u) {
+            e[u] = table[at[u]];
+            e1[u] = table[(at[u] + 1u) & mask];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kRounds; ++u) {
+            const bool past = e[u].x != key[u] && e[u].x != kEmptyKey;
+            if (past) e[u] = e1[u];
+            at[u] += past ? 1u : 0u;
+            for (uint32_t probe = 0; probe <= mask; ++probe) {
+                const bool open = e[u].x != key[u] && e[u].x != kEmptyKey && key[u] != kEmptyKey;
+                if (!__ballot(open)) break;
+                at[u] += 1u;
+                if (open) e[u] = table[at[u] & mask];
             }
+            e[u] = key[u] != kEmptyKey && e[u].x == key[u] ? clamp_entry(e[u], sc) : make_uint4(0u, 0u, 0u, 0u);
+        }
+        uint32_t total = 0, filled = 0;
+        bool logical = false;
+        wave_lds_order();
+#pragma unroll
+        for (uint32_t u = 0; u < kRounds; ++u) {
+            len[u] = e[u].y - e[u].x;
+            incl[u] = total + wave_prefix(len[u]);
+            start[u] = incl[u] - len[u];
+            total = lane_u(incl[u], 63u);
+            const uint64_t f = __ballot(len[u] != 0u);
+            // buckets whose slots are not consecutive (hash collisions) are read through physT
+            logical |= len[u] != 0u && e[u].w == 0u;
+            if (len[u] != 0u)
+                bucket[filled + lanes_below(f)] = make_uint2((e[u].w ? e[u].z : e[u].x) - start[u], e[u].w);
+            filled += (uint32_t)__builtin_popcountll(f);
+        }
+        const bool anyLogical = __ballot(logical) != 0ull;
+        wave_lds_order();
+
+        // ---- the stream, one candidate per lane: position and slot ----
+        uint32_t ranked = 0;  // non-empty buckets that begin before the next 64 positions, but for the first
+        const auto load = [&](uint32_t t0, uint32_t& ph) {
+            if (t0 >= total) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (t0 % kWaveWindow == 0u) {
+                wave_lds_order();
+                bitmap[lane] = 0u;
+                wave_lds_order();
+#pragma unroll
+                for (uint32_t u = 0; u < kRounds; ++u) {
+                    const uint32_t bit = start[u] - 1u - t0;
+                    if (len[u] != 0u && start[u] != 0u && bit < kWaveWindow) atomicOr(&bitmap[bit >> 5], 1u << (bit & 31u));
+                }
+                wave_lds_order();
+            }
+            const uint2 bits = *reinterpret_cast<const uint2*>(&bitmap[(t0 % kWaveWindow) >> 5]);
+            const uint64_t begins = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)bits.y) << 32) |
+                                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bits.x);
+            const uint2 of = bucket[ranked + lanes_below(begins)];
+            ranked += (uint32_t)__builtin_popcountll(begins);
+            const bool in = t0 + lane < total;
+            ph = in ? t0 + lane + of.x : base;
+            if (anyLogical) {
+                if (in && of.y == 0u) ph = ld(d.physT, ph);
+            }
+            return ld(Xs, ph);
+        };
+        uint32_t t0 = 0, ph = base, phNext = base;
+        float4 c = load(0u, ph), cNext = load(64u, phNext);
+        const auto advance = [&]() {
+            t0 += 64u;
+            c = cNext;
+            ph = phNext;
+            cNext = load(t0 + 64u, phNext);
+        };
+
+        uint32_t begin = 0;
+        for (uint32_t i = 0; i < nruns; ++i) {
+            const uint32_t last = 27u * i + 26u;  // the run's last entry
+            const uint32_t end = last < 64u ? lane_u(incl[0], last) : lane_u(incl[kRounds - 1u], last - 64u);
+            const uint32_t first = (uint32_t)__builtin_ctzll(heads);
+            heads &= heads - 1ull;
+            const uint32_t np = (heads ? (uint32_t)__builtin_ctzll(heads) : nvalid) - first;
+            if (rowEnd - row0 + np > kWaveRows) flush();
+            const uint32_t row = ldsAt + 4u * (rowEnd - row0) * rowWords;  // LDS byte address of the run's first row
+            rowEnd += np;
+            if (begin == end) continue;  // no candidates: empty lists
+            if (begin >= t0 + 64u) advance();
+            // the run's particles against its stretch of the stream.  Each pass over them leaves at
+            // np, compared anew after each particle (after the lists' growth, to the compiler):
+            // hoisted out of the loop, the results of the compares take a scalar register pair each
+            // and spill.
+            const auto done = [&](uint32_t q, uint32_t after) {
+                uint32_t n = np;
+                asm("" : "+s"(n) : "s"(after));
+                return q >= n;
+            };
+            float qx[kWaveRows], qy[kWaveRows], qz[kWaveRows];
+            uint32_t put[kWaveRows];  // LDS byte address of the particle's next entry
+#pragma unroll
+            for (uint32_t q = 0; q < kWaveRows; ++q) {
+                put[q] = row + 4u * q * rowWords;
+                qx[q] = qy[q] = qz[q] = 0.0f;
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kWaveRows; ++q) {
+                if (q >= np) break;
+                qx[q] = lane_f(xi.x, first + q);
+                qy[q] = lane_f(xi.y, first + q);
+                qz[q] = lane_f(xi.z, first + q);
+            }
+            for (;;) {
+                const uint32_t t = t0 + lane;
+                // other runs' candidates are never within h
+                const float cx1 = (t >= begin) & (t < end) ? c.x : __builtin_inff();
+                const auto within = [&](uint32_t q) {
+                    const f3 sep{qx[q] - cx1, qy[q] - c.y, qz[q] - c.z};
+                    return __builtin_amdgcn_ballot_w64(dot3(sep, sep) < h2) &
+                           __builtin_amdgcn_ballot_w64(ph != base + first + q);
+                };
+                bool room = t0 + 64u - begin <= maxN;  // no list can be longer than the stretch so far
+                if (!room) {
+                    uint32_t most = 0;
+#pragma unroll
+                    for (uint32_t q = 0; q < kWaveRows; ++q) {
+                        if (q >= np) break;
+                        most = max(most, put[q] - (row + 4u * q * rowWords));
+                    }
+                    room = most + 256u <= 4u * maxN;
+                }
+                uint32_t grown = 0;
+                if (room) {
+#pragma unroll
+                    for (uint32_t q = 0; q < kWaveRows; ++q) {
+                        if (q && done(q, grown)) break;
+                        const uint64_t m = within(q);
+                        grown = (uint32_t)__builtin_popcountll(m);
+                        *(lds_u32*)select(m, put[q] + 4u * lanes_below(m), spare) = ph;
+                        put[q] += 4u * grown;
+                    }
+                } else {  // lists near their cap
+#pragma unroll
+                    for (uint32_t q = 0; q < kWaveRows; ++q) {
+                        if (q && done(q, grown)) break;
+                        const uint64_t m = within(q);
+                        grown = (uint32_t)__builtin_popcountll(m);
+                        const uint32_t left = maxN - ((put[q] - (row + 4u * q * rowWords)) >> 2);
+                        const uint32_t k = lanes_below(m);
+                        *(lds_u32*)select(m & __builtin_amdgcn_ballot_w64(k < left), put[q] + 4u * k, spare) = ph;
+                        put[q] += 4u * min(grown, left);
+                    }
+                }
+                if (end <= t0 + 64u) break;
+                advance();
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kWaveRows; ++q) {
+                if (q >= np) break;
+                counts = lane == first + q ? (put[q] - (row + 4u * q * rowWords)) >> 2 : counts;
+            }
+            begin = end;
         }
     }
-    if (c == 0u) d.cnt[p] = min(total, maxN);
+    flush();
+    if (mine) d.cnt[slot] = counts;
 }
 
 // The balanced work order (launch_balance): one workgroup per tile of T physical slots.  The
@@ -651,129 +903,6 @@ __device__ __forceinline__ uint32_t work_slot(const DeviceState& d, uint32_t t) 
     return (d.work != nullptr && t < d.nslots) ? d.work[t] : t;
 }
 
-// The list build walking each dx slab of the stencil (its nine cells in (dy, dz) order) as one
-// stream of candidates.  The nine buckets' entries (first slot, length, contiguity) sit in a
-// register queue; a batch of B stream positions may span several buckets, so a lane tests about as
-// many candidates as its slab holds instead of a whole batch per bucket (per-wave candidate slots
-// drop by about half on the 1M dam break).  Each lane first maps its B positions to buckets by
-// shifting the queue past exhausted buckets, then issues the B loads, then tests and appends in
-// stream order, which is the reference's list order.  Lists equal k_neighbours' entry for entry.
-// Held to 7 waves per SIMD (at most 72 VGPRs, a few spilled): the 256-scene batch's list build
-// measured 3.26 -> 3.10 ms against 6 waves.
-template <int BS, int B>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
-void k_neighbours_slab(DeviceState d, SphParams P) {
-    const uint32_t p = xcd_slot<BS>();
-    uint32_t count = 0;
-    if (p < d.nslots) {
-        const SceneDev& sc = scene_of(d, p);
-        if (p < sc.end) {
-            const f3 xi = make3(d.XsA[p]);
-            int cx, cy, cz;
-            discretize(xi, P.cellSearch, cx, cy, cz);
-            uint32_t* out = reinterpret_cast<uint32_t*>(d.nbr4 + list_base(p, P.maxN));
-            const uint32_t maxN = (uint32_t)P.maxN;
-            constexpr uint32_t kRun = 0x80000000u, kLen = 0x7FFFFFFFu;
-            for (int g = 0; g < 3 && count < maxN; ++g) {
-                // the slab's nine buckets: base (physical start of a contiguous bucket, else the
-                // logical start) and length | contiguity flag
-                uint32_t qb[9], ql[9];
-#pragma unroll
-                for (int r = 0; r < 3; ++r) {
-                    uint32_t hq[3];
-                    uint4 rq[3];
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) {
-                        const int c = g * 9 + r * 3 + q;
-                        hq[q] = cell_hash((int)((uint32_t)cx + (uint32_t)(c / 9 - 1)),
-                                          (int)((uint32_t)cy + (uint32_t)((c / 3) % 3 - 1)),
-                                          (int)((uint32_t)cz + (uint32_t)(c % 3 - 1)), sc);
-                        rq[q] = d.table[sc.tabOffset + table_slot(hq[q], sc.tabLog2)];
-                    }
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) {
-                        uint4 e = make_uint4(0u, 0u, 0u, 0u);
-                        if (rq[q].x == hq[q]) {
-                            e = clamp_entry(rq[q], sc);
-                        } else if (rq[q].x != kEmptyKey) {
-                            if (!table_find(d.table, sc, hq[q], e)) e = make_uint4(0u, 0u, 0u, 0u);
-                        }
-                        qb[r * 3 + q] = e.w ? e.z : e.x;
-                        ql[r * 3 + q] = (e.y - e.x) | (e.w ? kRun : 0u);
-                    }
-                }
-                uint32_t total = 0;
-#pragma unroll
-                for (int q = 0; q < 9; ++q) total += ql[q] & kLen;
-                uint32_t segStart = 0, segEnd = ql[0] & kLen, left = 8;
-                for (uint32_t t0 = 0; t0 < total && count < maxN; t0 += B) {
-                    uint32_t mm[B];
-                    bool rr[B];
-#pragma unroll
-                    for (int u = 0; u < B; ++u) {
-                        const uint32_t t = t0 + u;
-                        // shift the queue past exhausted (and empty) buckets; the lengths sum
-                        // to total, so a position below total always stops in a bucket
-                        while (t < total && t >= segEnd && left > 0) {
-#pragma unroll
-                            for (int k = 0; k < 8; ++k) {
-                                qb[k] = qb[k + 1];
-                                ql[k] = ql[k + 1];
-                            }
-                            ql[8] = 0u;
-                            --left;
-                            segStart = segEnd;
-                            segEnd += ql[0] & kLen;
-                        }
-                        if (t < total) {
-                            mm[u] = qb[0] + (t - segStart);
-                            rr[u] = (ql[0] & kRun) != 0u;
-                        } else {  // past the stream: repeat the previous position (discarded)
-                            mm[u] = u ? mm[u - 1] : qb[0];
-                            rr[u] = u ? rr[u - 1] : true;
-                        }
-                    }
-                    float4 c[B];
-                    uint32_t ph[B];
-                    bool anyLogical = false;
-#pragma unroll
-                    for (int u = 0; u < B; ++u) {
-                        ph[u] = mm[u];
-                        anyLogical |= !rr[u];
-                    }
-                    if (__builtin_expect(anyLogical, 0)) {  // hash collisions: slots through physT
-#pragma unroll
-                        for (int u = 0; u < B; ++u)
-                            if (!rr[u]) ph[u] = ld(d.physT, mm[u]);
-                    }
-#pragma unroll
-                    for (int u = 0; u < B; ++u) c[u] = ld(d.XsA, ph[u]);
-                    uint32_t acc = 0u;
-#pragma unroll
-                    for (int u = 0; u < B; ++u) {
-                        const f3 sep = xi - make3(c[u]);
-                        const bool ok = (dot3(sep, sep) < P.h2) & (ph[u] != p) & (t0 + u < total);
-                        acc |= (uint32_t)ok << u;
-                    }
-                    const uint32_t room = maxN - count;
-                    while ((uint32_t)__popc(acc) > room) acc &= ~(1u << (31 - __clz(acc)));
-                    if (acc) {
-#pragma unroll
-                        for (int u = 0; u < B; ++u) {
-                            if (acc & (1u << u)) {
-                                const uint32_t k = count + (uint32_t)__popc(acc & ((1u << u) - 1u));
-                                out[((size_t)(k >> 2) * 64u) * 4u + (k & 3u)] = ph[u];
-                            }
-                        }
-                        count += (uint32_t)__popc(acc);
-                    }
-                }
-            }
-        }
-        d.cnt[p] = count;
-    }
-}
-
 // The non-parity search (SphParams::searchCells == 2): cells of c = h / 2, keyed by their packed
 // coordinates (cell_key_fine), so every bucket is one cell and none is walked twice.  A cell at
 // offset (dx, dy, dz) from the particle's cell, |d| <= 2, can hold a particle within h only if its
@@ -782,9 +911,8 @@ void k_neighbours_slab(DeviceState d, SphParams P) {
 // the squared distances sum below (h / c)^2 = 4 (with a margin of 0.25% for the rounding of f).
 // Walked cells go in (dx, dy, dz) order, each bucket in logical order, self skipped, r^2 < h^2
 // kept, at most maxNeighbours: the list holds every particle within h (up to the cap).
-template <int BS>
-__global__ __launch_bounds__(BS) void k_neighbours_fine(DeviceState d, SphParams P) {
-    const uint32_t p = xcd_slot<BS>();
+__global__ __launch_bounds__(kBlock) void k_neighbours_fine(DeviceState d, SphParams P) {
+    const uint32_t p = xcd_slot<kBlock>();
     uint32_t count = 0;
     if (p < d.nslots) {
         const SceneDev& sc = scene_of(d, p);
@@ -957,20 +1085,6 @@ __global__ __launch_bounds__(BS) void k_density_lambda(DeviceState d, SphParams 
         density_lambda_slot<BS, kFast, kBnd>(d, P, Xs, residSlot, gated, xcd_slot_of<BS>(vb, nvb));
 }
 
-// The list build followed, in the same thread, by the first Jacobi iteration's density/lambda
-// sweep at x*_pred over the list just written (each lane reads back only its own list, so no
-// synchronisation is needed; x*_pred is read-only in this kernel).  Results are those of
-// k_neighbours then k_density_lambda; the neighbours' positions are still in the caches.
-// Physical work order only (no balanced order), no boundary samples.
-// Held to the list build's 7 waves per SIMD (at most 72 VGPRs).
-template <int BS, bool kFast>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
-void k_neighbours_density(DeviceState d, SphParams P) {
-    const uint32_t p = xcd_slot<BS>();
-    neighbours_slot(d, P, p);
-    density_lambda_slot<BS, kFast, false>(d, P, d.XsA, -1, 0, p);
-}
-
 // Features of the learned warm start at x*_pred, one neighbour sweep (list order):
 //   0 C = rho / rho0 - 1 and 1 lambda, as the first Jacobi iteration computes them
 //   2 neighbour count, 3 lambda of the previous step
@@ -1042,16 +1156,6 @@ __device__ __forceinline__ void features_slot(const DeviceState& d, const SphPar
 template <int BS>
 __global__ __launch_bounds__(BS) void k_features(DeviceState d, SphParams P, int record) {
     features_slot(d, P, record, xcd_slot<BS>());
-}
-
-// The list build followed, in the same thread, by the feature sweep over the list just written
-// (as k_neighbours_density does for the density/lambda sweep).
-template <int BS>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
-void k_neighbours_features(DeviceState d, SphParams P, int record) {
-    const uint32_t p = xcd_slot<BS>();
-    neighbours_slot(d, P, p);
-    features_slot(d, P, record, p);
 }
 
 // Residual statistics per scene in two fixed-order stages (deterministic sums, no atomics).
@@ -1973,25 +2077,36 @@ void launch_invert_order(hipStream_t st, const DeviceState& d, uint32_t* phys) {
 void launch_bucket_phys(hipStream_t st, const DeviceState& d) {
     k_bucket_phys<<<grid(d.nslots), kBlock, 0, st>>>(d);
 }
-void launch_neighbours(hipStream_t st, const DeviceState& d, const SphParams& P, int bs,
-                       int slabBatch, bool density, int features, bool cells) {
-    if (cells) {
-        AKUA_BY_BLOCK(bs, (k_neighbours_cells<BS><<<grid_lanes(d.nslots, 32, BS), BS, 0, st>>>(d, P)));
-    } else if (features >= 0) {
-        AKUA_BY_BLOCK(bs, (k_neighbours_features<BS><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P, features)));
-    } else if (density) {
-        if (P.fast)
-            AKUA_BY_BLOCK(bs, (k_neighbours_density<BS, true><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));
-        else
-            AKUA_BY_BLOCK(bs, (k_neighbours_density<BS, false><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));
-    } else if (P.searchCells == 2)
-        AKUA_BY_BLOCK(bs, (k_neighbours_fine<BS><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));
-    else if (slabBatch == 4)
-        AKUA_BY_BLOCK(bs, (k_neighbours_slab<BS, 4><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));
-    else if (slabBatch == 8)
-        AKUA_BY_BLOCK(bs, (k_neighbours_slab<BS, 8><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));
+namespace {
+// Slots per wave of the list build: 64, or fewer in scenes that would leave the chip's 1,024 SIMDs
+// without waves (a wave's runs are worked through one after another).
+template <int S, uint32_t kWaveRows>
+void neighbours_wave_of(hipStream_t st, const DeviceState& d, const SphParams& P) {
+    constexpr uint32_t kWaves = kWaveBuildBlock / 64;
+    const unsigned lds = kWaves * wave_build_words<kWaveRows>(P.maxN) * (unsigned)sizeof(uint32_t);
+    k_neighbours_wave<S, kWaveRows><<<grid_xcd(d.nslots, (int)kWaves * S), kWaveBuildBlock, lds, st>>>(d, P);
+}
+template <uint32_t kWaveRows>
+void neighbours_wave(hipStream_t st, const DeviceState& d, const SphParams& P) {
+    if (d.nslots >= (1u << 19))
+        neighbours_wave_of<64, kWaveRows>(st, d, P);
+    else if (d.nslots >= (1u << 17))
+        neighbours_wave_of<32, kWaveRows>(st, d, P);
+    else if (d.nslots >= (1u << 16))
+        neighbours_wave_of<16, kWaveRows>(st, d, P);
     else
-        AKUA_BY_BLOCK(bs, (k_neighbours<BS><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));
+        neighbours_wave_of<8, kWaveRows>(st, d, P);
+}
+}  // namespace
+void launch_neighbours(hipStream_t st, const DeviceState& d, const SphParams& P) {
+    if (P.searchCells == 2)
+        k_neighbours_fine<<<grid_xcd(d.nslots, kBlock), kBlock, 0, st>>>(d, P);
+    else if (P.maxN <= kWaveBuildMaxN8)
+        neighbours_wave<8>(st, d, P);
+    else if (P.maxN <= kWaveBuildMaxN2)
+        neighbours_wave<2>(st, d, P);
+    else
+        k_neighbours<<<grid_xcd(d.nslots, kBlock), kBlock, 0, st>>>(d, P);
 }
 template <int BS>
 void density_lambda_bs(hipStream_t st, const DeviceState& d, const SphParams& P, const float4* Xs,

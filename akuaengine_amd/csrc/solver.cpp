@@ -631,31 +631,21 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
     const int bs = s->tuning.block;
     const int I = s->cfg.solverIterations;
     const bool learned = s->mode == 1 && !record;
-    const bool plainOrder = !d.work && s->tuning.slabBatch == 0 && P.searchCells == 1 && !P.bd.on;
-    // small scenes: lane groups in the sweeps of a plain step, one lane per stencil cell in the
-    // list build
+    const bool plainOrder = !d.work && P.searchCells == 1 && !P.bd.on;
+    // small scenes: lane groups in the sweeps of a plain step
     const int lanesSet = s->tuning.laneGroup > 1 && plainOrder && !learned && !record ? s->tuning.laneGroup : 1;
-    // with the work queue too, the queue runs the list build, the Jacobi sweeps and confinement, and
-    // the lane groups run vorticity and XSPH (two gathered records per neighbour, whose latency
+    // with the work queue too, the queue runs the Jacobi sweeps and confinement, and the lane groups run vorticity and XSPH (two gathered records per neighbour, whose latency
     // more lanes per particle hide better)
     const bool queueSet = s->tuning.workQueue > 0 && !learned && !record && s->queue.p &&
                           s->heads.n >= queue_heads_size(queue_passes(s));
     const int lanes = queueSet ? 1 : lanesSet;
     const int postLanes = lanesSet;
-    // the first plain density/lambda sweep, or the learned step's feature sweep, runs inside
-    // the list build's launch
-    const bool fusable = s->tuning.fuseSweep == 1 && plainOrder && lanes == 1;
-    const bool fusedDensity = fusable && I > 0 && !learned && !record;
-    const bool fusedFeatures = fusable && (learned || record);
     // the sweeps of a plain step as persistent launches over each XCD's queue of tiles
     const bool queued = queueSet;
     uint32_t pass = 0;
-    const char* nbrName = fusedDensity ? "neighbours_density" : fusedFeatures ? "neighbours_features"
-                                                                              : "neighbours";
-    L.before(nbrName);
-    launch_neighbours(st, d, P, bs, s->tuning.slabBatch, fusedDensity,
-                      fusedFeatures ? (record ? 1 : 0) : -1, lanes > 1);
-    L.after(nbrName);
+    L.before("neighbours");
+    launch_neighbours(st, d, P);
+    L.after("neighbours");
     if (d.work) {
         L.before("balance");
         launch_balance(st, d, P, (uint32_t)s->tuning.balanceTile, s->work.p, s->cntW.p,
@@ -675,7 +665,7 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
     // (scratch) and XsB (which the fallback may overwrite only
     // in scenes whose gate is set, where the warm chain's result is discarded)
     auto ws = [&](int j) { return j == 0 ? s->XsW.p : (j & 1) ? s->XsC.p : s->XsB.p; };
-    if ((learned || record) && !fusedFeatures) {
+    if (learned || record) {
         L.before("features");
         launch_features(st, d, P, record, bs);
         L.after("features");
@@ -707,14 +697,12 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
         const float4* in = xs[it & 1];
         float4* out = xs[(it + 1) & 1];
         const bool last = it + 1 == I;
-        if (!(fusedDensity && it == 0)) {
-            L.before(learned ? "density_lambda_fallback" : "density_lambda");
-            if (queued)
-                launch_density_lambda_queue(st, d, P, in, pass++);
-            else
-                launch_density_lambda(st, d, P, in, bs, record && it == I - Jt ? 2 : -1, learned, lanes);
-            L.after(learned ? "density_lambda_fallback" : "density_lambda");
-        }
+        L.before(learned ? "density_lambda_fallback" : "density_lambda");
+        if (queued)
+            launch_density_lambda_queue(st, d, P, in, pass++);
+        else
+            launch_density_lambda(st, d, P, in, bs, record && it == I - Jt ? 2 : -1, learned, lanes);
+        L.after(learned ? "density_lambda_fallback" : "density_lambda");
         if (record && it == I - Jt) {
             L.before("targets");
             launch_targets(st, d, P, in);
@@ -1511,27 +1499,23 @@ void autotune(akua_solver* s, float dt, const float* bmin, const float* bmax, in
     sweep(&akua_tuning::layoutDigitBits, {0, 5, 8});
     sweep(&akua_tuning::layoutInterval, {1, 2, 4});
     sweep(&akua_tuning::balanceTile, {0, 512, 1024, 2048});
-    sweep(&akua_tuning::slabBatch, {0, 4, 8});
     // the sweeps' launch forms interact (lane groups beside the work queue run only vorticity and
-    // XSPH, without it every sweep and then no fused first sweep), so they are timed together
+    // XSPH, without it every sweep), so they are timed together
     {
         const akua_tuning base = best;
-        for (int f : {0, 1})
-            for (int wq : {0, 1, 2})
-                for (int l : {0, 2, 4, 8, 16}) {
-                    if (l > 1 && wq == 0 && f == 1) continue;  // the same launches as f == 0
-                    if (f == base.fuseSweep && wq == base.workQueue && l == base.laneGroup) continue;
-                    akua_tuning t = base;
-                    t.fuseSweep = f;
-                    t.workQueue = wq;
-                    t.laneGroup = l;
-                    apply_tuning(s, t);
-                    const double ms = time_trial(s, q, dt, trialSteps);
-                    if (ms < bestMs) {
-                        bestMs = ms;
-                        best = t;
-                    }
+        for (int wq : {0, 1, 2})
+            for (int l : {0, 2, 4, 8, 16}) {
+                if (wq == base.workQueue && l == base.laneGroup) continue;
+                akua_tuning t = base;
+                t.workQueue = wq;
+                t.laneGroup = l;
+                apply_tuning(s, t);
+                const double ms = time_trial(s, q, dt, trialSteps);
+                if (ms < bestMs) {
+                    bestMs = ms;
+                    best = t;
                 }
+            }
     }
     // the non-parity search over h / 2 cells, only when the caller gave up bit-exactness
     int bestCells = s->sph.searchCells;

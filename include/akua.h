@@ -157,22 +157,17 @@ typedef struct akua_tuning {
                                  slots of each tile of this many sorted by neighbour count, so that
                                  the lanes of a wave walk lists of similar length (their gathers
                                  then spread over the tile) */
-    int32_t slabBatch;        /* 0: the list build walks each of the 27 stencil buckets in batches
-                                 of 8 candidates; 4 or 8: it walks each dx slab of nine buckets as
-                                 one stream of candidates in batches of this many */
-    int32_t fuseSweep;        /* 0 (the default): the list build is a launch of its own; 1: the
-                                 same launch then runs, in each thread over the list it just
-                                 wrote, the first density/lambda sweep (or, in a learned or
-                                 training step, the feature sweep); applies with balanceTile 0,
-                                 slabBatch 0, the reference's search and no boundary samples */
+    int32_t slabBatch;        /* 0, 4 or 8: accepted and without effect (it chose between forms of the
+                                 list build that one form has replaced) */
+    int32_t fuseSweep;        /* 0 or 1: accepted and without effect (it ran the first sweep in the
+                                 list build's launch, which costs more than it saves since) */
     int32_t laneGroup;        /* 0 (the default): one thread per particle; 2, 4, 8 or 16: for scenes
                                  too small to fill the chip, the neighbour sweeps of a plain step
                                  run that many lanes per particle (each list's terms in parallel,
-                                 summed in list order) and the list build one lane per stencil cell;
-                                 applies with balanceTile 0, slabBatch 0, the reference's search and
-                                 no boundary samples, and takes precedence over fuseSweep.  With
-                                 workQueue set too, only the vorticity and XSPH sweeps run in lane
-                                 groups; the queue runs the others */
+                                 summed in list order); applies with balanceTile 0, the reference's
+                                 search and no boundary samples.  With workQueue set too, only the
+                                 vorticity and XSPH sweeps run in lane groups; the queue runs the
+                                 others */
     int32_t workQueue;        /* 0 (the default): each neighbour sweep after the list build is one
                                  launch with a workgroup per block of slots; 1 or 2: after the list
                                  build, the 256-slot tiles each XCD serves are queued heaviest first
@@ -205,10 +200,8 @@ akua_status akua_solver_get_search(const akua_solver* s, int32_t* cellsPerH);
 akua_status akua_solver_set_exact(akua_solver* s, int32_t exact);
 akua_status akua_solver_get_tuning(const akua_solver* s, akua_tuning* t);
 /* Times short trials of candidate settings by coordinate descent (block, then layout level, then
- * the two digit widths, then the layout interval, the balance tile, the slab batch and the lane
- * group, then, without lane groups, the fused first sweep and the work queue) and keeps the
- * fastest.  Each trial restarts from a copy of the current
- * particle state, which is restored afterwards, so the call leaves the state as it found it.
+ * the two digit widths, then the layout interval and the balance tile, then the lane group and the
+ * work queue together) and keeps the fastest.  Each trial restarts from a copy of the current particle state, which is restored afterwards, so the call leaves the state as it found it.
  * boxMin/boxMax: the box the trials step in (NULL: each scene's current box).  trialSteps: timed
  * steps per candidate (1..1000), run twice; the faster run counts.  cachePath (NULL: no cache): a text file of earlier results keyed
  * by device architecture, log2 of the particle count, log2 of the scene count, neighbour cap and
