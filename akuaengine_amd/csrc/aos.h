@@ -5,6 +5,8 @@
 
 #include <cstdint>
 
+#include "pbf_types.h"
+
 namespace akua {
 
 // Same layout as akua_particle (include/akua.h) and AkuaEngine::Particle (Particle.h:8-31).
@@ -31,5 +33,19 @@ void launch_export_aos(hipStream_t st, AosParticle* out, uint32_t n, const float
                        const float4* V, const float4* VS, const float4* DP, const float* dens,
                        const float* lam, const uint32_t* id, const uint32_t* lid, const float4* W,
                        const uint32_t* hash, const float4* color, const float* size);
+
+// The particle state as arrays in logical order, scene after scene without the slots' padding:
+// xyz-interleaved positions and velocities, masses, densities, lambdas and ids of n particles.
+struct StateArrays {
+    float* pos;
+    float* vel;
+    float* mass;
+    float* dens;
+    float* lam;
+    uint32_t* id;
+};
+void launch_export_state(hipStream_t st, const StateArrays& out, uint32_t n, uint32_t nslots,
+                         const SceneDev* scenes, const uint32_t* chunkScene, const float4* X, const float4* V,
+                         const float* dens, const float* lam, const uint32_t* id, const uint32_t* lid);
 
 }  // namespace akua

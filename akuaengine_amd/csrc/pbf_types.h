@@ -19,6 +19,7 @@ struct SceneDev {
     uint32_t layoutBits;   // bits per axis of the super-cell Morton key (memory layout only)
     uint32_t modMagic;     // x % tableSize by multiply-high (fast_mod below)
     uint32_t modShift;
+    uint32_t first;        // particles of the scenes before this one
     int32_t layoutOrigin[4];  // super-cell coordinates mapped to Morton coordinate 0
     float bmin[4];         // box (xyz) for the wall clamp and the velocity damping
     float bmax[4];

@@ -7,14 +7,18 @@
 
 #include <algorithm>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <fstream>
 #include <map>
+#include <mutex>
 #include <new>
 #include <sstream>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/akua.h"
@@ -152,6 +156,51 @@ struct TimedLaunch {
     hipEvent_t a, b;
 };
 
+// Pinned host chunks that device memory passes through on its way to the caller's pageable memory,
+// each with the event of its last copy.  At most kStageChunks chunks, made when first used and kept
+// with the solver.
+constexpr size_t kStageChunk = 1u << 20, kStageChunks = 16;
+
+struct Staging {
+    std::vector<char*> chunk;
+    std::vector<hipEvent_t> ready;
+    size_t bytes = 0;  // of each chunk
+    Staging() = default;
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
+    // Chunks for `total` bytes: at least one, or false where the host has no pinned memory left.
+    bool ensure(size_t total) {
+        const size_t want = std::min(kStageChunk, (total + 65535) / 65536 * 65536);
+        if (want > bytes) {
+            release();
+            bytes = want;
+        }
+        const size_t count = std::min(kStageChunks, (total + bytes - 1) / bytes);
+        while (chunk.size() < count) {
+            if (ready.size() == chunk.size()) {
+                hipEvent_t e = nullptr;
+                HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+                ready.push_back(e);
+            }
+            void* p = nullptr;
+            if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();
+                break;
+            }
+            chunk.push_back(static_cast<char*>(p));
+        }
+        return !chunk.empty();
+    }
+    void release() {
+        for (auto e : ready) (void)hipEventDestroy(e);
+        for (auto p : chunk) (void)hipHostFree(p);
+        ready.clear();
+        chunk.clear();
+        bytes = 0;
+    }
+    ~Staging() { release(); }
+};
+
 }  // namespace
 
 struct akua_solver {
@@ -248,6 +297,7 @@ struct akua_solver {
     hipEvent_t orderEvent = nullptr;
     // record export staging (get_particles), allocated on first use
     DevBuf<AosParticle> aosStage;
+    Staging staging;  // pinned chunks of get_state and get_particles, allocated on first use
 
     // timing
     bool timing = false;
@@ -298,6 +348,7 @@ struct akua_solver {
     ~akua_solver() {
         if (stream) (void)hipStreamSynchronize(stream);
         release_buffers();
+        staging.release();
         for (auto& g : graphs)
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
         for (auto e : eventPool) (void)hipEventDestroy(e);
@@ -377,7 +428,7 @@ void setup(akua_solver* s, const std::vector<uint32_t>& counts) {
     HIP_CHECK(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
 
     // scene slot layout
-    uint32_t slot = 0, tab = 0;
+    uint32_t slot = 0, tab = 0, first = 0;
     uint32_t maxTable = 1;
     std::vector<uint32_t> sb, se;
     for (size_t i = 0; i < counts.size(); ++i) {
@@ -388,6 +439,8 @@ void setup(akua_solver* s, const std::vector<uint32_t>& counts) {
         SceneDev sc{};
         sc.begin = slot;
         sc.end = slot + (uint32_t)n;
+        sc.first = first;
+        first += (uint32_t)n;
         sc.tableSize = (uint32_t)T;
         const FastMod fm = make_fast_mod(sc.tableSize);
         sc.modMagic = fm.magic;
@@ -1030,6 +1083,130 @@ std::vector<T> download(akua_solver* s, const T* p, size_t n) {
     HIP_CHECK(hipStreamSynchronize(s->stream));
     if (n) HIP_CHECK(hipMemcpy(h.data(), p, n * sizeof(T), hipMemcpyDeviceToHost));
     return h;
+}
+
+// A piece of device memory and the caller's memory that takes it.
+struct Readback {
+    void* to;
+    const void* from;
+    size_t bytes;
+};
+
+// Copies the pieces, after the work already on the solver's stream, and returns when they are there.
+// A pageable hipMemcpy copies on one thread, which at these sizes mostly waits for the kernel to map
+// the caller's untouched pages (40 MB into new memory: 9.6 ms; 0.42 ms even for 1 MB).  Here the copy
+// engine fills pinned chunks and, above kReadbackInline bytes, several threads empty them (40 MB: 2.0 ms
+// with eight threads, 320 MB 77 -> 13 ms; below, threads cost more than they save).
+constexpr size_t kReadbackInline = 4u << 20, kReadbackPerThread = 2u << 20;
+constexpr unsigned kReadbackThreads = 8;
+
+void read_back(akua_solver* s, const std::vector<Readback>& pieces) {
+    struct Part {
+        char* to;
+        const char* from;
+        size_t bytes;
+    };
+    size_t total = 0;
+    for (const Readback& r : pieces) total += r.bytes;
+    if (!total) return;
+    if (!s->staging.ensure(total)) {
+        HIP_CHECK(hipStreamSynchronize(s->stream));
+        for (const Readback& r : pieces) HIP_CHECK(hipMemcpy(r.to, r.from, r.bytes, hipMemcpyDeviceToHost));
+        return;
+    }
+    const size_t chunk = s->staging.bytes, ring = s->staging.chunk.size();
+    std::vector<Part> parts;
+    for (const Readback& r : pieces)
+        for (size_t o = 0; o < r.bytes; o += chunk)
+            parts.push_back({static_cast<char*>(r.to) + o, static_cast<const char*>(r.from) + o,
+                             std::min(chunk, r.bytes - o)});
+    const auto issue = [&](size_t k) {
+        HIP_CHECK(hipMemcpyAsync(s->staging.chunk[k % ring], parts[k].from, parts[k].bytes, hipMemcpyDeviceToHost,
+                                 s->stream));
+        HIP_CHECK(hipEventRecord(s->staging.ready[k % ring], s->stream));
+    };
+    const auto empty = [&](size_t k) { std::memcpy(parts[k].to, s->staging.chunk[k % ring], parts[k].bytes); };
+    // whatever happens, no copy into the chunks is left in flight
+    struct Drain {
+        hipStream_t st;
+        ~Drain() { (void)hipStreamSynchronize(st); }
+    } drain{s->stream};
+
+    if (total <= kReadbackInline) {
+        size_t issued = 0;
+        for (size_t k = 0; k < parts.size(); ++k) {
+            for (; issued < parts.size() && issued < k + ring; ++issued) issue(issued);
+            HIP_CHECK(hipEventSynchronize(s->staging.ready[k % ring]));
+            empty(k);
+        }
+        return;
+    }
+    // the calling thread issues the copies and waits for them in order; the others empty the chunks
+    std::mutex mu;
+    std::condition_variable more, room;
+    size_t ready = 0, taken = 0;
+    std::vector<char> done(parts.size(), 0);
+    bool stop = false;
+    const auto work = [&] {
+        std::unique_lock<std::mutex> lock(mu);
+        for (;;) {
+            more.wait(lock, [&] { return stop || taken < ready || taken == parts.size(); });
+            if (stop || taken == parts.size()) return;
+            const size_t k = taken++;
+            lock.unlock();
+            empty(k);
+            lock.lock();
+            done[k] = 1;
+            room.notify_one();
+        }
+    };
+    struct Pool {
+        std::vector<std::thread> threads;
+        std::mutex& mu;
+        std::condition_variable& more;
+        bool& stop;
+        bool finished = false;
+        ~Pool() {
+            if (!finished) {
+                std::lock_guard<std::mutex> lock(mu);
+                stop = true;
+            }
+            more.notify_all();
+            for (auto& t : threads) t.join();
+        }
+    } pool{{}, mu, more, stop};
+    const unsigned cpus = std::max(1u, std::thread::hardware_concurrency());
+    const size_t want = std::min<size_t>({kReadbackThreads, cpus, total / kReadbackPerThread});
+    try {
+        for (size_t t = 0; t < want; ++t) pool.threads.emplace_back(work);
+    } catch (const std::system_error&) {  // no further thread: those that started do
+    }
+    const bool alone = pool.threads.empty();
+    size_t issued = 0;
+    for (size_t k = 0; k < parts.size(); ++k) {
+        for (; issued < parts.size() && issued < k + ring; ++issued) {
+            if (issued >= ring) {  // its chunk must have been emptied
+                std::unique_lock<std::mutex> lock(mu);
+                if (!done[issued - ring]) {
+                    if (issued > k) break;
+                    room.wait(lock, [&] { return done[issued - ring] != 0; });
+                }
+            }
+            issue(issued);
+        }
+        HIP_CHECK(hipEventSynchronize(s->staging.ready[k % ring]));
+        if (alone) {
+            empty(k);
+            done[k] = 1;
+            continue;
+        }
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            ready = k + 1;
+        }
+        more.notify_one();
+    }
+    pool.finished = true;
 }
 
 // ---- tuning ---------------------------------------------------------------------------------
@@ -1693,25 +1870,35 @@ akua_status akua_solver_get_state(akua_solver* s, float* pos, float* vel, float*
     return guarded([&] {
         if (!s) fail(AKUA_ERR_INVALID_ARG, "NULL solver");
         check_n(s, n);
-        auto X = download(s, s->X.p, s->nslots);
-        auto V = download(s, s->V.p, s->nslots);
-        auto D = download(s, s->dens.p, s->nslots);
-        auto L = download(s, s->lam.p, s->nslots);
-        auto I = download(s, s->id.p, s->nslots);
-        auto LI = download(s, s->lid.p, s->nslots);
-        size_t base = 0;
-        for (const SceneDev& sc : s->scenes) {
-            for (uint32_t slot = sc.begin; slot < sc.end; ++slot) {
-                const size_t k = base + (LI[slot] - sc.begin);  // logical position
-                if (pos) { pos[3 * k] = X[slot].x; pos[3 * k + 1] = X[slot].y; pos[3 * k + 2] = X[slot].z; }
-                if (vel) { vel[3 * k] = V[slot].x; vel[3 * k + 1] = V[slot].y; vel[3 * k + 2] = V[slot].z; }
-                if (mass) mass[k] = X[slot].w;
-                if (density) density[k] = D[slot];
-                if (lambda) lambda[k] = L[slot];
-                if (ids) ids[k] = I[slot];
-            }
-            base += sc.end - sc.begin;
+        const size_t np = s->nparticles;
+        const size_t f3 = 3 * np * sizeof(float), f1 = np * sizeof(float);
+        if (!s->hasState) {  // no particles yet
+            for (float* p : {pos, vel})
+                if (p) std::memset(p, 0, f3);
+            for (float* p : {mass, density, lambda})
+                if (p) std::memset(p, 0, f1);
+            if (ids) std::memset(ids, 0, f1);
+            return;
         }
+        upload_scenes(s);
+        // put in order on the device, in buffers that every step writes before it reads them
+        float* const rest = reinterpret_cast<float*>(s->XsC.p);
+        const StateArrays out{reinterpret_cast<float*>(s->X0.p), reinterpret_cast<float*>(s->Vc.p), rest, rest + np,
+                              rest + 2 * np, reinterpret_cast<uint32_t*>(rest + 3 * np)};
+        launch_export_state(s->stream, out, s->nparticles, s->nslots, s->dScenes.p, s->dChunkScene.p, s->X.p, s->V.p,
+                            s->dens.p, s->lam.p, s->id.p, s->lid.p);
+        HIP_CHECK(hipGetLastError());
+        std::vector<Readback> pieces;
+        const auto want = [&](void* to, const void* from, size_t bytes) {
+            if (to) pieces.push_back({to, from, bytes});
+        };
+        want(pos, out.pos, f3);
+        want(vel, out.vel, f3);
+        want(mass, out.mass, f1);
+        want(density, out.dens, f1);
+        want(lambda, out.lam, f1);
+        want(ids, out.id, f1);
+        read_back(s, pieces);
     });
 }
 
@@ -1726,8 +1913,7 @@ akua_status akua_solver_get_particles(akua_solver* s, akua_particle* out, int32_
                           s->dens.p, s->lam.p, s->id.p, s->lid.p, s->W.p, ds.skeys, s->color.p,
                           s->size.p);
         HIP_CHECK(hipGetLastError());
-        HIP_CHECK(hipStreamSynchronize(s->stream));
-        HIP_CHECK(hipMemcpy(out, s->aosStage.p, (size_t)n * sizeof(AosParticle), hipMemcpyDeviceToHost));
+        read_back(s, {{out, s->aosStage.p, (size_t)n * sizeof(AosParticle)}});
     });
 }
 
