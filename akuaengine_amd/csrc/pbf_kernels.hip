@@ -1032,11 +1032,12 @@ __device__ __forceinline__ void density_lambda_slot(const DeviceState& d, const 
                 f3 sep = xi - make3(xj4);
                 float d2 = dot3(sep, sep);
                 // m_j == 1 under kFast: every product by m_j is the other factor itself
-                rho = rho + (kFast ? poly6(d2, P) : xj4.w * poly6(d2, P));
+                const float w = poly6_of<kFast>(d2, P);
+                rho = rho + (kFast ? w : xj4.w * w);
                 // a zero gradient would add zeros to gi and sum, which change neither (both start
                 // at +0, and x + (-x) rounds to +0, so neither is ever -0): it is skipped
                 f3 g;
-                if (grad_spiky_nonzero<kFast>(sep, P, g)) {
+                if (grad_of<kFast>(sep, d2, P, g)) {
                     if (kFast) {
                         gi = gi + g;
                         f3 gj = negInv * g;
@@ -1055,8 +1056,8 @@ __device__ __forceinline__ void density_lambda_slot(const DeviceState& d, const 
                 boundary_visit(P.bd, xi.x, xi.y, xi.z, P.h, P.h2,
                                [&](uint32_t idx, float s0, float s1, float s2, float d2) {
                                    const float psi = P.bd.psi[idx];
-                                   rb = rb + psi * poly6(d2, P);
-                                   gb = gb + psi * grad_spiky<kFast>(f3{s0, s1, s2}, P);
+                                   rb = rb + psi * poly6_of<kFast>(d2, P);
+                                   gb = gb + psi * grad_or_zero<kFast>(f3{s0, s1, s2}, d2, P);
                                });
                 d.Bg[i] = make_float4(gb.x, gb.y, gb.z, 0.0f);
             }
@@ -1391,13 +1392,26 @@ __device__ __forceinline__ void delta_correct_slot(const DeviceState& d, const S
                 f3 sep = xi - make3(nb.x);
                 float d2 = dot3(sep, sep);
                 float coef = li + nb.lam;
-                if (kCorr) {  // w = poly6 >= +0
-                    const float w = poly6(d2, P);
-                    coef = coef + P.negCorrK * corr_pow(kFast ? div_rn_small_nonneg(w, Rdq) : div_rn(w, Rdq), P);
+                f3 g;
+                bool some;  // a gradient that is not zero
+                if constexpr (kFast) {
+                    // the quotient of s_corr and the gradient's, with one test for the rare cases of all
+                    const float w = kCorr ? poly6_bounded(d2, P) : 1.0f;
+                    float q = kCorr ? div_by(w, Rdq.b, Rdq.r) : 0.0f;
+                    GradTerm G;
+                    some = grad_term(sep, d2, P, G);
+                    if (__builtin_expect(some && (fminf(G.low, w) < kDivLowest || G.inexact), 0)) {
+                        if (kCorr) q = corr_by_division(w, q, Rdq);
+                        grad_by_division(G);
+                    }
+                    if (kCorr) coef = coef + P.negCorrK * corr_pow(q, P);
+                    if (some) g = G.g;
+                } else {
+                    if (kCorr) coef = coef + P.negCorrK * corr_pow(div_rn(poly6(d2, P), Rdq), P);
+                    some = grad_spiky_nonzero(sep, P, g);
                 }
                 const float c = kFast ? coef : coef * nb.x.w;  // m_j == 1 under kFast
-                f3 g;
-                if (__builtin_expect(grad_spiky_nonzero<kFast>(sep, P, g), 1)) {
+                if (__builtin_expect(some, 1)) {
                     dp = dp + c * g;
                 } else {  // the zero gradient's term c * 0: zeros, or NaN where c is not finite
                     const f3 z{0.0f, 0.0f, 0.0f};
@@ -1457,7 +1471,7 @@ __device__ __forceinline__ void vorticity_slot(const DeviceState& d, const SphPa
             f3 sep = xi - make3(nb.x);
             const float mj = kFast ? -1.0f : -nb.x.w;  // m_j == 1 under kFast
             f3 g;
-            if (__builtin_expect(grad_spiky_nonzero<kFast>(sep, P, g), 1))
+            if (__builtin_expect(grad_of<kFast>(sep, dot3(sep, sep), P, g), 1))
                 w = w + mj * cross3(vij, g);
             else  // the zero gradient's term: zeros, or NaN where v_ij is not finite
                 w = w + mj * cross3(vij, f3{0.0f, 0.0f, 0.0f});
@@ -1514,7 +1528,7 @@ __device__ __forceinline__ void confinement_slot(const DeviceState& d, const Sph
             f3 sep = xi - make3(nb.x);
             const float c = kFast ? diff : nb.w * diff;  // m_j == 1 under kFast
             f3 g;
-            if (__builtin_expect(grad_spiky_nonzero<kFast>(sep, P, g), 1))
+            if (__builtin_expect(grad_of<kFast>(sep, dot3(sep, sep), P, g), 1))
                 eta = eta + c * g;
             else  // the zero gradient's term c * 0: zeros, or NaN where c is not finite
                 eta = eta + c * f3{0.0f, 0.0f, 0.0f};
@@ -1783,9 +1797,9 @@ __global__ __launch_bounds__(BS) void k_density_lambda_group(DeviceState d, SphP
         [&](const float4& xj4, float (&t)[5]) {
             f3 sep = xi - make3(xj4);
             float d2 = dot3(sep, sep);
-            f3 gr = grad_spiky<kFast>(sep, P);
+            f3 gr = grad_or_zero<kFast>(sep, d2, P);
             if (kFast) {
-                t[0] = poly6(d2, P);
+                t[0] = poly6_bounded(d2, P);
                 t[1] = gr.x; t[2] = gr.y; t[3] = gr.z;
                 f3 gj = negInv * gr;
                 t[4] = dot3(gj, gj);
@@ -1836,10 +1850,11 @@ __global__ __launch_bounds__(BS) void k_delta_correct_group(DeviceState d, SphPa
             float d2 = dot3(sep, sep);
             float coef = li + nb.lam;
             if (P.corrOn) {
-                const float w = poly6(d2, P);
-                coef = coef + P.negCorrK * corr_pow(kFast ? div_rn_small(w, Rdq) : div_rn(w, Rdq), P);
+                const float w = poly6_of<kFast>(d2, P);
+                const float q = kFast ? corr_by_division(w, div_by(w, Rdq.b, Rdq.r), Rdq) : div_rn(w, Rdq);
+                coef = coef + P.negCorrK * corr_pow(q, P);
             }
-            f3 gr = grad_spiky<kFast>(sep, P);
+            f3 gr = grad_or_zero<kFast>(sep, d2, P);
             const f3 u = kFast ? coef * gr : (coef * nb.x.w) * gr;
             t[0] = u.x; t[1] = u.y; t[2] = u.z;
         },
@@ -1868,7 +1883,7 @@ __global__ __launch_bounds__(BS) void k_vorticity_group(DeviceState d, SphParams
         [&](const XV& nb, float (&t)[3]) {
             f3 vij = make3(nb.v) - vi;
             f3 sep = xi - make3(nb.x);
-            const f3 c = cross3(vij, grad_spiky<kFast>(sep, P));
+            const f3 c = cross3(vij, grad_or_zero<kFast>(sep, dot3(sep, sep), P));
             const f3 u = (kFast ? -1.0f : -nb.x.w) * c;
             t[0] = u.x; t[1] = u.y; t[2] = u.z;
         },
@@ -1896,7 +1911,7 @@ __global__ __launch_bounds__(BS) void k_confinement_group(DeviceState d, SphPara
         [&](const XW& nb, float (&t)[3]) {
             float diff = wi.w - nb.x.w;
             f3 sep = xi - make3(nb.x);
-            const f3 gr = grad_spiky<kFast>(sep, P);
+            const f3 gr = grad_or_zero<kFast>(sep, dot3(sep, sep), P);
             const f3 u = (kFast ? diff : nb.w * diff) * gr;
             t[0] = u.x; t[1] = u.y; t[2] = u.z;
         },

@@ -123,35 +123,6 @@ __device__ __forceinline__ f3 div3_rn(f3 v, float b) {
     return q;
 }
 
-// a / b where b and an upper bound of |a| are known to lie in the exact-division range: only
-// the lower bound of |a| (zero or >= 2^-40) is tested.
-// The fallback is marked unlikely so that the compiler keeps it behind a branch that every wave
-// skips, instead of computing the full division for every term and selecting.
-__device__ __forceinline__ float div_rn_small(float a, const Recip& R) {
-    float q = div_rn_unchecked(a, R);
-    if (__builtin_expect(low2(a) < kDivLo2, 0)) q = a / R.b;
-    return q;
-}
-
-// div_rn_small for a numerator that is +0 or positive: the one-correction quotient keeps the
-// sign by itself there (+0 stays +0), so no sign fix is needed.
-__device__ __forceinline__ float div_rn_small_nonneg(float a, const Recip& R) {
-    float q = a * R.r;
-    const float t = fmaf(-R.b, q, a);
-    q = fmaf(t, R.r, q);
-    if (__builtin_expect(low2(a) < kDivLo2, 0)) q = a / R.b;
-    return q;
-}
-
-// (x, y, z) / b on the same terms as div_rn_small.
-__device__ __forceinline__ f3 div3_rn_small(f3 v, float b) {
-    const Recip R = recip(b);
-    f3 q{div_rn_unchecked(v.x, R), div_rn_unchecked(v.y, R), div_rn_unchecked(v.z, R)};
-    const uint32_t lo = min(min(low2(v.x), low2(v.y)), low2(v.z));
-    if (lo < kDivLo2) q = {v.x / b, v.y / b, v.z / b};
-    return q;
-}
-
 // Correctly rounded sqrt for x >= 2^-96 (no scaling needed there): the 1-ulp hardware root,
 // corrected by the residuals of its two neighbours, as the compiler's own lowering does.  Below
 // 2^-96 it returns a value below 2^-47 (not necessarily correctly rounded): callers use it only
@@ -169,27 +140,123 @@ __device__ __forceinline__ float sqrt_rn_unscaled(float x) {
 
 // device_gradient_spiky (SmoothingKernelsCUDA.h:23-28): cs * (h - |r|)^2 * r / |r|.  |r| and
 // the three quotients are correctly rounded (the reference's length and '/'): a squared length
-// below 2^-96 gives |r| < 1e-5, the zero branch, whatever its last bits.  kFast: |r| lies in
-// [1e-5, h] and |cs| h^3 bounds the numerators, both inside the exact-division range
-// (SphParams::fast), so only the numerators' lower bound is tested.
+// below 2^-96 gives |r| < 1e-5, the zero branch, whatever its last bits.
 // grad_spiky_nonzero: the same gradient into g, or false (g untouched) where it is zero, for
 // callers whose sums a zero gradient leaves unchanged.
-template <bool kFast = false>
 __device__ __forceinline__ bool grad_spiky_nonzero(f3 r, const SphParams& P, f3& g) {
     const float d2 = dot3(r, r);
     const float rm = sqrt_rn_unscaled(d2);
     if (rm > P.h || rm < 1e-5f) return false;
     float t = P.h - rm;
     float s = P.cs * (t * t);
-    g = kFast ? div3_rn_small(s * r, rm) : div3_rn(s * r, rm);
+    g = div3_rn(s * r, rm);
     return true;
 }
 
-template <bool kFast = false>
 __device__ __forceinline__ f3 grad_spiky(f3 r, const SphParams& P) {
     f3 g{0.0f, 0.0f, 0.0f};
-    grad_spiky_nonzero<kFast>(r, P, g);
+    grad_spiky_nonzero(r, P, g);
     return g;
+}
+
+// ---- the sweeps with bounded quotients (SphParams::fast) ------------------------------------------
+// |r| lies in [1e-5, h] and |cs| h^3 bounds the numerators, both inside the exact-division range, so
+// of the range tests only the numerators' lower bound is left; and |r| and 1 / |r| come from one
+// hardware reciprocal root instead of a root, a reciprocal and their corrections (10 instead of 18
+// issue slots, a transcendental taking four):
+//   y = rsq(x); s0 = x y; s = fma(fma(-s0, s0, x), y / 2, s0) is RN(sqrt x) for every x, and
+//   i = fma(fma(-s, y, 1), y, y) is RN(1 / s) for every x but those whose root has a significand of
+//   all ones (there 1 / s lies just above the middle of two floats, and fma(-s, y, 1) is exactly 2^-24).
+// Both were checked over all 2^24 significands and exponent parities on the device (the exponent
+// only scales rsq here), and akua_selftest_arith checks them again.
+struct RootRecip {
+    float s, i;
+    bool inexact;  // i may not be the correctly rounded reciprocal
+};
+
+__device__ __forceinline__ RootRecip root_recip(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s0 = x * y;
+    const float d = fmaf(-s0, s0, x);
+    const float s = fmaf(d, 0.5f * y, s0);
+    const float e = fmaf(-s, y, 1.0f);
+    return {s, fmaf(e, y, y), e == 0x1p-24f};
+}
+
+// a / b from b's correctly rounded reciprocal where both lie in the exact-division range.  A zero
+// numerator gives a zero whose sign may differ: the sweeps only add terms to sums that start at
+// +0 and therefore are never -0, to which a zero of either sign is the same.
+__device__ __forceinline__ float div_by(float a, float b, float recip) {
+    const float q = a * recip;
+    return fmaf(fmaf(-b, q, a), recip, q);
+}
+
+// poly6 for squared lengths of any size, infinite and NaN included (cp is finite here, so cp * 0 is 0).
+__device__ __forceinline__ float poly6_bounded(float d2, const SphParams& P) {
+    const float t = __builtin_elementwise_maximum(P.h2 - d2, 0.0f);
+    return P.cp * ((t * t) * t);
+}
+
+// The gradient's quotients before their numerators' lower bound is looked at.
+struct GradTerm {
+    f3 n, g;      // numerators, quotients
+    float rm;     // |r|
+    float low;    // the smallest numerator's magnitude
+    bool inexact;
+};
+
+// False where the gradient is zero (d2 = |r|^2, NaN counting as inside, as the rounded length does).
+__device__ __forceinline__ bool grad_term(f3 r, float d2, const SphParams& P, GradTerm& G) {
+    if (d2 > P.d2Far || d2 < P.d2Near) return false;
+    const RootRecip R = root_recip(d2);
+    const float t = P.h - R.s;
+    G.n = (P.cs * (t * t)) * r;
+    G.g = {div_by(G.n.x, R.s, R.i), div_by(G.n.y, R.s, R.i), div_by(G.n.z, R.s, R.i)};
+    G.rm = R.s;
+    G.low = fminf(fminf(fabsf(G.n.x), fabsf(G.n.y)), fabsf(G.n.z));
+    G.inexact = R.inexact;
+    return true;
+}
+
+constexpr float kDivLowest = 0x1p-40f;
+
+// The quotients by '/' where the short form does not hold: a numerator below 2^-40 that is not zero,
+// or the reciprocal's exception.  Called where G.low < kDivLowest or G.inexact (also with a zero
+// numerator, whose quotient stands).
+__device__ __forceinline__ void grad_by_division(GradTerm& G) {
+    const uint32_t lo = min(min(low2(G.n.x), low2(G.n.y)), low2(G.n.z));
+    if (G.inexact || lo < kDivLo2) G.g = G.n / G.rm;
+}
+
+// The gradient into g, or false where it is zero.
+__device__ __forceinline__ bool grad_bounded(f3 r, float d2, const SphParams& P, f3& g) {
+    GradTerm G;
+    if (!grad_term(r, d2, P, G)) return false;
+    if (__builtin_expect(G.low < kDivLowest || G.inexact, 0)) grad_by_division(G);
+    g = G.g;
+    return true;
+}
+
+// The kernels' forms by kFast: bounded quotients or the general ones.
+template <bool kFast>
+__device__ __forceinline__ float poly6_of(float d2, const SphParams& P) {
+    return kFast ? poly6_bounded(d2, P) : poly6(d2, P);
+}
+template <bool kFast>
+__device__ __forceinline__ bool grad_of(f3 r, float d2, const SphParams& P, f3& g) {
+    return kFast ? grad_bounded(r, d2, P, g) : grad_spiky_nonzero(r, P, g);
+}
+template <bool kFast>
+__device__ __forceinline__ f3 grad_or_zero(f3 r, float d2, const SphParams& P) {
+    f3 g{0.0f, 0.0f, 0.0f};
+    grad_of<kFast>(r, d2, P, g);
+    return g;
+}
+
+// The artificial pressure's quotient w / wdq of the bounded sweeps (w is +0 or positive), before and
+// after its numerator's lower bound is looked at.
+__device__ __forceinline__ float corr_by_division(float w, float q, const Recip& R) {
+    return low2(w) < kDivLo2 ? w / R.b : q;
 }
 
 // powf(x, n) of the artificial pressure (ConstraintSolverCUDA.cu:124): an integer n is the n-fold

@@ -70,6 +70,10 @@ struct SphParams {
     // the kernel constants and delta_q, lie inside the exact-division range): the neighbour
     // sweeps then skip the multiplications by a neighbour's mass (identities) and those tests.
     int32_t fast;
+    // The squared lengths at which the rounded length leaves [1e-5, h], where the spiky gradient is
+    // not zero: the smallest with sqrtf(d2) >= 1e-5 and the largest with sqrtf(d2) <= h (both from
+    // the correctly rounded root, which is monotonic), for the sweeps with bounded quotients.
+    float d2Near, d2Far;
     BoundaryDev bd;    // boundary samples (bd.on == 0: none)
 };
 

@@ -62,6 +62,18 @@ __global__ void k_selftest(uint64_t n, uint64_t seed, unsigned long long* counts
         const float w = (float)(z1 >> 40) * 0x1p-26f;  // squared lengths of the SPH range
         if (!same_bits(akua::sqrt_rn_unscaled(w), sqrtf(w))) bad[3]++;
     }
+    // the sweeps' root and reciprocal from one reciprocal root, over squared lengths of [2^-34, 2^80),
+    // and a quotient by them
+    {
+        const float x = fabsf(rand_float(z1, -34, 79));
+        const akua::RootRecip r = akua::root_recip(x);
+        if (!same_bits(r.s, sqrtf(x))) bad[1]++;
+        if (!r.inexact) {
+            const float a = rand_float(z0, -40, 39);
+            if (!same_bits(r.i, 1.0f / r.s)) bad[0]++;
+            if (!same_bits(akua::div_by(a, r.s, r.i), a / r.s)) bad[0]++;
+        }
+    }
     for (int k = 0; k < 4; ++k)
         if (bad[k]) atomicAdd(&counts[k], bad[k]);
 }

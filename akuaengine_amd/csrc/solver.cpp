@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <fstream>
+#include <limits>
 #include <map>
 #include <mutex>
 #include <new>
@@ -100,6 +101,16 @@ SphParams make_sph(const akua_pbf_config& c, const akua_lambda_corr& corr) {
     P.vortEps = c.vorticityEpsilon;
     P.visc = c.viscosity;
     P.maxN = c.maxNeighbours;
+    // from the rounded squares, by steps of one float, to where the rounded root crosses
+    const float inf = std::numeric_limits<float>::infinity();
+    P.d2Near = 1e-5f * 1e-5f;
+    while (sqrtf(P.d2Near) >= 1e-5f) P.d2Near = nextafterf(P.d2Near, 0.0f);
+    while (sqrtf(P.d2Near) < 1e-5f) P.d2Near = nextafterf(P.d2Near, inf);
+    P.d2Far = P.h2;
+    if (P.d2Far > 0.0f && P.d2Far < inf) {
+        while (P.d2Far < inf && sqrtf(P.d2Far) <= P.h) P.d2Far = nextafterf(P.d2Far, inf);
+        while (sqrtf(P.d2Far) > P.h) P.d2Far = nextafterf(P.d2Far, 0.0f);
+    }
     return P;
 }
 
