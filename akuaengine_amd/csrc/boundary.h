@@ -26,6 +26,7 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "pbf_types.h"
@@ -47,60 +48,92 @@ __host__ __device__ inline float wall_plane(const BoundaryDev& B, int w, int l) 
     return (w & 1) ? B.hi[a] + (float)l * B.s : B.lo[a] - (float)l * B.s;
 }
 
-// Calls f(index, x - x_b (three floats), |x - x_b|^2) for every sample that counts for (x, y, z),
-// in ascending sample index.  The wall loop is unrolled so every axis index is a constant.
-template <class F>
-__host__ __device__ inline void boundary_visit(const BoundaryDev& B, float x, float y, float z,
-                                               float h, float h2, F&& f) {
-    const float xa[3] = {x, y, z};
-#pragma unroll
-    for (int w = 0; w < 6; ++w) {
-        const int a = w >> 1;
-        const int b = a == 0 ? 1 : 0;
-        const int c = a == 2 ? 1 : 2;
+// Axes of wall w: normal a, tangential b < c.
+template <int w>
+struct WallAxes {
+    static constexpr int a = w >> 1, b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+};
+
+// Tangential indices [b0, b1] x [c0, c1] that a point visits on each layer of a wall.
+struct BoundaryWindow {
+    int b0, b1, c0, c1;
+};
+
+// Calls f(wall w (an integral constant), layer, window) for every layer whose plane lies within h of
+// (x, y, z), in ascending (wall, layer).  The walls are unrolled so every axis index is a constant.
+template <class F, int w = 0>
+__host__ __device__ inline void boundary_windows(const BoundaryDev& B, float x, float y, float z, float h, float h2,
+                                                 F&& f) {
+    if constexpr (w < 6) {
+        constexpr int a = WallAxes<w>::a, b = WallAxes<w>::b, c = WallAxes<w>::c;
+        const float xa[3] = {x, y, z};
         const int tb0 = B.t0[w][0], tnb = B.tn[w][0], tc0 = B.t0[w][1], tnc = B.tn[w][1];
-        if (tnb == 0 || tnc == 0) continue;
-        // the layers whose plane lies within h (most walls have none: skip their windows)
-        uint32_t near = 0u;
-        for (int l = 0; l < B.layers; ++l) {
-            const float ra = xa[a] - wall_plane(B, w, l);
-            if (ra * ra < h2) near |= 1u << l;
-        }
-        if (!near) continue;
-        long long b0 = floor_sat((xa[b] - B.lo[b] - h) / B.d[b]) - 1;
-        long long b1 = floor_sat((xa[b] - B.lo[b] + h) / B.d[b]) + 1;
-        long long c0 = floor_sat((xa[c] - B.lo[c] - h) / B.d[c]) - 1;
-        long long c1 = floor_sat((xa[c] - B.lo[c] + h) / B.d[c]) + 1;
-        b0 = b0 < tb0 ? tb0 : b0;
-        b1 = b1 > tb0 + tnb - 1 ? tb0 + tnb - 1 : b1;
-        c0 = c0 < tc0 ? tc0 : c0;
-        c1 = c1 > tc0 + tnc - 1 ? tc0 + tnc - 1 : c1;
-        for (int l = 0; l < B.layers; ++l) {
-            if (!((near >> l) & 1u)) continue;
-            const float na = wall_plane(B, w, l);
-            const float ra = xa[a] - na;
-            for (int tb = (int)b0; tb <= (int)b1; ++tb) {
-                const float cb = B.lo[b] + (float)tb * B.d[b];
-                const float rb = xa[b] - cb;
-                if (rb * rb >= h2) continue;
-                for (int tc = (int)c0; tc <= (int)c1; ++tc) {
-                    const float cc = B.lo[c] + (float)tc * B.d[c];
-                    const float rc = xa[c] - cc;
-                    if (rc * rc >= h2) continue;
-                    float sep[3];
-                    sep[a] = ra;
-                    sep[b] = rb;
-                    sep[c] = rc;
-                    const float d2 = (sep[0] * sep[0] + sep[1] * sep[1]) + sep[2] * sep[2];
-                    if (!(d2 < h2)) continue;
-                    const uint32_t idx = B.base[w] + ((uint32_t)l * (uint32_t)tnb + (uint32_t)(tb - tb0)) *
-                                                         (uint32_t)tnc +
-                                         (uint32_t)(tc - tc0);
-                    f(idx, sep[0], sep[1], sep[2], d2);
+        if (tnb != 0 && tnc != 0) {
+            // the layers whose plane lies within h (most walls have none: skip their windows)
+            uint32_t near = 0u;
+            for (int l = 0; l < B.layers; ++l) {
+                const float ra = xa[a] - wall_plane(B, w, l);
+                if (ra * ra < h2) near |= 1u << l;
+            }
+            if (near) {
+                long long b0 = floor_sat((xa[b] - B.lo[b] - h) / B.d[b]) - 1;
+                long long b1 = floor_sat((xa[b] - B.lo[b] + h) / B.d[b]) + 1;
+                long long c0 = floor_sat((xa[c] - B.lo[c] - h) / B.d[c]) - 1;
+                long long c1 = floor_sat((xa[c] - B.lo[c] + h) / B.d[c]) + 1;
+                b0 = b0 < tb0 ? tb0 : b0;
+                b1 = b1 > tb0 + tnb - 1 ? tb0 + tnb - 1 : b1;
+                c0 = c0 < tc0 ? tc0 : c0;
+                c1 = c1 > tc0 + tnc - 1 ? tc0 + tnc - 1 : c1;
+                if (b0 <= b1 && c0 <= c1) {
+                    const BoundaryWindow win{(int)b0, (int)b1, (int)c0, (int)c1};
+                    for (int l = 0; l < B.layers; ++l)
+                        if ((near >> l) & 1u) f(std::integral_constant<int, w>{}, l, win);
                 }
             }
         }
+        boundary_windows<F, w + 1>(B, x, y, z, h, h2, static_cast<F&&>(f));
     }
+}
+
+// Sample (tb, tc) of layer l of wall w: x - x_b and its squared length; false where it does not count.
+template <int w>
+__host__ __device__ inline bool boundary_sample(const BoundaryDev& B, float x, float y, float z, float h2, int l,
+                                                int tb, int tc, float (&sep)[3], float& d2) {
+    constexpr int a = WallAxes<w>::a, b = WallAxes<w>::b, c = WallAxes<w>::c;
+    const float xa[3] = {x, y, z};
+    const float cb = B.lo[b] + (float)tb * B.d[b];
+    const float rb = xa[b] - cb;
+    if (rb * rb >= h2) return false;
+    const float cc = B.lo[c] + (float)tc * B.d[c];
+    const float rc = xa[c] - cc;
+    if (rc * rc >= h2) return false;
+    sep[a] = xa[a] - wall_plane(B, w, l);
+    sep[b] = rb;
+    sep[c] = rc;
+    d2 = (sep[0] * sep[0] + sep[1] * sep[1]) + sep[2] * sep[2];
+    return d2 < h2;
+}
+
+template <int w>
+__host__ __device__ inline uint32_t boundary_index(const BoundaryDev& B, int l, int tb, int tc) {
+    const uint32_t tnb = (uint32_t)B.tn[w][0], tnc = (uint32_t)B.tn[w][1];
+    return B.base[w] + ((uint32_t)l * tnb + (uint32_t)(tb - B.t0[w][0])) * tnc + (uint32_t)(tc - B.t0[w][1]);
+}
+
+// Calls f(index, x - x_b (three floats), |x - x_b|^2) for every sample that counts for (x, y, z),
+// in ascending sample index.
+template <class F>
+__host__ __device__ inline void boundary_visit(const BoundaryDev& B, float x, float y, float z,
+                                               float h, float h2, F&& f) {
+    boundary_windows(B, x, y, z, h, h2, [&](auto wall, int l, const BoundaryWindow& win) {
+        constexpr int w = decltype(wall)::value;
+        for (int tb = win.b0; tb <= win.b1; ++tb)
+            for (int tc = win.c0; tc <= win.c1; ++tc) {
+                float sep[3], d2;
+                if (boundary_sample<w>(B, x, y, z, h2, l, tb, tc, sep, d2))
+                    f(boundary_index<w>(B, l, tb, tc), sep[0], sep[1], sep[2], d2);
+            }
+    });
 }
 
 // True when some layer plane lies within h of the point along its normal: only then can a

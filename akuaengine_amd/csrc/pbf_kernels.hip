@@ -1328,17 +1328,24 @@ __device__ __forceinline__ f3 correct_position(f3 xi, f3& dp, const SphParams& P
 
 // kernel_update_position_and_velocity (IntegrationCUDA.cu:38-49) and the wall damping at the last
 // iteration's corrected position q, and the step's writes of slot i.
+struct FinishIn {
+    float4 x0;
+    uint32_t id, lid;
+};
+__device__ __forceinline__ FinishIn finish_in(const DeviceState& d, uint32_t i) {
+    return {d.X0[i], d.Tid[i], d.lidT[i]};
+}
+
 template <bool kApplyDelta>
-__device__ __forceinline__ void finish_step(const DeviceState& d, const StepParams& S,
-                                            const SceneDev& sc, uint32_t i, float4 xi4, f3 q, f3 dp) {
-    const float4 x0 = d.X0[i];
-    f3 v = div3_rn(q - make3(x0), S.dt);
+__device__ __forceinline__ void finish_step(const DeviceState& d, const StepParams& S, const SceneDev& sc,
+                                            uint32_t i, float4 xi4, const FinishIn& in, f3 q, f3 dp) {
+    f3 v = div3_rn(q - make3(in.x0), S.dt);
     d.VS[i] = make_float4(v.x, v.y, v.z, 0.0f);  // the record's new_velocity (IntegrationCUDA.cu:45)
     v = damp_walls(q, v, sc);
     d.X[i] = make_float4(q.x, q.y, q.z, xi4.w);
     d.V[i] = make_float4(v.x, v.y, v.z, 0.0f);
-    d.id[i] = d.Tid[i];
-    d.lid[i] = d.lidT[i];
+    d.id[i] = in.id;
+    d.lid[i] = in.lid;
     if (kApplyDelta) {  // the record's position_delta (ConstraintSolverCUDA.cu:129)
         d.DP[i] = make_float4(dp.x, dp.y, dp.z, 0.0f);
     } else {  // no iteration ran: density, lambda and the position delta carry over
@@ -1434,7 +1441,7 @@ __device__ __forceinline__ void delta_correct_slot(const DeviceState& d, const S
         XsOut[i] = make_float4(q.x, q.y, q.z, xi4.w);
         return;
     }
-    finish_step<kApplyDelta>(d, S, sc, i, xi4, q, dp);
+    finish_step<kApplyDelta>(d, S, sc, i, xi4, finish_in(d, i), q, dp);
 }
 
 // Unit masses: held to 8 waves per SIMD (its scalar registers, over the 8-wave budget, spill to
@@ -1489,17 +1496,16 @@ __global__ __launch_bounds__(BS) void k_vorticity(DeviceState d, SphParams P) {
 // The confinement force from the summed eta (IntegrationCUDA.cu:146-163) and the write of Vc.
 __device__ __forceinline__ void confine_finish(const DeviceState& d, const SphParams& P,
                                                const StepParams& S, uint32_t i, float xi4w, float4 wi,
-                                               f3 eta, float invD) {
-    eta = eta * invD;
+                                               float4 v, f3 eta, float rho) {
+    eta = eta * (1.0f / rho);
     float el = length3(eta);
-    float4 v = d.V[i];
     if (!(el < 1e-5f)) {
         f3 N = div3_rn(eta, el);
         f3 f = P.vortEps * cross3(N, make3(wi));
         f3 vn = make3(v) + S.dt * f;
         v = make_float4(vn.x, vn.y, vn.z, 0.0f);
     }
-    v.w = xi4w / d.dens[i];
+    v.w = xi4w / rho;
     d.Vc[i] = v;
 }
 
@@ -1516,7 +1522,6 @@ __device__ __forceinline__ void confinement_slot(const DeviceState& d, const Sph
     const f3 xi = make3(xi4);
     const float xi4w = xi4.w;
     const float4 wi = d.W[i];
-    const float invD = 1.0f / d.dens[i];
     const uint32_t n = d.cntW[t];
     const uint4* lp = d.nbrW + list_base(t, P.maxN);
     f3 eta{0.0f, 0.0f, 0.0f};
@@ -1533,7 +1538,7 @@ __device__ __forceinline__ void confinement_slot(const DeviceState& d, const Sph
             else  // the zero gradient's term c * 0: zeros, or NaN where c is not finite
                 eta = eta + c * f3{0.0f, 0.0f, 0.0f};
         });
-    confine_finish(d, P, S, i, xi4w, wi, eta, invD);
+    confine_finish(d, P, S, i, xi4w, wi, d.V[i], eta, d.dens[i]);
 }
 
 template <int BS, bool kFast>
@@ -1710,90 +1715,180 @@ __global__ __launch_bounds__(kQueueTile) void k_xsph_queue(DeviceState d, SphPar
 }
 
 // ---- lane groups: L lanes per particle, for scenes too small to fill the chip ------------------
-// Thread T of a lane-group launch works on particle T / L (physical order).  The group's L lanes
-// take the list entries L at a time, lane r entry k0 + r, kLaneBatch rounds of loads in flight,
-// and compute each entry's terms; each lane stores its terms in its wave's rows of LDS, and the
-// group's first lane adds the L terms of a round in entry order, so each sum is the one-lane
-// sweep's sum, term for term and in list order (only that lane's sums are used).  Entries past the list's end contribute +0: no sum here starts at or reaches -0 (each
-// starts at +0 or a positive value, and x + (-x) rounds to +0), so adding +0 changes nothing.
-// Only plain steps (no learned gate, no residual check), the physical order and no wall samples.
-constexpr int kLaneBatch = 4;
-
+// Thread T of a lane-group launch works on particle T / L (physical order).  A round takes 4 L list
+// entries (32 with 16 lanes): lane r loads its entries' chunk and gathers, computes their terms and
+// stores them in its group's rows of LDS, one row per sum; then lane c alone adds row c in entry
+// order.  Each sum is therefore the one-lane sweep's, term for term and in list order.  Entries past
+// the list's end contribute +0: no sum here starts at or reaches -0 (each starts at +0 or a positive
+// value, and x + (-x) rounds to +0), so adding +0 changes nothing.
+// Bound by one chain of dependent loads (count and list chunk, then gathers), the 4 L adds of a round
+// (4 cycles each, the sums side by side in different lanes) and the launch itself.
+// Plain steps only (no learned gate, no residual check), in the physical order.
 template <int L>
 struct LaneGroup {
+    static_assert(L >= 2 && L <= 16 && (L & (L - 1)) == 0, "2, 4, 8 or 16");
+    static constexpr int kEntries = L == 16 ? 2 : 4;          // list entries per lane and round
+    static constexpr uint32_t kRound = (uint32_t)(L * kEntries);
+    // floats of a row: 4 more than a round, so that the rows read together start on different banks
+    static constexpr uint32_t kRow = kRound + 4u;
     uint32_t i;     // particle slot
     uint32_t r;     // lane within the group
     uint32_t base;  // first lane of the group within the wave
 };
 
+constexpr int kGroupBlock = 256;
+
 template <int L>
-__device__ __forceinline__ LaneGroup<L> lane_group(uint32_t T) {
-    static_assert(L >= 2 && L <= 64 && (L & (L - 1)) == 0, "a power of two that divides 64");
+__device__ __forceinline__ LaneGroup<L> lane_group() {
+    const uint32_t T = xcd_slot<kGroupBlock>();
     return {T / (uint32_t)L, T % (uint32_t)L, __lane_id() & ~(uint32_t)(L - 1)};
 }
 
-__device__ __forceinline__ uint32_t list_entry(const uint4* __restrict__ lp, uint32_t k) {
-    return reinterpret_cast<const uint32_t*>(lp + (size_t)(k >> 2) * 64u)[k & 3u];
+// NA sums of a group: lane r keeps sums r, r + L, ...
+template <int L, int NA>
+struct GroupSums {
+    static constexpr int kMine = (NA + L - 1) / L;
+    float s[kMine];
+    float* rows;  // the group's NA rows
+
+    // start: sum 0's first value (the others start at 0)
+    __device__ __forceinline__ GroupSums(const LaneGroup<L>& g, float start, float* lds) {
+        rows = lds + (threadIdx.x / (uint32_t)L) * (NA * LaneGroup<L>::kRow);
+#pragma unroll
+        for (int q = 0; q < kMine; ++q) s[q] = q == 0 && g.r == 0u ? start : 0.0f;
+    }
+    // t[u][c]: this lane's terms of sum c, entries r * kEntries + u of the round
+    __device__ __forceinline__ void add(const LaneGroup<L>& g, const float (&t)[LaneGroup<L>::kEntries][NA]) {
+        constexpr int E = LaneGroup<L>::kEntries;
+        constexpr uint32_t kRow = LaneGroup<L>::kRow;
+#pragma unroll
+        for (int c = 0; c < NA; ++c) {
+            float* const at = rows + (uint32_t)c * kRow + g.r * (uint32_t)E;
+            if constexpr (E == 4)
+                *reinterpret_cast<float4*>(at) = make_float4(t[0][c], t[1][c], t[2][c], t[3][c]);
+            else
+                *reinterpret_cast<float2*>(at) = make_float2(t[0][c], t[1][c]);
+        }
+        wave_lds_order();
+#pragma unroll
+        for (int q = 0; q < kMine; ++q) {
+            const uint32_t c = g.r + (uint32_t)(q * L);
+            const float4* const row = reinterpret_cast<const float4*>(rows + min(c, (uint32_t)NA - 1u) * kRow);
+            float4 v[LaneGroup<L>::kRound / 4u];
+#pragma unroll
+            for (uint32_t m = 0; m < LaneGroup<L>::kRound / 4u; ++m) v[m] = row[m];
+#pragma unroll
+            for (uint32_t m = 0; m < LaneGroup<L>::kRound / 4u; ++m) s[q] = (((s[q] + v[m].x) + v[m].y) + v[m].z) + v[m].w;
+        }
+        wave_lds_order();
+    }
+    // sum c, in every lane of the group
+    __device__ __forceinline__ float of(const LaneGroup<L>& g, int c) const {
+        return __shfl(s[c / L], (int)(g.base + (uint32_t)(c % L)), 64);
+    }
+};
+
+// A group's list: the particle's entry count and this lane's chunk of the first round, loaded without
+// waiting for the count (the chunk lies inside the particle's row).
+template <int L>
+struct GroupList {
+    const uint4* lp;
+    uint32_t n;
+    uint4 first;
+};
+
+template <int L>
+__device__ __forceinline__ uint4 group_chunk(const uint4* __restrict__ lp, const LaneGroup<L>& g, uint32_t k0) {
+    if constexpr (LaneGroup<L>::kEntries == 4) return lp[(size_t)((k0 >> 2) + g.r) * 64u];
+    const uint2 e = *(reinterpret_cast<const uint2*>(lp + (size_t)((k0 >> 2) + (g.r >> 1)) * 64u) + (g.r & 1u));
+    return make_uint4(e.x, e.y, 0u, 0u);
 }
 
-// sm: this wave's NA rows of 64 floats in LDS.  LDS instructions of one wave complete in issue
-// order, so a lane reads the terms the other lanes stored before the wave barrier; the second
-// barrier keeps the next round's stores after this round's reads.
+template <int L>
+__device__ __forceinline__ GroupList<L> group_list(const DeviceState& d, const SphParams& P, const LaneGroup<L>& g) {
+    GroupList<L> l;
+    l.lp = d.nbr4 + list_base(g.i, P.maxN);
+    l.n = d.cnt[g.i];  // 0 in the padding slots past a scene's end
+    const uint32_t chunk = g.r * (uint32_t)LaneGroup<L>::kEntries / 4u;
+    l.first = chunk < list_chunks(P.maxN) ? group_chunk(l.lp, g, 0u) : make_uint4(0u, 0u, 0u, 0u);
+    return l;
+}
+
+// Adds the terms of every list entry to the sums.
 template <int L, int NA, class T, class Load, class Term>
-__device__ __forceinline__ void walk_split(const uint4* __restrict__ lp, uint32_t n,
-                                           const LaneGroup<L>& g, Load load, Term term,
-                                           float (&acc)[NA], float* sm) {
-    const uint32_t lane = __lane_id();
-    for (uint32_t k0 = 0; k0 < n; k0 += (uint32_t)(L * kLaneBatch)) {
-        T v[kLaneBatch];
-        bool ok[kLaneBatch];
+__device__ __forceinline__ void walk_split(const GroupList<L>& l, const LaneGroup<L>& g, GroupSums<L, NA>& sums,
+                                           Load load, Term term) {
+    constexpr int E = LaneGroup<L>::kEntries;
+    uint4 ch = l.first;
+    for (uint32_t k0 = 0; k0 < l.n; k0 += LaneGroup<L>::kRound) {
+        const uint32_t k = k0 + g.r * (uint32_t)E;
+        const uint32_t e[4] = {ch.x, ch.y, ch.z, ch.w};
+        T v[E];
 #pragma unroll
-        for (int b = 0; b < kLaneBatch; ++b) {
-            const uint32_t k = k0 + (uint32_t)(b * L) + g.r;
-            ok[b] = k < n;
-            v[b] = load(list_entry(lp, ok[b] ? k : 0u));  // past the end: a valid entry, discarded
+        for (int u = 0; u < E; ++u) v[u] = load(k + (uint32_t)u < l.n ? e[u] : g.i);  // past the end: discarded
+        if (k + LaneGroup<L>::kRound < l.n) ch = group_chunk(l.lp, g, k0 + LaneGroup<L>::kRound);
+        float t[E][NA];
+#pragma unroll
+        for (int u = 0; u < E; ++u) {
+            term(v[u], t[u]);
+            const bool in = k + (uint32_t)u < l.n;
+#pragma unroll
+            for (int c = 0; c < NA; ++c) t[u][c] = in ? t[u][c] : 0.0f;
         }
-#pragma unroll
-        for (int b = 0; b < kLaneBatch; ++b) {
-            if (k0 + (uint32_t)(b * L) >= n) break;  // the same for every lane of the group
-            float t[NA];
-            term(v[b], t);
-#pragma unroll
-            for (int c = 0; c < NA; ++c) sm[c * 64 + lane] = ok[b] ? t[c] : 0.0f;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (g.r == 0) {
-#pragma unroll
-                for (int c = 0; c < NA; ++c)
-#pragma unroll
-                    for (int s = 0; s < L; ++s) acc[c] = acc[c] + sm[c * 64 + g.base + s];
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
+        sums.add(g, t);
     }
 }
 
-// This wave's NA rows of 64 floats in the workgroup's LDS block.
-template <int NA>
-__device__ __forceinline__ float* wave_rows(float* block) {
-    return block + (threadIdx.x >> 6) * (NA * 64);
+template <int L, int NA>
+constexpr uint32_t group_lds_floats() {
+    return (uint32_t)(kGroupBlock / L * NA) * LaneGroup<L>::kRow;
 }
 
-template <int BS, int L, bool kFast>
-__global__ __launch_bounds__(BS) void k_density_lambda_group(DeviceState d, SphParams P,
-                                                             const float4* __restrict__ Xs) {
-    __shared__ float lds[(BS / 64) * 5 * 64];
-    const LaneGroup<L> g = lane_group<L>(xcd_slot<BS>());
-    if (g.i >= d.nslots || g.i >= scene_of(d, g.i).end) return;  // whole groups
+// The wall samples of the group's particle, in the order of boundary_visit: each plane's window is
+// one row-major stream of candidates, a round of them at a time; a candidate that does not count adds
+// +0.  sums: the samples' density and gradient.
+template <int L, bool kFast>
+__device__ __forceinline__ void boundary_split(const SphParams& P, f3 xi, const LaneGroup<L>& g, GroupSums<L, 4>& sums) {
+    constexpr int E = LaneGroup<L>::kEntries;
+    const BoundaryDev& B = P.bd;
+    boundary_windows(B, xi.x, xi.y, xi.z, P.h, P.h2, [&](auto wall, int l, const BoundaryWindow& win) {
+        const uint32_t nc = (uint32_t)(win.c1 - win.c0 + 1), total = (uint32_t)(win.b1 - win.b0 + 1) * nc;
+        for (uint32_t k0 = 0; k0 < total; k0 += LaneGroup<L>::kRound) {
+            float t[E][4];
+#pragma unroll
+            for (int u = 0; u < E; ++u) {
+                const uint32_t k = k0 + g.r * (uint32_t)E + (uint32_t)u, row = k / nc;
+                float sep[3], d2;
+                t[u][0] = t[u][1] = t[u][2] = t[u][3] = 0.0f;
+                if (k < total && boundary_sample<decltype(wall)::value>(B, xi.x, xi.y, xi.z, P.h2, l, win.b0 + (int)row,
+                                                                        win.c0 + (int)(k - row * nc), sep, d2)) {
+                    const float psi = B.psi[boundary_index<decltype(wall)::value>(B, l, win.b0 + (int)row,
+                                                                                  win.c0 + (int)(k - row * nc))];
+                    const f3 gr = psi * grad_or_zero<kFast>(f3{sep[0], sep[1], sep[2]}, d2, P);
+                    t[u][0] = psi * poly6_of<kFast>(d2, P);
+                    t[u][1] = gr.x; t[u][2] = gr.y; t[u][3] = gr.z;
+                }
+            }
+            sums.add(g, t);
+        }
+    });
+}
+
+template <int L, bool kFast, bool kBnd>
+__global__ __launch_bounds__(kGroupBlock) void k_density_lambda_group(DeviceState d, SphParams P,
+                                                                      const float4* __restrict__ Xs) {
+    __shared__ float4 lds[group_lds_floats<L, 5>() / 4u];
+    const LaneGroup<L> g = lane_group<L>();
+    if (g.i >= d.nslots) return;  // whole groups
+    const GroupList<L> list = group_list<L>(d, P, g);
+    const SceneDev& sc = scene_of(d, g.i);
     const float4 xi4 = Xs[g.i];
     const f3 xi = make3(xi4);
     const float negInv = -P.invRest;
-    float acc[5] = {xi4.w * P.w0, 0.0f, 0.0f, 0.0f, 0.0f};  // rho, grad_i C (x, y, z), sum |grad_j C|^2
+    // rho, grad_i C (x, y, z), sum |grad_j C|^2
+    GroupSums<L, 5> sums(g, xi4.w * P.w0, reinterpret_cast<float*>(lds));
     walk_split<L, 5, float4>(
-        d.nbr4 + list_base(g.i, P.maxN), d.cnt[g.i], g, [&](uint32_t j) { return ld(Xs, j); },
+        list, g, sums, [&](uint32_t j) { return ld(Xs, j); },
         [&](const float4& xj4, float (&t)[5]) {
             f3 sep = xi - make3(xj4);
             float d2 = dot3(sep, sep);
@@ -1810,34 +1905,54 @@ __global__ __launch_bounds__(BS) void k_density_lambda_group(DeviceState d, SphP
                 f3 gj = (negInv * xj4.w) * gr;
                 t[4] = dot3(gj, gj);
             }
-        },
-        acc, wave_rows<5>(lds));
-    if (g.r != 0) return;
-    f3 gi{acc[1], acc[2], acc[3]};
+        });
+    float rho = sums.of(g, 0);
+    f3 gi{sums.of(g, 1), sums.of(g, 2), sums.of(g, 3)};
+    const float sum = sums.of(g, 4);
+    const bool writes = g.r == 0u && g.i < sc.end;
+    if (kBnd) {
+        const bool near = g.i < sc.end && boundary_near(P.bd, xi.x, xi.y, xi.z, P.h2);
+        float rb = 0.0f;
+        f3 gb{0.0f, 0.0f, 0.0f};
+        if (near) {
+            GroupSums<L, 4> wall(g, 0.0f, reinterpret_cast<float*>(lds));
+            // the rows of its own group again: a group's rows of four sums lie inside its rows of five
+            wall.rows = sums.rows;
+            boundary_split<L, kFast>(P, xi, g, wall);
+            rb = wall.of(g, 0);
+            gb = f3{wall.of(g, 1), wall.of(g, 2), wall.of(g, 3)};
+            if (writes) d.Bg[g.i] = make_float4(gb.x, gb.y, gb.z, 0.0f);
+        }
+        rho = rho + rb;
+        gi = gi + gb;
+    }
+    if (!writes) return;
     gi = gi * P.invRest;
-    const float C = acc[0] * P.invRest - 1.0f;
-    d.dens[g.i] = acc[0];
-    const float lam = -C / ((acc[4] + dot3(gi, gi)) + P.relax);
+    const float C = rho * P.invRest - 1.0f;
+    d.dens[g.i] = rho;
+    const float lam = -C / ((sum + dot3(gi, gi)) + P.relax);
     d.lam[g.i] = lam;
     if (kFast) d.W[g.i] = make_float4(xi.x, xi.y, xi.z, lam);
 }
 
-template <int BS, int L, bool kFinal, bool kFast>
-__global__ __launch_bounds__(BS) void k_delta_correct_group(DeviceState d, SphParams P, StepParams S,
-                                                            const float4* __restrict__ XsIn,
-                                                            float4* __restrict__ XsOut) {
-    __shared__ float lds[(BS / 64) * 3 * 64];
-    const LaneGroup<L> g = lane_group<L>(xcd_slot<BS>());
+template <int L, bool kFinal, bool kFast, bool kBnd>
+__global__ __launch_bounds__(kGroupBlock) void k_delta_correct_group(DeviceState d, SphParams P, StepParams S,
+                                                                     const float4* __restrict__ XsIn,
+                                                                     float4* __restrict__ XsOut) {
+    __shared__ float4 lds[group_lds_floats<L, 3>() / 4u];
+    const LaneGroup<L> g = lane_group<L>();
     if (g.i >= d.nslots) return;
+    const GroupList<L> list = group_list<L>(d, P, g);
     const SceneDev& sc = scene_of(d, g.i);
-    if (g.i >= sc.end) return;
     const float4 xi4 = XsIn[g.i];
     const f3 xi = make3(xi4);
     const float li = d.lam[g.i];
+    FinishIn in{};
+    if (kFinal) in = finish_in(d, g.i);
     const Recip Rdq = recip(P.wdq);
-    float acc[3] = {0.0f, 0.0f, 0.0f};
+    GroupSums<L, 3> sums(g, 0.0f, reinterpret_cast<float*>(lds));
     walk_split<L, 3, XLam>(
-        d.nbr4 + list_base(g.i, P.maxN), d.cnt[g.i], g,
+        list, g, sums,
         [&](uint32_t j) {
             if (kFast) {
                 const float4 a = ld(d.W, j);
@@ -1857,90 +1972,96 @@ __global__ __launch_bounds__(BS) void k_delta_correct_group(DeviceState d, SphPa
             f3 gr = grad_or_zero<kFast>(sep, d2, P);
             const f3 u = kFast ? coef * gr : (coef * nb.x.w) * gr;
             t[0] = u.x; t[1] = u.y; t[2] = u.z;
-        },
-        acc, wave_rows<3>(lds));
-    if (g.r != 0) return;
-    f3 dp{acc[0], acc[1], acc[2]};
+        });
+    f3 dp{sums.of(g, 0), sums.of(g, 1), sums.of(g, 2)};
+    if (g.r != 0u || g.i >= sc.end) return;
+    if (kBnd) {  // lambda_i times the boundary gradient sum of the density pass (same x*)
+        f3 gb{0.0f, 0.0f, 0.0f};
+        if (boundary_near(P.bd, xi.x, xi.y, xi.z, P.h2)) gb = make3(d.Bg[g.i]);
+        dp = dp + li * gb;
+    }
     const f3 q = correct_position(xi, dp, P, sc);
     if (!kFinal) {
         XsOut[g.i] = make_float4(q.x, q.y, q.z, xi4.w);
         return;
     }
-    finish_step<true>(d, S, sc, g.i, xi4, q, dp);
+    finish_step<true>(d, S, sc, g.i, xi4, in, q, dp);
 }
 
-template <int BS, int L, bool kFast>
-__global__ __launch_bounds__(BS) void k_vorticity_group(DeviceState d, SphParams P) {
-    __shared__ float lds[(BS / 64) * 3 * 64];
-    const LaneGroup<L> g = lane_group<L>(xcd_slot<BS>());
-    if (g.i >= d.nslots || g.i >= scene_of(d, g.i).end) return;
+template <int L, bool kFast>
+__global__ __launch_bounds__(kGroupBlock) void k_vorticity_group(DeviceState d, SphParams P) {
+    __shared__ float4 lds[group_lds_floats<L, 3>() / 4u];
+    const LaneGroup<L> g = lane_group<L>();
+    if (g.i >= d.nslots) return;
+    const GroupList<L> list = group_list<L>(d, P, g);
+    const SceneDev& sc = scene_of(d, g.i);
     const f3 xi = make3(d.X[g.i]);
     const f3 vi = make3(d.V[g.i]);
-    float acc[3] = {0.0f, 0.0f, 0.0f};
+    GroupSums<L, 3> sums(g, 0.0f, reinterpret_cast<float*>(lds));
     walk_split<L, 3, XV>(
-        d.nbr4 + list_base(g.i, P.maxN), d.cnt[g.i], g,
-        [&](uint32_t j) { return XV{ld(d.X, j), ld(d.V, j)}; },
+        list, g, sums, [&](uint32_t j) { return XV{ld(d.X, j), ld(d.V, j)}; },
         [&](const XV& nb, float (&t)[3]) {
             f3 vij = make3(nb.v) - vi;
             f3 sep = xi - make3(nb.x);
             const f3 c = cross3(vij, grad_or_zero<kFast>(sep, dot3(sep, sep), P));
             const f3 u = (kFast ? -1.0f : -nb.x.w) * c;
             t[0] = u.x; t[1] = u.y; t[2] = u.z;
-        },
-        acc, wave_rows<3>(lds));
-    if (g.r != 0) return;
-    const f3 w{acc[0], acc[1], acc[2]};
+        });
+    const f3 w{sums.of(g, 0), sums.of(g, 1), sums.of(g, 2)};
+    if (g.r != 0u || g.i >= sc.end) return;
     const float wl = length3(w);
     d.W[g.i] = make_float4(w.x, w.y, w.z, wl);
     d.XsB[g.i] = make_float4(xi.x, xi.y, xi.z, wl);
 }
 
-template <int BS, int L, bool kFast>
-__global__ __launch_bounds__(BS) void k_confinement_group(DeviceState d, SphParams P, StepParams S) {
-    __shared__ float lds[(BS / 64) * 3 * 64];
-    const LaneGroup<L> g = lane_group<L>(xcd_slot<BS>());
-    if (g.i >= d.nslots || g.i >= scene_of(d, g.i).end) return;
+template <int L, bool kFast>
+__global__ __launch_bounds__(kGroupBlock) void k_confinement_group(DeviceState d, SphParams P, StepParams S) {
+    __shared__ float4 lds[group_lds_floats<L, 3>() / 4u];
+    const LaneGroup<L> g = lane_group<L>();
+    if (g.i >= d.nslots) return;
+    const GroupList<L> list = group_list<L>(d, P, g);
+    const SceneDev& sc = scene_of(d, g.i);
     const float4 xi4 = d.X[g.i];
     const f3 xi = make3(xi4);
-    const float4 wi = d.W[g.i];
-    const float invD = 1.0f / d.dens[g.i];
-    float acc[3] = {0.0f, 0.0f, 0.0f};
+    const float4 wi = d.W[g.i], vi = d.V[g.i];
+    const float rho = d.dens[g.i];
+    GroupSums<L, 3> sums(g, 0.0f, reinterpret_cast<float*>(lds));
     walk_split<L, 3, XW>(
-        d.nbr4 + list_base(g.i, P.maxN), d.cnt[g.i], g,
-        [&](uint32_t j) { return XW{ld(d.XsB, j), kFast ? 1.0f : ld(d.X, j).w}; },
+        list, g, sums, [&](uint32_t j) { return XW{ld(d.XsB, j), kFast ? 1.0f : ld(d.X, j).w}; },
         [&](const XW& nb, float (&t)[3]) {
             float diff = wi.w - nb.x.w;
             f3 sep = xi - make3(nb.x);
             const f3 gr = grad_or_zero<kFast>(sep, dot3(sep, sep), P);
             const f3 u = (kFast ? diff : nb.w * diff) * gr;
             t[0] = u.x; t[1] = u.y; t[2] = u.z;
-        },
-        acc, wave_rows<3>(lds));
-    if (g.r != 0) return;
-    confine_finish(d, P, S, g.i, xi4.w, wi, f3{acc[0], acc[1], acc[2]}, invD);
+        });
+    const f3 eta{sums.of(g, 0), sums.of(g, 1), sums.of(g, 2)};
+    if (g.r != 0u || g.i >= sc.end) return;
+    confine_finish(d, P, S, g.i, xi4.w, wi, vi, eta, rho);
 }
 
-template <int BS, int L>
-__global__ __launch_bounds__(BS) void k_xsph_group(DeviceState d, SphParams P) {
-    __shared__ float lds[(BS / 64) * 3 * 64];
-    const LaneGroup<L> g = lane_group<L>(xcd_slot<BS>());
-    if (g.i >= d.nslots || g.i >= scene_of(d, g.i).end) return;
+template <int L>
+__global__ __launch_bounds__(kGroupBlock) void k_xsph_group(DeviceState d, SphParams P) {
+    __shared__ float4 lds[group_lds_floats<L, 3>() / 4u];
+    const LaneGroup<L> g = lane_group<L>();
+    if (g.i >= d.nslots) return;
+    const GroupList<L> list = group_list<L>(d, P, g);
+    const SceneDev& sc = scene_of(d, g.i);
     const f3 xi = make3(d.X[g.i]);
     const f3 vi = make3(d.Vc[g.i]);
-    float acc[3] = {0.0f, 0.0f, 0.0f};
+    GroupSums<L, 3> sums(g, 0.0f, reinterpret_cast<float*>(lds));
     walk_split<L, 3, XV>(
-        d.nbr4 + list_base(g.i, P.maxN), d.cnt[g.i], g,
-        [&](uint32_t j) { return XV{ld(d.X, j), ld(d.Vc, j)}; },
+        list, g, sums, [&](uint32_t j) { return XV{ld(d.X, j), ld(d.Vc, j)}; },
         [&](const XV& nb, float (&t)[3]) {
             f3 vij = make3(nb.v) - vi;
             f3 sep = xi - make3(nb.x);
             float w = poly6(dot3(sep, sep), P);
             const f3 u = (nb.v.w * vij) * w;
             t[0] = u.x; t[1] = u.y; t[2] = u.z;
-        },
-        acc, wave_rows<3>(lds));
-    if (g.r != 0) return;
-    f3 vn = vi + P.visc * f3{acc[0], acc[1], acc[2]};
+        });
+    const f3 dv{sums.of(g, 0), sums.of(g, 1), sums.of(g, 2)};
+    if (g.r != 0u || g.i >= sc.end) return;
+    f3 vn = vi + P.visc * dv;
     d.V[g.i] = make_float4(vn.x, vn.y, vn.z, 0.0f);
 }
 
@@ -2048,8 +2169,8 @@ inline unsigned grid_xcd(uint32_t n, int bs) {
         }                               \
     } while (0)
 
-inline unsigned grid_lanes(uint32_t nslots, int lanes, int bs) {
-    return grid_xcd(nslots * (uint32_t)lanes, bs);
+inline unsigned grid_lanes(uint32_t nslots, int lanes) {
+    return grid_xcd(nslots * (uint32_t)lanes, kGroupBlock);
 }
 
 }  // namespace
@@ -2142,11 +2263,14 @@ void density_lambda_bs(hipStream_t st, const DeviceState& d, const SphParams& P,
 void launch_density_lambda(hipStream_t st, const DeviceState& d, const SphParams& P,
                            const float4* Xs, int bs, int residSlot, bool gated, int lanes) {
     if (lanes > 1) {
-        const unsigned g = grid_lanes(d.nslots, lanes, bs);
-        if (P.fast)
-            AKUA_BY_BLOCK(bs, AKUA_BY_LANES(lanes, (k_density_lambda_group<BS, L, true><<<g, BS, 0, st>>>(d, P, Xs))));
-        else
-            AKUA_BY_BLOCK(bs, AKUA_BY_LANES(lanes, (k_density_lambda_group<BS, L, false><<<g, BS, 0, st>>>(d, P, Xs))));
+        const unsigned g = grid_lanes(d.nslots, lanes);
+#define AKUA_DLG(K, B) AKUA_BY_LANES(lanes, (k_density_lambda_group<L, K, B><<<g, kGroupBlock, 0, st>>>(d, P, Xs)))
+        if (P.bd.on) {
+            if (P.fast) AKUA_DLG(true, true); else AKUA_DLG(false, true);
+        } else {
+            if (P.fast) AKUA_DLG(true, false); else AKUA_DLG(false, false);
+        }
+#undef AKUA_DLG
         return;
     }
     AKUA_BY_BLOCK(bs, (density_lambda_bs<BS>(st, d, P, Xs, residSlot, gated)));
@@ -2210,13 +2334,19 @@ void launch_delta_correct(hipStream_t st, const DeviceState& d, const SphParams&
                           const StepParams& S, const float4* XsIn, float4* XsOut, bool final,
                           bool applyDelta, int bs, int gate, const float4* XsAlt, int lanes) {
     if (lanes > 1 && applyDelta) {
-        const unsigned g = grid_lanes(d.nslots, lanes, bs);
-#define AKUA_DCG(F, K) \
-    AKUA_BY_BLOCK(bs, AKUA_BY_LANES(lanes, (k_delta_correct_group<BS, L, F, K><<<g, BS, 0, st>>>(d, P, S, XsIn, XsOut))))
-        if (final) {
-            if (P.fast) AKUA_DCG(true, true); else AKUA_DCG(true, false);
+        const unsigned g = grid_lanes(d.nslots, lanes);
+#define AKUA_DCG(F, K, B) \
+    AKUA_BY_LANES(lanes, (k_delta_correct_group<L, F, K, B><<<g, kGroupBlock, 0, st>>>(d, P, S, XsIn, XsOut)))
+        if (P.bd.on) {
+            if (final) {
+                if (P.fast) AKUA_DCG(true, true, true); else AKUA_DCG(true, false, true);
+            } else {
+                if (P.fast) AKUA_DCG(false, true, true); else AKUA_DCG(false, false, true);
+            }
+        } else if (final) {
+            if (P.fast) AKUA_DCG(true, true, false); else AKUA_DCG(true, false, false);
         } else {
-            if (P.fast) AKUA_DCG(false, true); else AKUA_DCG(false, false);
+            if (P.fast) AKUA_DCG(false, true, false); else AKUA_DCG(false, false, false);
         }
 #undef AKUA_DCG
         return;
@@ -2226,11 +2356,11 @@ void launch_delta_correct(hipStream_t st, const DeviceState& d, const SphParams&
 }
 void launch_vorticity(hipStream_t st, const DeviceState& d, const SphParams& P, int bs, int lanes) {
     if (lanes > 1) {
-        const unsigned g = grid_lanes(d.nslots, lanes, bs);
+        const unsigned g = grid_lanes(d.nslots, lanes);
         if (P.fast)
-            AKUA_BY_BLOCK(bs, AKUA_BY_LANES(lanes, (k_vorticity_group<BS, L, true><<<g, BS, 0, st>>>(d, P))));
+            AKUA_BY_LANES(lanes, (k_vorticity_group<L, true><<<g, kGroupBlock, 0, st>>>(d, P)));
         else
-            AKUA_BY_BLOCK(bs, AKUA_BY_LANES(lanes, (k_vorticity_group<BS, L, false><<<g, BS, 0, st>>>(d, P))));
+            AKUA_BY_LANES(lanes, (k_vorticity_group<L, false><<<g, kGroupBlock, 0, st>>>(d, P)));
         return;
     }
     if (P.fast)
@@ -2241,11 +2371,11 @@ void launch_vorticity(hipStream_t st, const DeviceState& d, const SphParams& P, 
 void launch_confinement(hipStream_t st, const DeviceState& d, const SphParams& P,
                         const StepParams& S, int bs, int lanes) {
     if (lanes > 1) {
-        const unsigned g = grid_lanes(d.nslots, lanes, bs);
+        const unsigned g = grid_lanes(d.nslots, lanes);
         if (P.fast)
-            AKUA_BY_BLOCK(bs, AKUA_BY_LANES(lanes, (k_confinement_group<BS, L, true><<<g, BS, 0, st>>>(d, P, S))));
+            AKUA_BY_LANES(lanes, (k_confinement_group<L, true><<<g, kGroupBlock, 0, st>>>(d, P, S)));
         else
-            AKUA_BY_BLOCK(bs, AKUA_BY_LANES(lanes, (k_confinement_group<BS, L, false><<<g, BS, 0, st>>>(d, P, S))));
+            AKUA_BY_LANES(lanes, (k_confinement_group<L, false><<<g, kGroupBlock, 0, st>>>(d, P, S)));
         return;
     }
     if (P.fast)
@@ -2255,8 +2385,8 @@ void launch_confinement(hipStream_t st, const DeviceState& d, const SphParams& P
 }
 void launch_xsph(hipStream_t st, const DeviceState& d, const SphParams& P, int bs, int lanes) {
     if (lanes > 1) {
-        const unsigned g = grid_lanes(d.nslots, lanes, bs);
-        AKUA_BY_BLOCK(bs, AKUA_BY_LANES(lanes, (k_xsph_group<BS, L><<<g, BS, 0, st>>>(d, P))));
+        const unsigned g = grid_lanes(d.nslots, lanes);
+        AKUA_BY_LANES(lanes, (k_xsph_group<L><<<g, kGroupBlock, 0, st>>>(d, P)));
         return;
     }
     AKUA_BY_BLOCK(bs, (k_xsph<BS><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));

@@ -658,6 +658,25 @@ void sort_layout(akua_solver* s, hipStream_t st, bool timed) {
 // sweep, then vorticity, confinement and XSPH.
 uint32_t queue_passes(const akua_solver* s) { return 2u * (uint32_t)s->cfg.solverIterations + 3u; }
 
+// Lanes per particle in the neighbour sweeps: the setting, or, left to the solver, by the slots.  Up to
+// 2^18 as many as keep the chip's 1,024 SIMDs at a few waves each; measured, us per step with 1 / 2 / 4 /
+// 8 / 16 lanes: 4,000 particles 198 / 153 / 125 / 112 / 103, 27,000 203 / 163 / 138 / 142 / 138 (with
+// wall samples 297 / 265 / 201 / 189 / 172), 60,000 223 / 190 / 183 / 197 / 199, 200,000 385 / 378 / 381 /
+// 424 / 463 (uneven masses 547 / 516 / 505 / 538 / 574), 400,000 578 / 580 / 591 / 689 / 783.
+// In larger scenes the sweeps that wait for their gathers keep a few, those bound by arithmetic one;
+// us at 1M with 1 / 2 / 4 lanes: density and lambda 55 / 64 / 64, position delta 67 / 69 / 66, the
+// last one 83 / 78 / 83, vorticity 94 / 82 / 79, confinement 55 / 50 / 53, XSPH 92 / 75 / 72.
+struct SweepLanes {
+    int jacobi, last, vorticity, confinement, xsph;
+};
+SweepLanes sweep_lanes(const akua_solver* s) {
+    const auto all = [](int n) { return SweepLanes{n, n, n, n, n}; };
+    if (s->tuning.laneGroup > 0) return all(s->tuning.laneGroup);
+    if (s->nslots <= (1u << 15)) return all(16);
+    if (s->nslots <= (1u << 18)) return all(4);
+    return SweepLanes{1, 2, 4, 2, 4};
+}
+
 void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool timed,
                   bool record = false, bool keepLayout = false) {
     Launcher L{s, st, timed};
@@ -695,15 +714,15 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
     const int bs = s->tuning.block;
     const int I = s->cfg.solverIterations;
     const bool learned = s->mode == 1 && !record;
-    const bool plainOrder = !d.work && P.searchCells == 1 && !P.bd.on;
-    // small scenes: lane groups in the sweeps of a plain step
-    const int lanesSet = s->tuning.laneGroup > 1 && plainOrder && !learned && !record ? s->tuning.laneGroup : 1;
+    // small scenes: lane groups in the sweeps of a plain step, and in those after the position update
+    // of every step
+    const bool plainOrder = !d.work && P.searchCells == 1;
+    SweepLanes lanes = plainOrder ? sweep_lanes(s) : SweepLanes{1, 1, 1, 1, 1};
     // with the work queue too, the queue runs the Jacobi sweeps and confinement, and the lane groups run vorticity and XSPH (two gathered records per neighbour, whose latency
     // more lanes per particle hide better)
     const bool queueSet = s->tuning.workQueue > 0 && !learned && !record && s->queue.p &&
                           s->heads.n >= queue_heads_size(queue_passes(s));
-    const int lanes = queueSet ? 1 : lanesSet;
-    const int postLanes = lanesSet;
+    if (queueSet || learned || record) lanes.jacobi = lanes.last = 1;
     // the sweeps of a plain step as persistent launches over each XCD's queue of tiles
     const bool queued = queueSet;
     uint32_t pass = 0;
@@ -765,7 +784,7 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
         if (queued)
             launch_density_lambda_queue(st, d, P, in, pass++);
         else
-            launch_density_lambda(st, d, P, in, bs, record && it == I - Jt ? 2 : -1, learned, lanes);
+            launch_density_lambda(st, d, P, in, bs, record && it == I - Jt ? 2 : -1, learned, lanes.jacobi);
         L.after(learned ? "density_lambda_fallback" : "density_lambda");
         if (record && it == I - Jt) {
             L.before("targets");
@@ -781,26 +800,26 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
             launch_delta_correct_queue(st, d, P, S, in, out, last, pass++);
         else
             launch_delta_correct(st, d, P, S, in, out, last, true, bs, learned ? (last ? 2 : 1) : 0,
-                                 learned ? ws(J - 1) : nullptr, lanes);
+                                 learned ? ws(J - 1) : nullptr, last ? lanes.last : lanes.jacobi);
         L.after(name);
     }
     L.before("vorticity");
-    if (queued && postLanes == 1)
+    if (queued && lanes.vorticity == 1)
         launch_vorticity_queue(st, d, P, pass++);
     else
-        launch_vorticity(st, d, P, bs, postLanes);
+        launch_vorticity(st, d, P, bs, lanes.vorticity);
     L.after("vorticity");
     L.before("confinement");
     if (queued)
         launch_confinement_queue(st, d, P, S, pass++);
     else
-        launch_confinement(st, d, P, S, bs, lanes);
+        launch_confinement(st, d, P, S, bs, lanes.confinement);
     L.after("confinement");
     L.before("xsph");
-    if (queued && postLanes == 1)
+    if (queued && lanes.xsph == 1)
         launch_xsph_queue(st, d, P, pass++);
     else
-        launch_xsph(st, d, P, bs, postLanes);
+        launch_xsph(st, d, P, bs, lanes.xsph);
     L.after("xsph");
 }
 

@@ -161,13 +161,14 @@ typedef struct akua_tuning {
                                  list build that one form has replaced) */
     int32_t fuseSweep;        /* 0 or 1: accepted and without effect (it ran the first sweep in the
                                  list build's launch, which costs more than it saves since) */
-    int32_t laneGroup;        /* 0 (the default): one thread per particle; 2, 4, 8 or 16: for scenes
-                                 too small to fill the chip, the neighbour sweeps of a plain step
-                                 run that many lanes per particle (each list's terms in parallel,
-                                 summed in list order); applies with balanceTile 0, the reference's
-                                 search and no boundary samples.  With workQueue set too, only the
-                                 vorticity and XSPH sweeps run in lane groups; the queue runs the
-                                 others */
+    int32_t laneGroup;        /* lanes per particle in the neighbour sweeps (each list's terms in
+                                 parallel, summed in list order), for scenes too small to fill the
+                                 chip: 0 (the default) by the number of particles (one for large
+                                 scenes), or 2, 4, 8 or 16; applies with balanceTile 0 and the
+                                 reference's search, in learned and training steps only to the
+                                 sweeps after the position update.  With workQueue set too, only
+                                 the vorticity and XSPH sweeps run in lane groups; the queue runs
+                                 the others */
     int32_t workQueue;        /* 0 (the default): each neighbour sweep after the list build is one
                                  launch with a workgroup per block of slots; 1 or 2: after the list
                                  build, the 256-slot tiles each XCD serves are queued heaviest first

@@ -1,0 +1,62 @@
+"""Lane groups in the neighbour sweeps (several lanes per particle, sums in list order), bit for bit
+against the FP32 oracle: lists that end inside, at and past a group's round, uneven masses, wall
+samples whose windows take several rounds, and the sizes at which the default changes its group."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+DT = 0.004
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+    if torch.cuda.device_count() < 1:
+        pytest.fail("no GPU visible: the gpu tests need an MI355X")
+    from akuaengine_amd.solver import PBFSolver
+    return PBFSolver
+
+
+def _check(gpu, oracle_mod, cfg, corr, pos, mass, lo, hi, layers, lanes, steps):
+    s = gpu(len(pos), cfg, corr)
+    o = oracle_mod.Oracle(len(pos), cfg, corr, 32)
+    for x in (s, o):
+        x.set_state(pos, np.zeros_like(pos), mass)
+        if layers:
+            x.set_boundary(layers, 0.0)
+    if lanes:
+        s.set_tuning(laneGroup=lanes)
+    for _ in range(steps):
+        s.step(DT, lo, hi)
+        o.step(DT, lo, hi)
+    g, r = s.get_state(), o.state()
+    for k in ("pos", "vel", "density", "lam", "ids"):
+        np.testing.assert_array_equal(g[k], r[k].astype(g[k].dtype), err_msg=k)
+    return s.debug_neighbours()[1]
+
+
+@pytest.mark.parametrize("layers", [0, 1, 3])
+@pytest.mark.parametrize("cap", [3, 8, 9, 31, 32, 33, 64, 65, 90])
+@pytest.mark.parametrize("lanes", [2, 4, 8, 16])
+def test_list_lengths(gpu, oracle_mod, dam_params, lanes, cap, layers):
+    from akuaengine_amd import scenes
+    cfg, corr = dam_params
+    cfg = dataclasses.replace(cfg, maxNeighbours=cap)
+    rng = np.random.default_rng(cap)
+    pos = scenes.lattice(11, 9, 7, 0.035, (0.02, 0.02, 0.02))  # about 95 neighbours inside
+    pos = (pos + rng.uniform(-0.004, 0.004, pos.shape)).astype(np.float32)
+    mass = rng.uniform(0.5, 1.5, len(pos)).astype(np.float32) if cap % 2 else None
+    print(f"[lane groups] {lanes} lanes, cap {cap}, {layers} layers", flush=True)
+    cnt = _check(gpu, oracle_mod, cfg, corr, pos, mass, (0.0, 0.0, 0.0), (0.7, 0.5, 0.27), layers, lanes, 2)
+    assert cnt.max() == cap
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 32767, 32769, 262145])
+def test_default_group_by_size(gpu, oracle_mod, dam_params, n):
+    from akuaengine_amd import scenes
+    cfg, corr = dam_params
+    sc = scenes.batched_scene(n, index=n % 5)
+    print(f"[lane groups] n={n}", flush=True)
+    _check(gpu, oracle_mod, cfg, corr, sc.pos, None, sc.box_min, sc.box_max, 0, 0, 2)
