@@ -36,10 +36,11 @@ struct MlpLossWeights {
     float w[4];
 };
 
-// Workgroups of the gradient kernel: each of its kMlpGradWaves waves writes one partial row.
-constexpr int kMlpGradBlocks = 128;
-constexpr int kMlpGradWaves = 2;
-constexpr int kMlpPartRows = kMlpGradBlocks * kMlpGradWaves;
+// The gradient kernel: a workgroup of four waves takes kMlpGradSamples samples at a time and writes one
+// partial row; at most kMlpPartRows workgroups (16,384 samples at one round each).
+constexpr int kMlpGradWaves = 4;
+constexpr int kMlpGradSamples = 16 * kMlpGradWaves;
+constexpr int kMlpPartRows = 256;
 
 struct DeviceState;
 
@@ -51,15 +52,15 @@ void launch_mlp_eval(hipStream_t st, const float* params, const float* feat, uin
 void launch_mlp_apply(hipStream_t st, const DeviceState& d, const float* params, float h,
                       const float4* XsPred, float4* XsWarm, float* lamHat);
 
-// Per-wave gradient partials of the mean loss over n samples (rows of feat/targ), for
-// launch_mlp_reduce / launch_mlp_adam.  part: kMlpPartRows * kMlpPartRow floats.
-void launch_mlp_grad(hipStream_t st, const float* params, const float* feat, const float* targ,
-                     uint32_t n, MlpLossWeights lw, float* part);
+// Gradient partials of the mean loss over n >= 1 samples (rows of feat/targ), for launch_mlp_reduce /
+// launch_mlp_adam.  part: kMlpPartRows * kMlpPartRow floats; returns the rows written.
+int launch_mlp_grad(hipStream_t st, const float* params, const float* feat, const float* targ,
+                    uint32_t n, MlpLossWeights lw, float* part);
 // Sums the partial rows in a fixed order: grad[kMlpTrainable], loss -> *loss.
-void launch_mlp_reduce(hipStream_t st, const float* part, float* grad, float* loss);
+void launch_mlp_reduce(hipStream_t st, const float* part, int rows, float* grad, float* loss);
 // Sums the partials and applies one Adam step to the trainable parameters in place.
 // c1 = 1 / (1 - beta1^t), c2 = 1 / (1 - beta2^t).
-void launch_mlp_adam(hipStream_t st, const float* part, float* params, float* m, float* v, float lr,
+void launch_mlp_adam(hipStream_t st, const float* part, int rows, float* params, float* m, float* v, float lr,
                      float beta1, float beta2, float eps, float c1, float c2, float* loss);
 
 }  // namespace akua

@@ -16,8 +16,8 @@ namespace akua {
 namespace {
 
 // The gradient partial rows of k_mlp_grad: kMlpPartRows rows of kMlpPartRow floats, 5.64 MB,
-// whatever the number of samples.  Every call rewrites every row before k_mlp_adam reads them,
-// so nothing needs clearing between calls.
+// whatever the number of samples.  Every call writes each row that its k_mlp_adam reads, so nothing
+// needs clearing between calls.
 constexpr size_t kScratchFloats = (size_t)kMlpPartRows * kMlpPartRow;
 static __device__ __align__(256) float scratch[kScratchFloats];
 
@@ -75,8 +75,8 @@ extern "C" akua_status akua_mlp_adam_step_device(float* params, float* m, float*
     const MlpLossWeights lw{{lossWeights[0], lossWeights[1], lossWeights[2], lossWeights[3]}};
     const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, (double)t)));
     const float c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)t)));
-    launch_mlp_grad(st, params, features, targets, (uint32_t)n, lw, part);
-    launch_mlp_adam(st, part, params, m, v, learningRate, 0.9f, 0.999f, 1e-8f, c1, c2, loss);
+    const int rows = launch_mlp_grad(st, params, features, targets, (uint32_t)n, lw, part);
+    launch_mlp_adam(st, part, rows, params, m, v, learningRate, 0.9f, 0.999f, 1e-8f, c1, c2, loss);
     e = hipGetLastError();
     if (e != hipSuccess) return fail_with(AKUA_ERR_HIP, std::string("launch: ") + hipGetErrorString(e));
     set_last_error("");

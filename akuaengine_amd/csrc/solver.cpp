@@ -1588,12 +1588,12 @@ void train(akua_solver* s, float dt, const float* bmin, const float* bmax, int s
         } else {
             for (int e = 0; e < c.epochs; ++e) {
                 for (uint32_t mb = 0; mb < nb; ++mb) {
-                    launch_mlp_grad(st, s->net.p, s->batchF.p + (size_t)mb * M * kMlpFeatures,
-                                    s->batchT.p + (size_t)mb * M * 4, M, lw, s->part.p);
+                    const int rows = launch_mlp_grad(st, s->net.p, s->batchF.p + (size_t)mb * M * kMlpFeatures,
+                                                     s->batchT.p + (size_t)mb * M * 4, M, lw, s->part.p);
                     s->adamT++;
                     const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, (double)s->adamT)));
                     const float c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)s->adamT)));
-                    launch_mlp_adam(st, s->part.p, s->net.p, s->adamM.p, s->adamV.p,
+                    launch_mlp_adam(st, s->part.p, rows, s->net.p, s->adamM.p, s->adamV.p,
                                     c.learningRate, b1, b2, eps, c1, c2,
                                     s->lossBuf.p + (size_t)k * perStep + (size_t)e * nb + mb);
                 }
@@ -2350,8 +2350,8 @@ akua_status akua_mlp_gradient(const float* params, const float* features, const 
         G.alloc(kMlpTrainable);
         L.alloc(1);
         MlpLossWeights lw{{lossWeights[0], lossWeights[1], lossWeights[2], lossWeights[3]}};
-        launch_mlp_grad(nullptr, P.p, F.p, T.p, (uint32_t)n, lw, part.p);
-        launch_mlp_reduce(nullptr, part.p, G.p, L.p);
+        const int rows = launch_mlp_grad(nullptr, P.p, F.p, T.p, (uint32_t)n, lw, part.p);
+        launch_mlp_reduce(nullptr, part.p, rows, G.p, L.p);
         HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipDeviceSynchronize());
         HIP_CHECK(hipMemcpy(grad, G.p, kMlpTrainable * sizeof(float), hipMemcpyDeviceToHost));
@@ -2377,8 +2377,8 @@ akua_status akua_mlp_adam_step(float* params, float* m, float* v, int64_t t, flo
         MlpLossWeights lw{{lossWeights[0], lossWeights[1], lossWeights[2], lossWeights[3]}};
         const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, (double)t)));
         const float c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)t)));
-        launch_mlp_grad(nullptr, P.p, F.p, T.p, (uint32_t)n, lw, part.p);
-        launch_mlp_adam(nullptr, part.p, P.p, M.p, V.p, lr, 0.9f, 0.999f, 1e-8f, c1, c2, L.p);
+        const int rows = launch_mlp_grad(nullptr, P.p, F.p, T.p, (uint32_t)n, lw, part.p);
+        launch_mlp_adam(nullptr, part.p, rows, P.p, M.p, V.p, lr, 0.9f, 0.999f, 1e-8f, c1, c2, L.p);
         HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipDeviceSynchronize());
         HIP_CHECK(hipMemcpy(params, P.p, kMlpParams * sizeof(float), hipMemcpyDeviceToHost));
