@@ -6,7 +6,8 @@
 //               neighbour-list order, the permutation tap and akua_solver_get_state use it.
 //   physical -- where the particle's data lives in HBM: sorted by the Morton code of its
 //               2x2x2 super-cell (ties in logical order), so the 64 particles of a wave are
-//               spatial neighbours and their neighbour gathers hit the same cache lines.
+//               spatial neighbours and their neighbour gathers hit the same cache lines; in small
+//               scenes (launch_order) the logical order.
 // lid[p] is the logical index of physical slot p (kept by the step); its inverse, the physical slot
 // of each logical index, is physT during a step and is rebuilt from lid where needed outside it.
 // Every per-particle sum runs over the neighbour list in the reference's order, so the physical
@@ -68,6 +69,14 @@ struct DeviceState {
     uint32_t* keysL;           // hashes at their previous logical index (first sort's input)
     const uint32_t* skeys;     // hashes in logical order (first sort's output)
     const uint32_t* perm1;     // logical index -> previous logical index
+    // small scenes (launch_order): particles per group of hashes, the groups' first places, and
+    // (hash, previous logical index, previous physical slot, 0) at each place
+    uint32_t* groupCount;
+    uint32_t* groupBase;
+    uint4* placed;
+    uint32_t groups, groupShift;  // a hash's group is its bits from groupShift on
+    uint32_t* skeysOut;        // skeys and perm1, for their writer
+    uint32_t* perm1Out;
     uint32_t* keysM;           // super-cell Morton keys in logical order (second sort's input)
     const uint32_t* perm2;     // physical slot -> logical index
     uint32_t* perm2keep;       // the same map for a step that keeps the physical layout
@@ -140,6 +149,11 @@ void launch_gather(hipStream_t st, const DeviceState& d, const SphParams& P, con
 // Physical start and contiguity of every bucket (after the gather).
 void launch_bucket_phys(hipStream_t st, const DeviceState& d);
 // phys[lid[p]] = p over every scene's slots.
+// Small single scenes: hashes, both orders (the physical is the logical), the cell table and the move,
+// instead of launch_predict_hash, the two sorts, launch_cell_keys, launch_gather and launch_bucket_phys.
+constexpr uint32_t kOrderMaxSlots = 1u << 17, kOrderMaxGroups = 1u << 13;
+void launch_order(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
+                  bool carryDelta);
 void launch_invert_order(hipStream_t st, const DeviceState& d, uint32_t* phys);
 // The neighbour lists.  Below: bs is the workgroup size of the neighbour sweeps (128, 256 or 512;
 // results do not depend on it).

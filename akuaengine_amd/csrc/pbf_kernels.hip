@@ -302,6 +302,165 @@ __global__ __launch_bounds__(kBlock) void k_gather(DeviceState d, SphParams P, S
     d.physT[k] = p;
 }
 
+// Inclusive prefix sum over the wave's 64 lanes.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
+    int x = (int)v;
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)x;
+}
+
+// ---- small scenes: both orders from one counting pass ----------------------------------------------
+// Up to kOrderMaxSlots slots of a single scene take three launches where the two radix sorts, the cell
+// table and the move take thirteen, each at the launch's own cost (27,000 particles: 85 us of a 235 us
+// step before, 14 now; 1,000: 57 and 13).  The physical order is the logical order: the particles of a
+// cell are still neighbours in memory, and the arrays of such a scene fit the caches.  The sweeps lose
+// a little to it where they no longer do, which sets the limit: us per step against the (paired) sorts
+// and the cell order, 27,000 particles 107 / 139, 60,000 157 / 183, 100,000 221 / 243, 130,000 258 / 271
+// (sprayed 291 / 292).
+//   1. k_order_count: hashes; each particle takes a place in the group of its hash's upper bits;
+//   2. k_order_place: the groups' prefix (each workgroup its own, in LDS), hashes to their groups;
+//   3. k_order_rank: each particle's rank by (hash, previous logical index) among its group's few
+//      members, which also gives its bucket's bounds: the move and the table entry.
+constexpr uint32_t kOrderBlock = 1024;
+
+// Groups are counted by runs: particles of one cell mostly lie side by side.
+__global__ __launch_bounds__(kBlock) void k_order_count(DeviceState d, SphParams P, StepParams S, uint32_t countBlocks) {
+    if (blockIdx.x >= countBlocks) {
+        const uint32_t i = (blockIdx.x - countBlocks) * kBlock + threadIdx.x;
+        if (i < d.tableTotal) d.table[i] = make_uint4(kEmptyKey, kEmptyKey, kEmptyKey, kEmptyKey);
+        return;
+    }
+    const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    const SceneDev& sc = d.scenes[0];
+    const bool valid = p < d.nslots;
+    uint32_t h = 0, k = 0, group = kEmptyKey;
+    if (valid) {
+        k = d.lid[p];
+        const f3 xs = predict_x(make3(d.X[p]), make3(d.V[p]), S);
+        int cx, cy, cz;
+        discretize(xs, P.cellHash, cx, cy, cz);
+        h = cell_hash(cx, cy, cz, sc);
+        group = h >> d.groupShift;
+    }
+    const uint32_t lane = __lane_id();
+    const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)group, 0x138, 0xF, 0xF, false);  // wave_shr:1
+    const uint64_t heads = __ballot(lane == 0u || before != group);
+    const uint32_t head = 63u - (uint32_t)__builtin_clzll(heads & (~0ull >> (63u - lane)));
+    uint32_t place = 0;
+    if (valid && lane == head) {
+        const uint64_t after = lane == 63u ? 0ull : heads & (~0ull << (lane + 1u));
+        const uint32_t end = after ? (uint32_t)__builtin_ctzll(after) : 64u;
+        place = atomicAdd(&d.groupCount[group], end - lane);  // the lanes past the last slot are a run of their own
+    }
+    place = (uint32_t)__shfl((int)place, (int)head, 64) + (lane - head);
+    if (!valid || k >= d.nslots) return;  // a consistent order never produces k >= nslots
+    d.keysL[k] = h;
+    d.layPhys[k] = make_uint2(place, p);
+}
+
+__global__ __launch_bounds__(kOrderBlock) void k_order_place(DeviceState d) {
+    __shared__ uint32_t base[kOrderMaxGroups];
+    __shared__ uint32_t waveSum[kOrderBlock / 64];
+    const uint32_t t = threadIdx.x;
+    const uint32_t k = blockIdx.x * kOrderBlock + t;
+    uint32_t h = 0;
+    uint2 r = make_uint2(0u, 0u);
+    if (k < d.nslots) {
+        h = d.keysL[k];
+        r = d.layPhys[k];
+    }
+    // eight consecutive counts per thread (groups is a multiple of 8, the rest of the array is zero)
+    constexpr uint32_t kPer = kOrderMaxGroups / kOrderBlock;
+    static_assert(kPer == 8, "two chunks of four");
+    uint32_t c[kPer] = {};
+    if (t * kPer < d.groups) {
+        const uint4* const g = reinterpret_cast<const uint4*>(d.groupCount) + 2u * t;
+        const uint4 a = g[0], b = g[1];
+        c[0] = a.x; c[1] = a.y; c[2] = a.z; c[3] = a.w;
+        c[4] = b.x; c[5] = b.y; c[6] = b.z; c[7] = b.w;
+    }
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; ++u) sum += c[u];
+    const uint32_t inclusive = wave_prefix(sum);
+    if (__lane_id() == 63u) waveSum[t >> 6] = inclusive;
+    __syncthreads();
+    uint32_t run = inclusive - sum;
+    for (uint32_t w = 0; w < (t >> 6); ++w) run += waveSum[w];
+#pragma unroll
+    for (uint32_t u = 0; u < kPer; ++u) {
+        base[t * kPer + u] = run;
+        run += c[u];
+    }
+    __syncthreads();
+    if (blockIdx.x == 0) {
+        for (uint32_t g = t; g < d.groups; g += kOrderBlock) d.groupBase[g] = base[g];
+        if (t == 0) d.groupBase[d.groups] = d.nslots;
+    }
+    if (k >= d.nslots) return;
+    const uint32_t q = base[(h >> d.groupShift) & (kOrderMaxGroups - 1u)] + r.x;
+    if (q < d.nslots) d.placed[q] = make_uint4(h, k, r.y, 0u);
+}
+
+// kCarry, kCarryDelta: as in k_gather.
+template <bool kCarry, bool kCarryDelta>
+__global__ __launch_bounds__(kBlock) void k_order_rank(DeviceState d, StepParams S) {
+    const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
+    // the counts were read by the launch before: empty for the next step
+    for (uint32_t g = q; g < d.groups; g += gridDim.x * kBlock) d.groupCount[g] = 0u;
+    if (q >= d.nslots) return;
+    const SceneDev& sc = d.scenes[0];
+    const uint4 me = d.placed[q];
+    const uint32_t h = me.x, k = me.y, src = me.z, group = h >> d.groupShift;
+    if (k >= d.nslots || src >= d.nslots || group >= d.groups) return;  // consistent counts never produce these
+    const float4 x = d.X[src], v = d.V[src];
+    const uint32_t id = d.id[src];
+    const uint32_t b = d.groupBase[group], e = min(d.groupBase[group + 1u], d.nslots);
+    uint32_t smaller = 0, same = 0, sameBefore = 0;
+    constexpr uint32_t kBatch = 8;
+    for (uint32_t m0 = b; m0 < e; m0 += kBatch) {
+        uint2 o[kBatch];
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) o[u] = *reinterpret_cast<const uint2*>(&d.placed[min(m0 + u, e - 1u)]);
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) {
+            const bool in = m0 + u < e;
+            smaller += in && o[u].x < h ? 1u : 0u;
+            same += in && o[u].x == h ? 1u : 0u;
+            sameBefore += in && o[u].x == h && o[u].y < k ? 1u : 0u;
+        }
+    }
+    const uint32_t first = b + smaller, to = first + sameBefore;
+    if (to >= d.nslots) return;  // consistent counts never produce this
+    if (sameBefore == 0u) {
+        const uint32_t slot = table_insert(d.table, sc, h);
+        if (slot != kEmptyKey) {
+            d.table[slot].y = first;
+            d.table[slot].z = first + same;
+            // physical order is logical order: the bucket is one run (256 particles at most, as in k_bucket_phys)
+            d.table[slot].w = first | (same <= 256u ? 0x80000000u : 0u);
+        }
+    }
+    d.skeysOut[to] = h;
+    d.perm1Out[to] = k;
+    const f3 xs = predict_x(make3(x), make3(v), S);
+    d.X0[to] = x;
+    d.XsA[to] = make_float4(xs.x, xs.y, xs.z, x.w);
+    if (kCarry) {
+        d.Tdens[to] = d.dens[src];
+        d.Tlam[to] = d.lam[src];
+    }
+    if (kCarryDelta) d.TDP[to] = d.DP[src];
+    d.Tid[to] = id;
+    d.lidT[to] = to;
+    d.physT[to] = to;
+}
+
 // The physical slot of each logical index from the step's persistent lid (outside a step, where
 // physT no longer holds it: rendering draws in logical order).
 __global__ __launch_bounds__(kBlock) void k_invert_order(DeviceState d, uint32_t* __restrict__ phys) {
@@ -542,18 +701,6 @@ __device__ __forceinline__ void wave_lds_order() {
 
 __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-// Inclusive prefix sum over the wave's 64 lanes.
-__device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
-    int x = (int)v;
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
-    return (uint32_t)x;
 }
 
 __device__ __forceinline__ uint32_t lane_u(uint32_t v, uint32_t lane) {
@@ -2205,6 +2352,18 @@ void launch_gather(hipStream_t st, const DeviceState& d, const SphParams& P, con
         k_gather<true, false><<<grid(d.nslots), kBlock, 0, st>>>(d, P, S, layoutPrev);
     else
         k_gather<false, false><<<grid(d.nslots), kBlock, 0, st>>>(d, P, S, layoutPrev);
+}
+void launch_order(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
+                  bool carryDelta) {
+    const uint32_t count = grid(d.nslots);
+    k_order_count<<<count + grid(d.tableTotal), kBlock, 0, st>>>(d, P, S, count);
+    k_order_place<<<(d.nslots + kOrderBlock - 1) / kOrderBlock, kOrderBlock, 0, st>>>(d);
+    if (carryDelta)
+        k_order_rank<true, true><<<count, kBlock, 0, st>>>(d, S);
+    else if (carry)
+        k_order_rank<true, false><<<count, kBlock, 0, st>>>(d, S);
+    else
+        k_order_rank<false, false><<<count, kBlock, 0, st>>>(d, S);
 }
 void launch_invert_order(hipStream_t st, const DeviceState& d, uint32_t* phys) {
     k_invert_order<<<grid(d.nslots), kBlock, 0, st>>>(d, phys);

@@ -214,6 +214,8 @@ struct Staging {
 
 }  // namespace
 
+constexpr akua_tuning kDefaultTuning{256, 1, 0, 0, 1, 0, 0, 0, 0, 0};
+
 struct akua_solver {
     akua_pbf_config cfg{};
     akua_lambda_corr corr{};
@@ -231,7 +233,7 @@ struct akua_solver {
     int hashBits = 1;        // bits of the reference's hashes (log2 of the largest table size)
     SortPlan plan2;          // super-cell sort (physical layout)
     // block, layout level, digit bits (0: balanced), layout interval, balance tile
-    akua_tuning tuning{256, 1, 0, 0, 1, 0, 0, 0, 0, 0};
+    akua_tuning tuning = kDefaultTuning;
     int layoutPhase = 0;           // steps since the physical layout was last re-sorted (0: now)
     std::vector<SortTile> tilesHost;
     std::vector<SortScene> sortScenesHost;
@@ -245,6 +247,9 @@ struct akua_solver {
     DevBuf<float> dens, lam, Tdens, Tlam, size;
     DevBuf<uint32_t> id, Tid, lid, phys, lidT, physT, srcL, bslot, nbr, cnt, perm2keep;
     DevBuf<uint2> layPhys;
+    DevBuf<uint32_t> groupCount, groupBase;  // small scenes (launch_order); groupCount is zero between steps
+    DevBuf<uint4> placed;
+    uint32_t groups = 0;
     DevBuf<uint32_t> s1KA, s1VA, s1KB, s1VB, s2KA, s2VA, s2KB, s2VB, counts, totals, look, tickets;
     DevBuf<uint32_t> counts2, totals2, look2, tickets2;  // the layout sort's, beside the hash sort
     DevBuf<uint4> table;
@@ -332,8 +337,11 @@ struct akua_solver {
         d.srcL = srcL.p; d.layPhys = layPhys.p;
         const bool r1 = plan1.passes() % 2 == 1, r2 = plan2.passes() % 2 == 1;
         d.keysL = s1KA.p;
-        d.skeys = r1 ? s1KB.p : s1KA.p;
-        d.perm1 = r1 ? s1VB.p : s1VA.p;
+        d.skeys = d.skeysOut = r1 ? s1KB.p : s1KA.p;
+        d.perm1 = d.perm1Out = r1 ? s1VB.p : s1VA.p;
+        d.groupCount = groupCount.p; d.groupBase = groupBase.p; d.placed = placed.p;
+        d.groups = groups;
+        d.groupShift = (uint32_t)std::max(0, hashBits - (int)ceil_log2(groups));
         d.keysM = s2KA.p;
         d.perm2 = keepLayout ? perm2keep.p : (r2 ? s2VB.p : s2VA.p);
         d.perm2keep = perm2keep.p;
@@ -379,7 +387,7 @@ struct akua_solver {
                         &totals, &look, &tickets, &counts2, &totals2, &look2, &tickets2, &gate, &fallbacks, &work, &cntW, &nbrW, &qcost,
                         &queue, &qcount, &heads})
             b->release();
-        layPhys.release(); table.release(); dTiles.release(); dSortScenes.release(); nbrSum.release();
+        layPhys.release(); groupCount.release(); groupBase.release(); placed.release(); table.release(); dTiles.release(); dSortScenes.release(); nbrSum.release();
         probeMax.release(); probeSum.release(); renderKeys.release(); renderRgb.release();
         resid.release(); residPart.release(); residBlk.release(); aosStage.release();
     }
@@ -509,6 +517,14 @@ void setup(akua_solver* s, const std::vector<uint32_t>& counts) {
     if (s->numTiles <= kOneSweepMaxTiles) {
         for (auto* l : {&s->look, &s->look2}) l->alloc((size_t)2 * s->numTiles * (1u << kMaxDigitBits));
         for (auto* t : {&s->tickets, &s->tickets2}) t->alloc((size_t)kMaxPasses);
+    }
+    if (s->scenes.size() == 1 && s->nslots <= kOrderMaxSlots) {
+        // about four particles a group: cells hold more, so that most groups are one cell
+        s->groups = std::min(kOrderMaxGroups, std::max(256u, 1u << ceil_log2((s->nslots + 3u) / 4u)));
+        s->groupCount.alloc(s->groups);
+        s->groupBase.alloc(s->groups + 1);
+        s->placed.alloc(ns);
+        HIP_CHECK(hipMemset(s->groupCount.p, 0, s->groups * 4));
     }
     s->table.alloc(s->tableTotal);
     s->bslot.alloc(ns);
@@ -677,40 +693,55 @@ SweepLanes sweep_lanes(const akua_solver* s) {
     return SweepLanes{1, 2, 4, 2, 4};
 }
 
+// Whether the step orders its particles by launch_order: a small single scene whose layout is left to
+// the solver, with the reference's search.
+bool small_order(const akua_solver* s) {
+    const akua_tuning& t = s->tuning;
+    return s->groups > 0 && s->sph.searchCells == 1 && t.layoutLevel == kDefaultTuning.layoutLevel &&
+           t.hashDigitBits == kDefaultTuning.hashDigitBits && t.layoutDigitBits == kDefaultTuning.layoutDigitBits &&
+           t.layoutInterval == kDefaultTuning.layoutInterval;
+}
+
 void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool timed,
                   bool record = false, bool keepLayout = false) {
     Launcher L{s, st, timed};
     DeviceState d = s->devState(keepLayout);
     const SphParams& P = s->sph;
-    // single-cell super-cells: the layout keys are sorted in the previous logical order, which
-    // agrees with the new one within each key, so both sorts share their launches
-    const bool together = !keepLayout && s->tuning.layoutLevel == 0 && s->plan1.digitBits == s->plan2.digitBits;
-    // the prediction's launch also clears the cell table and, for paired look-back sorts, their
-    // scratch
-    const SortZeroSpans zero = together ? sort_both_zero_spans(s) : SortZeroSpans{};
-    L.before("predict_hash");
-    launch_predict_hash(st, d, P, S, together, true, &zero);
-    L.after("predict_hash");
-    if (together) {
-        if (!sort_both(s, st, timed, zero.count > 0)) fail(AKUA_ERR_STATE, "paired sorts need equal digit widths");
-        L.before("cell_keys");
-        launch_cell_keys(st, d, P, S, false, true);
-        L.after("cell_keys");
+    const bool carryDelta = s->cfg.solverIterations == 0;
+    const bool carry = carryDelta || record || (s->mode == 1 && s->haveNet);
+    if (small_order(s)) {
+        L.before("order");
+        launch_order(st, d, P, S, carry, carryDelta);
+        L.after("order");
     } else {
-        sort_hash(s, st, timed);
-        L.before("cell_keys");
-        launch_cell_keys(st, d, P, S, keepLayout, false);
-        L.after("cell_keys");
-        if (!keepLayout) sort_layout(s, st, timed);
+        // single-cell super-cells: the layout keys are sorted in the previous logical order, which
+        // agrees with the new one within each key, so both sorts share their launches
+        const bool together = !keepLayout && s->tuning.layoutLevel == 0 && s->plan1.digitBits == s->plan2.digitBits;
+        // the prediction's launch also clears the cell table and, for paired look-back sorts, their
+        // scratch
+        const SortZeroSpans zero = together ? sort_both_zero_spans(s) : SortZeroSpans{};
+        L.before("predict_hash");
+        launch_predict_hash(st, d, P, S, together, true, &zero);
+        L.after("predict_hash");
+        if (together) {
+            if (!sort_both(s, st, timed, zero.count > 0)) fail(AKUA_ERR_STATE, "paired sorts need equal digit widths");
+            L.before("cell_keys");
+            launch_cell_keys(st, d, P, S, false, true);
+            L.after("cell_keys");
+        } else {
+            sort_hash(s, st, timed);
+            L.before("cell_keys");
+            launch_cell_keys(st, d, P, S, keepLayout, false);
+            L.after("cell_keys");
+            if (!keepLayout) sort_layout(s, st, timed);
+        }
+        L.before("gather");
+        launch_gather(st, d, P, S, carry, carryDelta, together);
+        L.after("gather");
+        L.before("bucket_phys");
+        launch_bucket_phys(st, d);
+        L.after("bucket_phys");
     }
-    L.before("gather");
-    launch_gather(st, d, P, S,
-                  s->cfg.solverIterations == 0 || record || (s->mode == 1 && s->haveNet),
-                  s->cfg.solverIterations == 0, together);
-    L.after("gather");
-    L.before("bucket_phys");
-    launch_bucket_phys(st, d);
-    L.after("bucket_phys");
     const int bs = s->tuning.block;
     const int I = s->cfg.solverIterations;
     const bool learned = s->mode == 1 && !record;

@@ -1,0 +1,79 @@
+"""Ordering of small scenes by counting (one group of hash bits at a time) against the FP32 oracle: the
+sorted hashes, the permutation, the buckets' ranges and the lists, over several steps, at the edges of
+waves, workgroups, group counts and of the largest such scene, with crowded and shared buckets, and
+where the layout setting changes between steps."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+DT = 0.004
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+    if torch.cuda.device_count() < 1:
+        pytest.fail("no GPU visible: the gpu tests need an MI355X")
+    from akuaengine_amd.solver import PBFSolver
+    return PBFSolver
+
+
+def _check(gpu, oracle_mod, cfg, corr, pos, lo, hi, steps, between=None):
+    vel = np.random.default_rng(len(pos)).uniform(-0.5, 0.5, pos.shape).astype(np.float32)
+    s = gpu(len(pos), cfg, corr)
+    o = oracle_mod.Oracle(len(pos), cfg, corr, 32)
+    s.set_state(pos, vel)
+    o.set_state(pos, vel)
+    for k in range(steps):
+        if between:
+            between(s, k)
+        s.step(DT, lo, hi)
+        o.step(DT, lo, hi)
+        t = o.taps()
+        np.testing.assert_array_equal(s.debug_hashes(), t["sorted_hash"])
+        np.testing.assert_array_equal(s.debug_permutation(), t["perm"])
+        nbr, cnt = s.debug_neighbours()
+        np.testing.assert_array_equal(cnt, t["cnt"])
+        np.testing.assert_array_equal(nbr, t["nbr"])
+        h, start, end = s.debug_cell_ranges()
+        np.testing.assert_array_equal(h, np.unique(t["sorted_hash"]))
+        np.testing.assert_array_equal(start, np.searchsorted(t["sorted_hash"], h))
+        np.testing.assert_array_equal(end, np.searchsorted(t["sorted_hash"], h, side="right"))
+    g, r = s.get_state(), o.state()
+    for k in ("pos", "vel", "density", "lam", "ids"):
+        np.testing.assert_array_equal(g[k], r[k].astype(g[k].dtype), err_msg=k)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 255, 257, 1023, 1025, 2049, 16383, 32769, 131071, 131072, 131073])
+def test_sizes(gpu, oracle_mod, dam_params, n):
+    from akuaengine_amd import scenes
+    cfg, corr = dam_params
+    sc = scenes.batched_scene(n, index=n % 7)
+    print(f"[small order] n={n}", flush=True)
+    _check(gpu, oracle_mod, cfg, corr, sc.pos, sc.box_min, sc.box_max, 3 if n < 100000 else 2)
+
+
+@pytest.mark.parametrize("over", [dict(), dict(maxNeighbours=1), dict(maxNeighbours=2), dict(solverIterations=0)])
+def test_crowded_and_shared_buckets(gpu, oracle_mod, dam_params, over):
+    """1,500 particles in one cell (one group, a bucket longer than a run), particles outside the box,
+    tables of one and two entries per particle, and a step without iterations."""
+    cfg, corr = dam_params
+    rng = np.random.default_rng(3)
+    pos = np.concatenate([1.0 + rng.uniform(0.0, 0.099, (1500, 3)), rng.uniform(-1.0, 3.0, (3001, 3))])
+    _check(gpu, oracle_mod, dataclasses.replace(cfg, **over), corr, rng.permutation(pos).astype(np.float32),
+           (0.0, 0.0, 0.0), (2.0, 2.0, 2.0), 2)
+
+
+def test_setting_changes_between_steps(gpu, oracle_mod, dam_params):
+    from akuaengine_amd import scenes
+    cfg, corr = dam_params
+    sc = scenes.dam_break_scaled(14, seed=2)
+
+    def between(s, k):
+        default = (k // 2) % 2 == 0
+        s.set_tuning(block=256, layoutLevel=s_default if default else 2, layoutInterval=1 if default else 2)
+
+    s_default = gpu(1, cfg, corr).get_tuning()["layoutLevel"]
+    _check(gpu, oracle_mod, cfg, corr, sc.pos, sc.box_min, sc.box_max, 7, between)
