@@ -154,7 +154,6 @@ void launch_bucket_phys(hipStream_t st, const DeviceState& d);
 constexpr uint32_t kOrderMaxSlots = 1u << 17, kOrderMaxGroups = 1u << 13;
 void launch_order(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
                   bool carryDelta);
-void launch_invert_order(hipStream_t st, const DeviceState& d, uint32_t* phys);
 // The neighbour lists.  Below: bs is the workgroup size of the neighbour sweeps (128, 256 or 512;
 // results do not depend on it).
 void launch_neighbours(hipStream_t st, const DeviceState& d, const SphParams& P);

@@ -461,17 +461,6 @@ __global__ __launch_bounds__(kBlock) void k_order_rank(DeviceState d, StepParams
     d.physT[to] = to;
 }
 
-// The physical slot of each logical index from the step's persistent lid (outside a step, where
-// physT no longer holds it: rendering draws in logical order).
-__global__ __launch_bounds__(kBlock) void k_invert_order(DeviceState d, uint32_t* __restrict__ phys) {
-    const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= d.nslots) return;
-    const SceneDev& sc = scene_of(d, p);
-    if (p >= sc.end) return;
-    const uint32_t k = d.lid[p];
-    if (k < d.nslots) phys[k] = p;
-}
-
 // Per bucket: where it starts in physical order and whether its particles occupy consecutive
 // physical slots in logical order (always true for a bucket of one cell, which lies inside one
 // super-cell; buckets of more than 256 particles are not marked).  One thread per logical index k,
@@ -2365,10 +2354,6 @@ void launch_order(hipStream_t st, const DeviceState& d, const SphParams& P, cons
     else
         k_order_rank<false, false><<<count, kBlock, 0, st>>>(d, S);
 }
-void launch_invert_order(hipStream_t st, const DeviceState& d, uint32_t* phys) {
-    k_invert_order<<<grid(d.nslots), kBlock, 0, st>>>(d, phys);
-}
-
 void launch_bucket_phys(hipStream_t st, const DeviceState& d) {
     k_bucket_phys<<<grid(d.nslots), kBlock, 0, st>>>(d);
 }

@@ -25,7 +25,7 @@ void camera_setup(const float position[3], float yawDeg, float pitchDeg, float f
 // (draw) index of each slot and the slot of each logical index.  zbuf: width * height keys;
 // rgb: width * height * 3 bytes (device memory).
 void launch_render(hipStream_t st, const float4* X, const float4* color, const float* size,
-                   const uint32_t* id, const uint32_t* lid, const uint32_t* phys, uint32_t n,
+                   const uint32_t* id, const uint32_t* lid, uint32_t* phys, uint32_t n,
                    const RenderParams& R, unsigned long long* zbuf, unsigned char* rgb);
 
 }  // namespace akua

@@ -15,6 +15,7 @@
 //                    colour; written as RGB8 rows from the top.
 #include "render.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace akua {
@@ -25,9 +26,15 @@ constexpr float kMaxPointSize = 256.0f;  // GL clamps sprites to an implementati
 constexpr float kFloorY = -0.02f;        // FLOOR_LEVEL (Application.cpp:16)
 constexpr float kFloorExtent = 100.0f;   // floor quad x, z in [0, 100] (Application.cpp:130-135)
 
-__global__ void k_render_clear(unsigned long long* __restrict__ z, uint32_t n) {
+// Empties the pixels' keys and inverts the draw order: phys[k], the slot drawn k-th.
+__global__ void k_render_clear(unsigned long long* __restrict__ z, uint32_t pixels, const uint32_t* __restrict__ lid,
+                               uint32_t* __restrict__ phys, uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) z[i] = ~0ull;
+    if (i < pixels) z[i] = ~0ull;
+    if (i < n) {
+        const uint32_t k = lid[i];
+        if (k < n) phys[k] = i;
+    }
 }
 
 struct Sprite {
@@ -65,14 +72,22 @@ __device__ __forceinline__ float sprite_d2(const Sprite& sp, int fx, int fy) {
     return ox * ox + oy * oy;
 }
 
-__global__ void k_render_splat(const float4* __restrict__ X, const float4* __restrict__ color,
-                               const float* __restrict__ size, const uint32_t* __restrict__ id,
-                               const uint32_t* __restrict__ lid, uint32_t n, RenderParams R,
-                               unsigned long long* __restrict__ zbuf) {
-    (void)color;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// kSplatLanes lanes per particle share its sprite's fragments: at the reference's point size a sprite
+// has some 80, and one thread per particle left the chip to a few waves of long serial loops.  A key that
+// the pixel already undercuts needs no atomic (keys only fall, so an old value read decides the same):
+// sprites overlap many deep.  Measured at 27,000 particles, 1280 x 720: 79 us with one thread, 36 with
+// eight lanes, 28 with their keys read four at a time, 25 with sixteen (300,000: 188 and 158).
+constexpr uint32_t kSplatLanes = 16, kSplatBatch = 4;
+
+__global__ __launch_bounds__(256) void k_render_splat(const float4* __restrict__ X, const float* __restrict__ size,
+                                                      const uint32_t* __restrict__ id,
+                                                      const uint32_t* __restrict__ lid, uint32_t n, RenderParams R,
+                                                      unsigned long long* zbuf) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = t / kSplatLanes;
     if (i >= n) return;
     const float4 x = X[i];
+    const uint32_t draw = lid[i];
     const float sz = R.pointSize > 0.0f ? R.pointSize : size[id[i]];
     Sprite sp;
     if (!sprite_of(R, x.x, x.y, x.z, sz, sp)) return;
@@ -84,13 +99,27 @@ __global__ void k_render_splat(const float4* __restrict__ X, const float4* __res
     fy0 = max(fy0, 0);
     fx1 = min(fx1, R.width - 1);
     fy1 = min(fy1, R.height - 1);
-    const unsigned long long key =
-        ((unsigned long long)__float_as_uint(sp.zw) << 32) | (unsigned long long)lid[i];
-    for (int fy = fy0; fy <= fy1; ++fy)
-        for (int fx = fx0; fx <= fx1; ++fx) {
-            if (sprite_d2(sp, fx, fy) > 0.25f) continue;
-            atomicMin(&zbuf[(size_t)(R.height - 1 - fy) * (size_t)R.width + (size_t)fx], key);
+    if (fx1 < fx0 || fy1 < fy0) return;
+    const unsigned long long key = ((unsigned long long)__float_as_uint(sp.zw) << 32) | (unsigned long long)draw;
+    // fragments of the rectangle row by row (at most 257 x 257), kSplatBatch of this lane's at a time:
+    // their pixels' keys are read together
+    const uint32_t w = (uint32_t)(fx1 - fx0 + 1), count = w * (uint32_t)(fy1 - fy0 + 1);
+    uint32_t row = (t % kSplatLanes) / w, column = t % kSplatLanes - row * w;
+    for (uint32_t f = t % kSplatLanes; f < count; f += kSplatLanes * kSplatBatch) {
+        unsigned long long* at[kSplatBatch];
+        unsigned long long old[kSplatBatch];
+#pragma unroll
+        for (uint32_t u = 0; u < kSplatBatch; ++u) {
+            const int fx = fx0 + (int)column, fy = fy0 + (int)row;
+            const bool in = f + u * kSplatLanes < count && !(sprite_d2(sp, fx, fy) > 0.25f);
+            at[u] = in ? &zbuf[(size_t)(R.height - 1 - fy) * (size_t)R.width + (size_t)fx] : nullptr;
+            old[u] = in ? __hip_atomic_load(at[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0ull;
+            for (column += kSplatLanes; column >= w; column -= w) ++row;
         }
+#pragma unroll
+        for (uint32_t u = 0; u < kSplatBatch; ++u)
+            if (old[u] > key) atomicMin(at[u], key);
+    }
 }
 
 __device__ __forceinline__ unsigned char to_u8(float c) {
@@ -218,11 +247,14 @@ void camera_setup(const float position[3], float yawDeg, float pitchDeg, float f
 }
 
 void launch_render(hipStream_t st, const float4* X, const float4* color, const float* size,
-                   const uint32_t* id, const uint32_t* lid, const uint32_t* phys, uint32_t n,
+                   const uint32_t* id, const uint32_t* lid, uint32_t* phys, uint32_t n,
                    const RenderParams& R, unsigned long long* zbuf, unsigned char* rgb) {
     const uint32_t pixels = (uint32_t)(R.width * R.height);
-    k_render_clear<<<(pixels + 255) / 256, 256, 0, st>>>(zbuf, pixels);
-    if (n) k_render_splat<<<(n + 255) / 256, 256, 0, st>>>(X, color, size, id, lid, n, R, zbuf);
+    k_render_clear<<<(std::max(pixels, n) + 255) / 256, 256, 0, st>>>(zbuf, pixels, lid, phys, n);
+    if (n) {
+        // n * kSplatLanes stays below 2^32: slots number at most 2^28
+        k_render_splat<<<(n * kSplatLanes + 255) / 256, 256, 0, st>>>(X, size, id, lid, n, R, zbuf);
+    }
     k_render_resolve<<<(pixels + 255) / 256, 256, 0, st>>>(X, color, size, id, phys, R, zbuf, rgb);
 }
 

@@ -2265,16 +2265,15 @@ akua_status akua_render(akua_solver* s, const akua_camera* cam, int32_t width, i
         R.pointSize = pointSize;
         R.drawFloor = drawFloor ? 1 : 0;
         const size_t pixels = (size_t)width * (size_t)height;
-        HIP_CHECK(hipStreamSynchronize(s->stream));
-        if (s->renderKeys.n < pixels) s->renderKeys.alloc(pixels);
-        if (s->renderRgb.n < 3 * pixels) s->renderRgb.alloc(3 * pixels);
-        upload_scenes(s);  // the order inversion reads the scene ranges
-        launch_invert_order(s->stream, s->devState(), s->phys.p);
+        if (s->renderKeys.n < pixels || s->renderRgb.n < 3 * pixels) {
+            HIP_CHECK(hipStreamSynchronize(s->stream));
+            if (s->renderKeys.n < pixels) s->renderKeys.alloc(pixels);
+            if (s->renderRgb.n < 3 * pixels) s->renderRgb.alloc(3 * pixels);
+        }
         launch_render(s->stream, s->X.p, s->color.p, s->size.p, s->id.p, s->lid.p, s->phys.p,
                       s->scenes[0].end, R, s->renderKeys.p, s->renderRgb.p);
         HIP_CHECK(hipGetLastError());
-        HIP_CHECK(hipStreamSynchronize(s->stream));
-        HIP_CHECK(hipMemcpy(rgb, s->renderRgb.p, 3 * pixels, hipMemcpyDeviceToHost));
+        read_back(s, {{rgb, s->renderRgb.p, 3 * pixels}});
     });
 }
 

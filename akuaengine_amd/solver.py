@@ -163,7 +163,7 @@ class PBFSolver:
         """(height, width, 3) uint8 image of the particles as the reference draws them (point
         sprites over the checkered floor); camera: an akua_camera (default: the reference's)."""
         cam = camera if camera is not None else default_camera()
-        img = np.zeros((int(height), int(width), 3), np.uint8)
+        img = np.empty((int(height), int(width), 3), np.uint8)  # written whole
         _lib.check(self._L.akua_render(self._h, ctypes.byref(cam), int(width), int(height),
                                        float(point_size), 1 if floor else 0, _p(img)))
         return img
