@@ -7,23 +7,28 @@ namespace akua {
 namespace {
 
 // Records in buffer order become both the logical and the physical order (lid = phys = identity).
+// blockMasses: per 256 records, whether a mass differs from 1.
 __global__ void k_import_aos(const AosParticle* __restrict__ in, uint32_t n, float4* X, float4* V,
                              float4* VS, float4* DP, float* dens, float* lam, uint32_t* id,
-                             uint32_t* lid, uint32_t* phys, float4* color, float* size) {
+                             uint32_t* lid, uint32_t* phys, float4* color, float* size, uint32_t* blockMasses) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const AosParticle& p = in[i];
-    X[i] = make_float4(p.position[0], p.position[1], p.position[2], p.mass);
-    V[i] = make_float4(p.velocity[0], p.velocity[1], p.velocity[2], 0.0f);
-    VS[i] = make_float4(p.new_velocity[0], p.new_velocity[1], p.new_velocity[2], 0.0f);
-    DP[i] = make_float4(p.position_delta[0], p.position_delta[1], p.position_delta[2], 0.0f);
-    dens[i] = p.density;
-    lam[i] = p.lambda;
-    id[i] = i;
-    lid[i] = i;
-    phys[i] = i;
-    color[i] = make_float4(p.color[0], p.color[1], p.color[2], p.color[3]);
-    size[i] = p.size;
+    const AosParticle& p = in[min(i, n - 1u)];
+    const float mass = p.mass;
+    if (i < n) {
+        X[i] = make_float4(p.position[0], p.position[1], p.position[2], mass);
+        V[i] = make_float4(p.velocity[0], p.velocity[1], p.velocity[2], 0.0f);
+        VS[i] = make_float4(p.new_velocity[0], p.new_velocity[1], p.new_velocity[2], 0.0f);
+        DP[i] = make_float4(p.position_delta[0], p.position_delta[1], p.position_delta[2], 0.0f);
+        dens[i] = p.density;
+        lam[i] = p.lambda;
+        id[i] = i;
+        lid[i] = i;
+        phys[i] = i;
+        color[i] = make_float4(p.color[0], p.color[1], p.color[2], p.color[3]);
+        size[i] = p.size;
+    }
+    const int differ = __syncthreads_or(i < n && mass != 1.0f);  // NaN differs
+    if (threadIdx.x == 0) blockMasses[blockIdx.x] = differ ? 1u : 0u;
 }
 
 // Physical slot i is written to its logical position, the order of the reference's buffer.
@@ -92,10 +97,10 @@ void launch_export_state(hipStream_t st, const StateArrays& out, uint32_t n, uin
 
 void launch_import_aos(hipStream_t st, const AosParticle* in, uint32_t n, float4* X, float4* V,
                        float4* VS, float4* DP, float* dens, float* lam, uint32_t* id, uint32_t* lid,
-                       uint32_t* phys, float4* color, float* size) {
+                       uint32_t* phys, float4* color, float* size, uint32_t* blockMasses) {
     if (n)
         k_import_aos<<<(n + 255) / 256, 256, 0, st>>>(in, n, X, V, VS, DP, dens, lam, id, lid, phys,
-                                                      color, size);
+                                                      color, size, blockMasses);
 }
 
 void launch_export_aos(hipStream_t st, AosParticle* out, uint32_t n, const float4* X,

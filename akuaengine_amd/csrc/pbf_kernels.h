@@ -75,6 +75,9 @@ struct DeviceState {
     uint32_t* groupBase;
     uint4* placed;
     uint32_t groups, groupShift;  // a hash's group is its bits from groupShift on
+    // SphParams::fast 2: per 256 imported records, whether a mass differs from 1; of all of them
+    const uint32_t* blockMasses;
+    uint32_t* massesDiffer;
     uint32_t* skeysOut;        // skeys and perm1, for their writer
     uint32_t* perm1Out;
     uint32_t* keysM;           // super-cell Morton keys in logical order (second sort's input)

@@ -165,14 +165,29 @@ __device__ __forceinline__ uint32_t layout_key(int cx, int cy, int cz, const Sce
 // launches (single-cell super-cells, where the previous and the new logical order agree within
 // every layout key): its keys go straight into its input (keysM) and the record keeps only the
 // slot, to which k_cell_keys adds the new logical index.
-// Blocks from predictBlocks on clear the cell table instead (every record empty), and the last
-// kZeroBlocks zero the sorts' scratch spans: neither is touched by the prediction, so one launch
-// serves all three.
+// Blocks from predictBlocks on clear the cell table instead (every record empty), the next kZeroBlocks
+// zero the sorts' scratch spans and the last gathers what the import found in the masses: none of it is
+// touched by the prediction, so one launch serves all four.
 constexpr uint32_t kZeroBlocks = 8;
+
+// Masses taken from device memory (SphParams::fast 2): massesDiffer becomes 0 where every 256 imported
+// records had unit masses, else 1.  Every thread of one workgroup.
+__device__ __forceinline__ void gather_masses(const DeviceState& d, const SphParams& P) {
+    if (P.fast != 2) return;
+    const uint32_t blocks = (d.nslots + 255u) / 256u;
+    int differ = 0;
+    for (uint32_t b = threadIdx.x; b < blocks; b += kBlock) differ |= d.blockMasses[b] != 0u;
+    differ = __syncthreads_or(differ);
+    if (threadIdx.x == 0) *d.massesDiffer = differ ? 1u : 0u;
+}
 
 __global__ __launch_bounds__(kBlock) void k_predict_hash(DeviceState d, SphParams P, StepParams S,
                                                          bool layoutPrev, uint32_t predictBlocks,
                                                          uint32_t clearBlocks, SortZeroSpans zero) {
+    if (blockIdx.x == gridDim.x - 1u) {
+        gather_masses(d, P);
+        return;
+    }
     if (blockIdx.x >= predictBlocks + clearBlocks) {
         const uint32_t i = (blockIdx.x - predictBlocks - clearBlocks) * kBlock + threadIdx.x;
 #pragma unroll
@@ -328,8 +343,13 @@ __device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
 //      members, which also gives its bucket's bounds: the move and the table entry.
 constexpr uint32_t kOrderBlock = 1024;
 
-// Groups are counted by runs: particles of one cell mostly lie side by side.
+// Groups are counted by runs: particles of one cell mostly lie side by side.  The last block gathers what
+// the import found in the masses (gather_masses).
 __global__ __launch_bounds__(kBlock) void k_order_count(DeviceState d, SphParams P, StepParams S, uint32_t countBlocks) {
+    if (blockIdx.x == gridDim.x - 1u) {
+        gather_masses(d, P);
+        return;
+    }
     if (blockIdx.x >= countBlocks) {
         const uint32_t i = (blockIdx.x - countBlocks) * kBlock + threadIdx.x;
         if (i < d.tableTotal) d.table[i] = make_uint4(kEmptyKey, kEmptyKey, kEmptyKey, kEmptyKey);
@@ -1138,6 +1158,22 @@ __device__ __forceinline__ void wave_resid_partial(const DeviceState& d, int slo
     if (__lane_id() == 0) d.residPart[(size_t)slot * d.nWaves + (i >> 6)] = make_float2(m, t);
 }
 
+// A sweep's body by SphParams::fast: f(std::true_type) or f(std::false_type), chosen by the launch, or,
+// where the masses came from device memory (2), by what the device found in them.  The branch is the same
+// for a whole launch; with it a sweep of unit masses costs what it does where the host knows them, plus
+// one scalar load.
+template <int kFast, class F>
+__device__ __forceinline__ void by_masses(const DeviceState& d, F f) {
+    if constexpr (kFast == 2) {
+        if (*d.massesDiffer == 0u)
+            f(std::true_type{});
+        else
+            f(std::false_type{});
+    } else {
+        f(std::bool_constant<kFast == 1>{});
+    }
+}
+
 // kFast (SphParams::fast): unit masses, range-tested quotients bounded in advance.
 // kBnd: boundary samples (SphParams::bd): their density and gradient sums join rho and grad_i C
 // after the neighbour sweep; the gradient sum is kept in Bg for the position-delta pass, which
@@ -1214,12 +1250,14 @@ __device__ __forceinline__ void density_lambda_slot(const DeviceState& d, const 
 
 // One workgroup per virtual workgroup (the loop runs once); the loop form lets a launch use any
 // grid size.
-template <int BS, bool kFast, bool kBnd>
+template <int BS, int kFast, bool kBnd>
 __global__ __launch_bounds__(BS) void k_density_lambda(DeviceState d, SphParams P,
                                                            const float4* __restrict__ Xs,
                                                            int residSlot, int gated, uint32_t nvb) {
-    for (uint32_t vb = blockIdx.x; vb < nvb; vb += gridDim.x)
-        density_lambda_slot<BS, kFast, kBnd>(d, P, Xs, residSlot, gated, xcd_slot_of<BS>(vb, nvb));
+    by_masses<kFast>(d, [&](auto fast) {
+        for (uint32_t vb = blockIdx.x; vb < nvb; vb += gridDim.x)
+            density_lambda_slot<BS, decltype(fast)::value, kBnd>(d, P, Xs, residSlot, gated, xcd_slot_of<BS>(vb, nvb));
+    });
 }
 
 // Features of the learned warm start at x*_pred, one neighbour sweep (list order):
@@ -1582,16 +1620,18 @@ __device__ __forceinline__ void delta_correct_slot(const DeviceState& d, const S
 
 // Unit masses: held to 8 waves per SIMD (its scalar registers, over the 8-wave budget, spill to
 // vector lanes); the general kernels would spill vector registers there.
-template <int BS, bool kFinal, bool kApplyDelta, bool kFast, bool kBnd>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kFast && !kBnd ? 8 : 1)))
+template <int BS, bool kFinal, bool kApplyDelta, int kFast, bool kBnd>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(kFast == 1 && !kBnd ? 8 : 1)))
 void k_delta_correct(DeviceState d, SphParams P, StepParams S,
                                                           const float4* __restrict__ XsSet,
                                                           float4* __restrict__ XsOut,
                                                           const float4* __restrict__ XsAlt,
                                                           int gateMode, uint32_t nvb) {
-    for (uint32_t vb = blockIdx.x; vb < nvb; vb += gridDim.x)
-        delta_correct_slot<BS, kFinal, kApplyDelta, kFast, kBnd>(d, P, S, XsSet, XsOut, XsAlt, gateMode,
-                                                                 xcd_slot_of<BS>(vb, nvb));
+    by_masses<kFast>(d, [&](auto fast) {
+        for (uint32_t vb = blockIdx.x; vb < nvb; vb += gridDim.x)
+            delta_correct_slot<BS, kFinal, kApplyDelta, decltype(fast)::value, kBnd>(d, P, S, XsSet, XsOut, XsAlt,
+                                                                                     gateMode, xcd_slot_of<BS>(vb, nvb));
+    });
 }
 
 // kernel_compute_vorticities (IntegrationCUDA.cu:104-128).  W.w keeps |omega| for the next pass,
@@ -1624,9 +1664,9 @@ __device__ __forceinline__ void vorticity_slot(const DeviceState& d, const SphPa
     d.XsB[i] = make_float4(xi.x, xi.y, xi.z, wl);
 }
 
-template <int BS, bool kFast>
+template <int BS, int kFast>
 __global__ __launch_bounds__(BS) void k_vorticity(DeviceState d, SphParams P) {
-    vorticity_slot<kFast>(d, P, xcd_slot<BS>());
+    by_masses<kFast>(d, [&](auto fast) { vorticity_slot<decltype(fast)::value>(d, P, xcd_slot<BS>()); });
 }
 
 // The confinement force from the summed eta (IntegrationCUDA.cu:146-163) and the write of Vc.
@@ -1677,9 +1717,9 @@ __device__ __forceinline__ void confinement_slot(const DeviceState& d, const Sph
     confine_finish(d, P, S, i, xi4w, wi, d.V[i], eta, d.dens[i]);
 }
 
-template <int BS, bool kFast>
+template <int BS, int kFast>
 __global__ __launch_bounds__(BS) void k_confinement(DeviceState d, SphParams P, StepParams S) {
-    confinement_slot<kFast>(d, P, S, xcd_slot<BS>());
+    by_masses<kFast>(d, [&](auto fast) { confinement_slot<decltype(fast)::value>(d, P, S, xcd_slot<BS>()); });
 }
 
 // kernel_apply_xsph_viscosity (IntegrationCUDA.cu:167-195), Jacobi: reads Vc, writes V.
@@ -2011,9 +2051,7 @@ __device__ __forceinline__ void boundary_split(const SphParams& P, f3 xi, const 
 }
 
 template <int L, bool kFast, bool kBnd>
-__global__ __launch_bounds__(kGroupBlock) void k_density_lambda_group(DeviceState d, SphParams P,
-                                                                      const float4* __restrict__ Xs) {
-    __shared__ float4 lds[group_lds_floats<L, 5>() / 4u];
+__device__ __forceinline__ void density_lambda_group_slots(const DeviceState& d, const SphParams& P, const float4* __restrict__ Xs, float* lds) {
     const LaneGroup<L> g = lane_group<L>();
     if (g.i >= d.nslots) return;  // whole groups
     const GroupList<L> list = group_list<L>(d, P, g);
@@ -2022,7 +2060,7 @@ __global__ __launch_bounds__(kGroupBlock) void k_density_lambda_group(DeviceStat
     const f3 xi = make3(xi4);
     const float negInv = -P.invRest;
     // rho, grad_i C (x, y, z), sum |grad_j C|^2
-    GroupSums<L, 5> sums(g, xi4.w * P.w0, reinterpret_cast<float*>(lds));
+    GroupSums<L, 5> sums(g, xi4.w * P.w0, lds);
     walk_split<L, 5, float4>(
         list, g, sums, [&](uint32_t j) { return ld(Xs, j); },
         [&](const float4& xj4, float (&t)[5]) {
@@ -2051,7 +2089,7 @@ __global__ __launch_bounds__(kGroupBlock) void k_density_lambda_group(DeviceStat
         float rb = 0.0f;
         f3 gb{0.0f, 0.0f, 0.0f};
         if (near) {
-            GroupSums<L, 4> wall(g, 0.0f, reinterpret_cast<float*>(lds));
+            GroupSums<L, 4> wall(g, 0.0f, lds);
             // the rows of its own group again: a group's rows of four sums lie inside its rows of five
             wall.rows = sums.rows;
             boundary_split<L, kFast>(P, xi, g, wall);
@@ -2071,11 +2109,17 @@ __global__ __launch_bounds__(kGroupBlock) void k_density_lambda_group(DeviceStat
     if (kFast) d.W[g.i] = make_float4(xi.x, xi.y, xi.z, lam);
 }
 
+template <int L, int kFast, bool kBnd>
+__global__ __launch_bounds__(kGroupBlock) void k_density_lambda_group(DeviceState d, SphParams P, const float4* __restrict__ Xs) {
+    __shared__ float4 lds[group_lds_floats<L, 5>() / 4u];
+    by_masses<kFast>(d, [&](auto fast) {
+        density_lambda_group_slots<L, decltype(fast)::value, kBnd>(d, P, Xs, reinterpret_cast<float*>(lds));
+    });
+}
+
 template <int L, bool kFinal, bool kFast, bool kBnd>
-__global__ __launch_bounds__(kGroupBlock) void k_delta_correct_group(DeviceState d, SphParams P, StepParams S,
-                                                                     const float4* __restrict__ XsIn,
-                                                                     float4* __restrict__ XsOut) {
-    __shared__ float4 lds[group_lds_floats<L, 3>() / 4u];
+__device__ __forceinline__ void delta_correct_group_slots(const DeviceState& d, const SphParams& P, const StepParams& S,
+    const float4* __restrict__ XsIn, float4* __restrict__ XsOut, float* lds) {
     const LaneGroup<L> g = lane_group<L>();
     if (g.i >= d.nslots) return;
     const GroupList<L> list = group_list<L>(d, P, g);
@@ -2086,7 +2130,7 @@ __global__ __launch_bounds__(kGroupBlock) void k_delta_correct_group(DeviceState
     FinishIn in{};
     if (kFinal) in = finish_in(d, g.i);
     const Recip Rdq = recip(P.wdq);
-    GroupSums<L, 3> sums(g, 0.0f, reinterpret_cast<float*>(lds));
+    GroupSums<L, 3> sums(g, 0.0f, lds);
     walk_split<L, 3, XLam>(
         list, g, sums,
         [&](uint32_t j) {
@@ -2124,16 +2168,24 @@ __global__ __launch_bounds__(kGroupBlock) void k_delta_correct_group(DeviceState
     finish_step<true>(d, S, sc, g.i, xi4, in, q, dp);
 }
 
-template <int L, bool kFast>
-__global__ __launch_bounds__(kGroupBlock) void k_vorticity_group(DeviceState d, SphParams P) {
+template <int L, bool kFinal, int kFast, bool kBnd>
+__global__ __launch_bounds__(kGroupBlock) void k_delta_correct_group(DeviceState d, SphParams P, StepParams S,
+    const float4* __restrict__ XsIn, float4* __restrict__ XsOut) {
     __shared__ float4 lds[group_lds_floats<L, 3>() / 4u];
+    by_masses<kFast>(d, [&](auto fast) {
+        delta_correct_group_slots<L, kFinal, decltype(fast)::value, kBnd>(d, P, S, XsIn, XsOut, reinterpret_cast<float*>(lds));
+    });
+}
+
+template <int L, bool kFast>
+__device__ __forceinline__ void vorticity_group_slots(const DeviceState& d, const SphParams& P, float* lds) {
     const LaneGroup<L> g = lane_group<L>();
     if (g.i >= d.nslots) return;
     const GroupList<L> list = group_list<L>(d, P, g);
     const SceneDev& sc = scene_of(d, g.i);
     const f3 xi = make3(d.X[g.i]);
     const f3 vi = make3(d.V[g.i]);
-    GroupSums<L, 3> sums(g, 0.0f, reinterpret_cast<float*>(lds));
+    GroupSums<L, 3> sums(g, 0.0f, lds);
     walk_split<L, 3, XV>(
         list, g, sums, [&](uint32_t j) { return XV{ld(d.X, j), ld(d.V, j)}; },
         [&](const XV& nb, float (&t)[3]) {
@@ -2150,9 +2202,16 @@ __global__ __launch_bounds__(kGroupBlock) void k_vorticity_group(DeviceState d, 
     d.XsB[g.i] = make_float4(xi.x, xi.y, xi.z, wl);
 }
 
-template <int L, bool kFast>
-__global__ __launch_bounds__(kGroupBlock) void k_confinement_group(DeviceState d, SphParams P, StepParams S) {
+template <int L, int kFast>
+__global__ __launch_bounds__(kGroupBlock) void k_vorticity_group(DeviceState d, SphParams P) {
     __shared__ float4 lds[group_lds_floats<L, 3>() / 4u];
+    by_masses<kFast>(d, [&](auto fast) {
+        vorticity_group_slots<L, decltype(fast)::value>(d, P, reinterpret_cast<float*>(lds));
+    });
+}
+
+template <int L, bool kFast>
+__device__ __forceinline__ void confinement_group_slots(const DeviceState& d, const SphParams& P, const StepParams& S, float* lds) {
     const LaneGroup<L> g = lane_group<L>();
     if (g.i >= d.nslots) return;
     const GroupList<L> list = group_list<L>(d, P, g);
@@ -2161,7 +2220,7 @@ __global__ __launch_bounds__(kGroupBlock) void k_confinement_group(DeviceState d
     const f3 xi = make3(xi4);
     const float4 wi = d.W[g.i], vi = d.V[g.i];
     const float rho = d.dens[g.i];
-    GroupSums<L, 3> sums(g, 0.0f, reinterpret_cast<float*>(lds));
+    GroupSums<L, 3> sums(g, 0.0f, lds);
     walk_split<L, 3, XW>(
         list, g, sums, [&](uint32_t j) { return XW{ld(d.XsB, j), kFast ? 1.0f : ld(d.X, j).w}; },
         [&](const XW& nb, float (&t)[3]) {
@@ -2174,6 +2233,14 @@ __global__ __launch_bounds__(kGroupBlock) void k_confinement_group(DeviceState d
     const f3 eta{sums.of(g, 0), sums.of(g, 1), sums.of(g, 2)};
     if (g.r != 0u || g.i >= sc.end) return;
     confine_finish(d, P, S, g.i, xi4.w, wi, vi, eta, rho);
+}
+
+template <int L, int kFast>
+__global__ __launch_bounds__(kGroupBlock) void k_confinement_group(DeviceState d, SphParams P, StepParams S) {
+    __shared__ float4 lds[group_lds_floats<L, 3>() / 4u];
+    by_masses<kFast>(d, [&](auto fast) {
+        confinement_group_slots<L, decltype(fast)::value>(d, P, S, reinterpret_cast<float*>(lds));
+    });
 }
 
 template <int L>
@@ -2305,6 +2372,21 @@ inline unsigned grid_xcd(uint32_t n, int bs) {
         }                               \
     } while (0)
 
+// The masses' form: K is P.fast.
+#define AKUA_BY_FAST(CALL)       \
+    do {                         \
+        if (P.fast == 2) {       \
+            constexpr int K = 2; \
+            CALL;                \
+        } else if (P.fast) {     \
+            constexpr int K = 1; \
+            CALL;                \
+        } else {                 \
+            constexpr int K = 0; \
+            CALL;                \
+        }                        \
+    } while (0)
+
 inline unsigned grid_lanes(uint32_t nslots, int lanes) {
     return grid_xcd(nslots * (uint32_t)lanes, kGroupBlock);
 }
@@ -2324,7 +2406,7 @@ void launch_predict_hash(hipStream_t st, const DeviceState& d, const SphParams& 
     SortZeroSpans z{};
     if (zero) z = *zero;
     const uint32_t zeroBlocks = z.count ? kZeroBlocks : 0u;
-    k_predict_hash<<<predict + clear + zeroBlocks, kBlock, 0, st>>>(d, P, S, layoutPrev, predict, clear, z);
+    k_predict_hash<<<predict + clear + zeroBlocks + 1u, kBlock, 0, st>>>(d, P, S, layoutPrev, predict, clear, z);
 }
 void launch_cell_keys(hipStream_t st, const DeviceState& d, const SphParams& P,
                       const StepParams& S, bool keepLayout, bool layoutPrev) {
@@ -2345,7 +2427,7 @@ void launch_gather(hipStream_t st, const DeviceState& d, const SphParams& P, con
 void launch_order(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
                   bool carryDelta) {
     const uint32_t count = grid(d.nslots);
-    k_order_count<<<count + grid(d.tableTotal), kBlock, 0, st>>>(d, P, S, count);
+    k_order_count<<<count + grid(d.tableTotal) + 1u, kBlock, 0, st>>>(d, P, S, count);
     k_order_place<<<(d.nslots + kOrderBlock - 1) / kOrderBlock, kOrderBlock, 0, st>>>(d);
     if (carryDelta)
         k_order_rank<true, true><<<count, kBlock, 0, st>>>(d, S);
@@ -2394,26 +2476,18 @@ void density_lambda_bs(hipStream_t st, const DeviceState& d, const SphParams& P,
     const unsigned nvb = grid_xcd(d.nslots, BS);
     const int g = gated ? 1 : 0;
     if (P.bd.on) {
-        if (P.fast)
-            k_density_lambda<BS, true, true><<<nvb, BS, 0, st>>>(d, P, Xs, residSlot, g, nvb);
-        else
-            k_density_lambda<BS, false, true><<<nvb, BS, 0, st>>>(d, P, Xs, residSlot, g, nvb);
-    } else if (P.fast) {
-        k_density_lambda<BS, true, false><<<nvb, BS, 0, st>>>(d, P, Xs, residSlot, g, nvb);
+        AKUA_BY_FAST((k_density_lambda<BS, K, true><<<nvb, BS, 0, st>>>(d, P, Xs, residSlot, g, nvb)));
     } else {
-        k_density_lambda<BS, false, false><<<nvb, BS, 0, st>>>(d, P, Xs, residSlot, g, nvb);
+        AKUA_BY_FAST((k_density_lambda<BS, K, false><<<nvb, BS, 0, st>>>(d, P, Xs, residSlot, g, nvb)));
     }
 }
 void launch_density_lambda(hipStream_t st, const DeviceState& d, const SphParams& P,
                            const float4* Xs, int bs, int residSlot, bool gated, int lanes) {
     if (lanes > 1) {
         const unsigned g = grid_lanes(d.nslots, lanes);
-#define AKUA_DLG(K, B) AKUA_BY_LANES(lanes, (k_density_lambda_group<L, K, B><<<g, kGroupBlock, 0, st>>>(d, P, Xs)))
-        if (P.bd.on) {
-            if (P.fast) AKUA_DLG(true, true); else AKUA_DLG(false, true);
-        } else {
-            if (P.fast) AKUA_DLG(true, false); else AKUA_DLG(false, false);
-        }
+#define AKUA_DLG(B) \
+    AKUA_BY_FAST(AKUA_BY_LANES(lanes, (k_density_lambda_group<L, K, B><<<g, kGroupBlock, 0, st>>>(d, P, Xs))))
+        if (P.bd.on) AKUA_DLG(true); else AKUA_DLG(false);
 #undef AKUA_DLG
         return;
     }
@@ -2460,17 +2534,13 @@ void delta_correct_bs(hipStream_t st, const DeviceState& d, const SphParams& P,
 #define AKUA_DC(F, A, K, B) \
     k_delta_correct<BS, F, A, K, B><<<g, BS, 0, st>>>(d, P, S, XsIn, XsOut, XsAlt, gate, nvb)
     if (final && !applyDelta) {
-        AKUA_DC(true, false, false, false);  // a step without iterations
+        AKUA_DC(true, false, 0, false);  // a step without iterations
     } else if (P.bd.on) {
-        if (final) {
-            if (P.fast) AKUA_DC(true, true, true, true); else AKUA_DC(true, true, false, true);
-        } else {
-            if (P.fast) AKUA_DC(false, true, true, true); else AKUA_DC(false, true, false, true);
-        }
+        if (final) AKUA_BY_FAST(AKUA_DC(true, true, K, true)); else AKUA_BY_FAST(AKUA_DC(false, true, K, true));
     } else if (final) {
-        if (P.fast) AKUA_DC(true, true, true, false); else AKUA_DC(true, true, false, false);
+        AKUA_BY_FAST(AKUA_DC(true, true, K, false));
     } else {
-        if (P.fast) AKUA_DC(false, true, true, false); else AKUA_DC(false, true, false, false);
+        AKUA_BY_FAST(AKUA_DC(false, true, K, false));
     }
 #undef AKUA_DC
 }
@@ -2479,18 +2549,13 @@ void launch_delta_correct(hipStream_t st, const DeviceState& d, const SphParams&
                           bool applyDelta, int bs, int gate, const float4* XsAlt, int lanes) {
     if (lanes > 1 && applyDelta) {
         const unsigned g = grid_lanes(d.nslots, lanes);
-#define AKUA_DCG(F, K, B) \
-    AKUA_BY_LANES(lanes, (k_delta_correct_group<L, F, K, B><<<g, kGroupBlock, 0, st>>>(d, P, S, XsIn, XsOut)))
+#define AKUA_DCG(F, B) \
+    AKUA_BY_FAST(      \
+        AKUA_BY_LANES(lanes, (k_delta_correct_group<L, F, K, B><<<g, kGroupBlock, 0, st>>>(d, P, S, XsIn, XsOut))))
         if (P.bd.on) {
-            if (final) {
-                if (P.fast) AKUA_DCG(true, true, true); else AKUA_DCG(true, false, true);
-            } else {
-                if (P.fast) AKUA_DCG(false, true, true); else AKUA_DCG(false, false, true);
-            }
-        } else if (final) {
-            if (P.fast) AKUA_DCG(true, true, false); else AKUA_DCG(true, false, false);
+            if (final) AKUA_DCG(true, true); else AKUA_DCG(false, true);
         } else {
-            if (P.fast) AKUA_DCG(false, true, false); else AKUA_DCG(false, false, false);
+            if (final) AKUA_DCG(true, false); else AKUA_DCG(false, false);
         }
 #undef AKUA_DCG
         return;
@@ -2501,31 +2566,19 @@ void launch_delta_correct(hipStream_t st, const DeviceState& d, const SphParams&
 void launch_vorticity(hipStream_t st, const DeviceState& d, const SphParams& P, int bs, int lanes) {
     if (lanes > 1) {
         const unsigned g = grid_lanes(d.nslots, lanes);
-        if (P.fast)
-            AKUA_BY_LANES(lanes, (k_vorticity_group<L, true><<<g, kGroupBlock, 0, st>>>(d, P)));
-        else
-            AKUA_BY_LANES(lanes, (k_vorticity_group<L, false><<<g, kGroupBlock, 0, st>>>(d, P)));
+        AKUA_BY_FAST(AKUA_BY_LANES(lanes, (k_vorticity_group<L, K><<<g, kGroupBlock, 0, st>>>(d, P))));
         return;
     }
-    if (P.fast)
-        AKUA_BY_BLOCK(bs, (k_vorticity<BS, true><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));
-    else
-        AKUA_BY_BLOCK(bs, (k_vorticity<BS, false><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P)));
+    AKUA_BY_FAST(AKUA_BY_BLOCK(bs, (k_vorticity<BS, K><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P))));
 }
 void launch_confinement(hipStream_t st, const DeviceState& d, const SphParams& P,
                         const StepParams& S, int bs, int lanes) {
     if (lanes > 1) {
         const unsigned g = grid_lanes(d.nslots, lanes);
-        if (P.fast)
-            AKUA_BY_LANES(lanes, (k_confinement_group<L, true><<<g, kGroupBlock, 0, st>>>(d, P, S)));
-        else
-            AKUA_BY_LANES(lanes, (k_confinement_group<L, false><<<g, kGroupBlock, 0, st>>>(d, P, S)));
+        AKUA_BY_FAST(AKUA_BY_LANES(lanes, (k_confinement_group<L, K><<<g, kGroupBlock, 0, st>>>(d, P, S))));
         return;
     }
-    if (P.fast)
-        AKUA_BY_BLOCK(bs, (k_confinement<BS, true><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P, S)));
-    else
-        AKUA_BY_BLOCK(bs, (k_confinement<BS, false><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P, S)));
+    AKUA_BY_FAST(AKUA_BY_BLOCK(bs, (k_confinement<BS, K><<<grid_xcd(d.nslots, BS), BS, 0, st>>>(d, P, S))));
 }
 void launch_xsph(hipStream_t st, const DeviceState& d, const SphParams& P, int bs, int lanes) {
     if (lanes > 1) {
@@ -2580,9 +2633,9 @@ void launch_density_lambda_queue(hipStream_t st, const DeviceState& d, const Sph
 #define AKUA_DLQ(K, B) \
     k_density_lambda_queue<K, B><<<queue_grid(k_density_lambda_queue<K, B>, d), kQueueTile, 0, st>>>(d, P, Xs, pass)
     if (P.bd.on) {
-        if (P.fast) AKUA_DLQ(true, true); else AKUA_DLQ(false, true);
+        if (P.fast == 1) AKUA_DLQ(true, true); else AKUA_DLQ(false, true);
     } else {
-        if (P.fast) AKUA_DLQ(true, false); else AKUA_DLQ(false, false);
+        if (P.fast == 1) AKUA_DLQ(true, false); else AKUA_DLQ(false, false);
     }
 #undef AKUA_DLQ
 }
@@ -2594,26 +2647,26 @@ void launch_delta_correct_queue(hipStream_t st, const DeviceState& d, const SphP
         d, P, S, XsIn, XsOut, pass)
     if (P.bd.on) {
         if (final) {
-            if (P.fast) AKUA_DCQ(true, true, true); else AKUA_DCQ(true, false, true);
+            if (P.fast == 1) AKUA_DCQ(true, true, true); else AKUA_DCQ(true, false, true);
         } else {
-            if (P.fast) AKUA_DCQ(false, true, true); else AKUA_DCQ(false, false, true);
+            if (P.fast == 1) AKUA_DCQ(false, true, true); else AKUA_DCQ(false, false, true);
         }
     } else if (final) {
-        if (P.fast) AKUA_DCQ(true, true, false); else AKUA_DCQ(true, false, false);
+        if (P.fast == 1) AKUA_DCQ(true, true, false); else AKUA_DCQ(true, false, false);
     } else {
-        if (P.fast) AKUA_DCQ(false, true, false); else AKUA_DCQ(false, false, false);
+        if (P.fast == 1) AKUA_DCQ(false, true, false); else AKUA_DCQ(false, false, false);
     }
 #undef AKUA_DCQ
 }
 void launch_vorticity_queue(hipStream_t st, const DeviceState& d, const SphParams& P, uint32_t pass) {
-    if (P.fast)
+    if (P.fast == 1)
         k_vorticity_queue<true><<<queue_grid(k_vorticity_queue<true>, d), kQueueTile, 0, st>>>(d, P, pass);
     else
         k_vorticity_queue<false><<<queue_grid(k_vorticity_queue<false>, d), kQueueTile, 0, st>>>(d, P, pass);
 }
 void launch_confinement_queue(hipStream_t st, const DeviceState& d, const SphParams& P,
                               const StepParams& S, uint32_t pass) {
-    if (P.fast)
+    if (P.fast == 1)
         k_confinement_queue<true><<<queue_grid(k_confinement_queue<true>, d), kQueueTile, 0, st>>>(d, P, S, pass);
     else
         k_confinement_queue<false><<<queue_grid(k_confinement_queue<false>, d), kQueueTile, 0, st>>>(d, P, S, pass);

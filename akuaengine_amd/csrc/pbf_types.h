@@ -69,6 +69,8 @@ struct SphParams {
     // the artificial pressure need no upper-bound or divisor range test (their bounds, from h,
     // the kernel constants and delta_q, lie inside the exact-division range): the neighbour
     // sweeps then skip the multiplications by a neighbour's mass (identities) and those tests.
+    // 2 when the quotients are bounded and the masses came from device memory: the kernels look at
+    // DeviceState::massesDiffer.
     int32_t fast;
     // The squared lengths at which the rounded length leaves [1e-5, h], where the spiky gradient is
     // not zero: the smallest with sqrtf(d2) >= 1e-5 and the largest with sqrtf(d2) <= h (both from

@@ -264,6 +264,8 @@ struct akua_solver {
     bool hasState = false;
     bool exact = true;             // the autotuner keeps the reference's search (akua_solver_set_exact)
     bool unitMass = false;         // every particle's mass is exactly 1 (known from the upload)
+    bool deviceMasses = false;     // the masses came from device memory (akua_solver_step_device)
+    DevBuf<uint32_t> blockMasses, massesDiffer;  // what the device found in them
     bool boundedQuotients = false; // quotients_bounded(sph)
 
     // learned warm start
@@ -339,6 +341,7 @@ struct akua_solver {
         d.keysL = s1KA.p;
         d.skeys = d.skeysOut = r1 ? s1KB.p : s1KA.p;
         d.perm1 = d.perm1Out = r1 ? s1VB.p : s1VA.p;
+        d.blockMasses = blockMasses.p; d.massesDiffer = massesDiffer.p;
         d.groupCount = groupCount.p; d.groupBase = groupBase.p; d.placed = placed.p;
         d.groups = groups;
         d.groupShift = (uint32_t)std::max(0, hashBits - (int)ceil_log2(groups));
@@ -382,7 +385,7 @@ struct akua_solver {
         for (auto* b : {&dens, &lam, &Tdens, &Tlam, &size, &probeRho, &bndPsi, &net, &feat, &targ,
                         &lamHat, &adamM, &adamV, &part, &batchF, &batchT, &lossBuf})
             b->release();
-        for (auto* b : {&id, &Tid, &lid, &phys, &lidT, &physT, &srcL, &bslot, &nbr, &cnt,
+        for (auto* b : {&blockMasses, &massesDiffer, &id, &Tid, &lid, &phys, &lidT, &physT, &srcL, &bslot, &nbr, &cnt,
                         &perm2keep, &s1KA, &s1VA, &s1KB, &s1VB, &s2KA, &s2VA, &s2KB, &s2VB, &counts,
                         &totals, &look, &tickets, &counts2, &totals2, &look2, &tickets2, &gate, &fallbacks, &work, &cntW, &nbrW, &qcost,
                         &queue, &qcount, &heads})
@@ -518,6 +521,10 @@ void setup(akua_solver* s, const std::vector<uint32_t>& counts) {
         for (auto* l : {&s->look, &s->look2}) l->alloc((size_t)2 * s->numTiles * (1u << kMaxDigitBits));
         for (auto* t : {&s->tickets, &s->tickets2}) t->alloc((size_t)kMaxPasses);
     }
+    if (s->scenes.size() == 1) {  // record stepping is per single-scene solver
+        s->massesDiffer.alloc(1);
+        s->blockMasses.alloc((ns + 255) / 256);
+    }
     if (s->scenes.size() == 1 && s->nslots <= kOrderMaxSlots) {
         // about four particles a group: cells hold more, so that most groups are one cell
         s->groups = std::min(kOrderMaxGroups, std::max(256u, 1u << ceil_log2((s->nslots + 3u) / 4u)));
@@ -567,9 +574,11 @@ void setup(akua_solver* s, const std::vector<uint32_t>& counts) {
 }
 
 // SphParams::fast from the masses and the parameters; the step graphs capture the kernels it
-// selects, so a change re-captures them.
+// selects, so a change re-captures them.  Masses on the device are looked at in scenes of more than
+// kDeviceMassSlots: below, a sweep's time is its chain of loads, which the look at the flag lengthens.
+constexpr uint32_t kDeviceMassSlots = 1u << 15;
 void update_fast(akua_solver* s) {
-    const int f = (s->unitMass && s->boundedQuotients) ? 1 : 0;
+    const int f = !s->boundedQuotients ? 0 : s->deviceMasses && s->nslots > kDeviceMassSlots ? 2 : s->unitMass ? 1 : 0;
     if (s->sph.fast != f) {
         s->sph.fast = f;
         s->graphDirty = true;
@@ -1135,6 +1144,7 @@ void upload_soa(akua_solver* s, const float* pos, const float* vel, const float*
     s->hasState = true;
     s->layoutPhase = 0;  // the uploaded order is not cell ordered: re-sort on the next step
     s->unitMass = unit;
+    s->deviceMasses = false;
     update_fast(s);
 }
 
@@ -2016,10 +2026,12 @@ akua_status akua_solver_step_device(akua_solver* s, void* dParticles, int32_t n,
         HIP_CHECK(hipStreamWaitEvent(s->stream, ev, 0));
         auto* buf = static_cast<AosParticle*>(dParticles);
         launch_import_aos(s->stream, buf, (uint32_t)n, s->X.p, s->V.p, s->VS.p, s->DP.p, s->dens.p,
-                          s->lam.p, s->id.p, s->lid.p, s->phys.p, s->color.p, s->size.p);
+                          s->lam.p, s->id.p, s->lid.p, s->phys.p, s->color.p, s->size.p,
+                          s->blockMasses.p);
         s->hasState = true;
         s->layoutPhase = 0;
-        s->unitMass = false;  // the masses came from device memory: not known here
+        s->unitMass = false;  // the masses came from device memory: the kernels look at them
+        s->deviceMasses = true;
         update_fast(s);
         run_steps(s, dt, 1);
         DeviceState ds = s->devState();
