@@ -311,8 +311,28 @@ struct akua_solver {
     bool graphDirty = false;
     uint64_t stepsSinceStats = 0;
 
-    // step_device: orders the solver's stream with the caller's stream (created on first use)
-    hipEvent_t orderEvent = nullptr;
+    // step_device runs on the caller's stream: the end of its last step there, which the solver's own
+    // stream (joined()) waits for before its next work, and whether that stream has had work since
+    // step_device last waited for it (events created on first use)
+    hipEvent_t callerEvent = nullptr, orderEvent = nullptr;
+    hipStream_t callerStream = nullptr;
+    bool callerPending = false, ownPending = false;
+
+    // The solver's own stream, behind the steps on the caller's.
+    hipStream_t joined() {
+        if (callerPending) {
+            const hipError_t e = hipStreamWaitEvent(stream, callerEvent, 0);
+            if (e != hipSuccess) throw std::runtime_error(std::string("hipStreamWaitEvent: ") + hipGetErrorString(e));
+            callerPending = false;
+            callerStream = nullptr;
+        }
+        ownPending = true;
+        return stream;
+    }
+    void wait_for_caller() {
+        if (callerPending) (void)hipEventSynchronize(callerEvent);
+        callerPending = false;
+    }
     // record export staging (get_particles), allocated on first use
     DevBuf<AosParticle> aosStage;
     Staging staging;  // pinned chunks of get_state and get_particles, allocated on first use
@@ -368,6 +388,7 @@ struct akua_solver {
     // Teardown: wait for the stream's work, free the device buffers, then destroy the graphs,
     // the events and last the stream.
     ~akua_solver() {
+        wait_for_caller();
         if (stream) (void)hipStreamSynchronize(stream);
         release_buffers();
         staging.release();
@@ -375,6 +396,7 @@ struct akua_solver {
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
         for (auto e : eventPool) (void)hipEventDestroy(e);
         if (orderEvent) (void)hipEventDestroy(orderEvent);
+        if (callerEvent) (void)hipEventDestroy(callerEvent);
         if (stream) (void)hipStreamDestroy(stream);
     }
 
@@ -612,18 +634,18 @@ void timing_hook(void* ctx, const char* name, int phase) {
     auto* s = static_cast<akua_solver*>(ctx);
     if (phase == 0) {
         TimedLaunch t{name, next_event(s), nullptr};
-        HIP_CHECK(hipEventRecord(t.a, s->stream));
+        HIP_CHECK(hipEventRecord(t.a, s->joined()));
         s->pending.push_back(t);
     } else {
         TimedLaunch& t = s->pending.back();
         t.b = next_event(s);
-        HIP_CHECK(hipEventRecord(t.b, s->stream));
+        HIP_CHECK(hipEventRecord(t.b, s->joined()));
     }
 }
 
 void collect_timing(akua_solver* s) {
     if (s->pending.empty()) return;
-    HIP_CHECK(hipStreamSynchronize(s->stream));
+    HIP_CHECK(hipStreamSynchronize(s->joined()));
     for (auto& t : s->pending) {
         float ms = 0.0f;
         HIP_CHECK(hipEventElapsedTime(&ms, t.a, t.b));
@@ -865,7 +887,7 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
 
 void upload_scenes(akua_solver* s) {
     if (!s->scenesDirty) return;
-    HIP_CHECK(hipStreamSynchronize(s->stream));
+    HIP_CHECK(hipStreamSynchronize(s->joined()));
     HIP_CHECK(hipMemcpy(s->dScenes.p, s->scenes.data(), s->scenes.size() * sizeof(SceneDev),
                         hipMemcpyHostToDevice));
     s->scenesDirty = false;
@@ -964,7 +986,7 @@ void ensure_boundary(akua_solver* s) {
     const float sp = s->bndSpacing > 0.0f ? s->bndSpacing : s->cfg.particle_spacing;
     if (!build_boundary(sc.bmin, sc.bmax, sp, s->bndLayers, s->sph, s->cfg.restDensity, B, psi, err))
         fail(AKUA_ERR_INVALID_ARG, err);
-    HIP_CHECK(hipStreamSynchronize(s->stream));  // earlier steps may still read the old weights
+    HIP_CHECK(hipStreamSynchronize(s->joined()));  // earlier steps may still read the old weights
     if (s->bndPsi.n < psi.size()) s->bndPsi.alloc(psi.size());
     HIP_CHECK(hipMemcpy(s->bndPsi.p, psi.data(), psi.size() * sizeof(float), hipMemcpyHostToDevice));
     if (s->Bg.n < s->nslots) s->Bg.alloc(s->nslots);
@@ -978,7 +1000,7 @@ void ensure_boundary(akua_solver* s) {
 // capture: a graph records no allocation).
 void ensure_balance(akua_solver* s) {
     if (s->tuning.balanceTile <= 0 || s->nbrW.p) return;
-    HIP_CHECK(hipStreamSynchronize(s->stream));
+    HIP_CHECK(hipStreamSynchronize(s->joined()));
     s->work.alloc(s->nslots);
     s->cntW.alloc(s->nslots);
     s->nbrW.alloc(s->nbr.n);
@@ -991,7 +1013,7 @@ void ensure_queue(akua_solver* s) {
     if (s->tuning.workQueue <= 0) return;
     const uint32_t passes = queue_passes(s);
     if (s->queue.p && s->heads.n >= queue_heads_size(passes)) return;
-    HIP_CHECK(hipStreamSynchronize(s->stream));
+    HIP_CHECK(hipStreamSynchronize(s->joined()));
     const uint32_t ntiles = (s->nslots + kQueueTileSlots - 1) / kQueueTileSlots;
     const uint32_t t8 = (ntiles + kXcdCount - 1) / kXcdCount;
     s->qcost.alloc(std::max<uint32_t>(ntiles, 1));
@@ -1001,7 +1023,8 @@ void ensure_queue(akua_solver* s) {
     s->graphDirty = true;
 }
 
-void run_steps(akua_solver* s, float dt, int nsteps) {
+// On the solver's own stream, or (stream given) on the caller's, which step_device has put behind it.
+void run_steps(akua_solver* s, float dt, int nsteps, const hipStream_t* caller = nullptr) {
     if (!s->hasState) fail(AKUA_ERR_STATE, "set the particles before stepping");
     if (!(dt > 0.0f) || !std::isfinite(dt)) fail(AKUA_ERR_INVALID_ARG, "deltaTime must be > 0");
     upload_scenes(s);
@@ -1013,11 +1036,12 @@ void run_steps(akua_solver* s, float dt, int nsteps) {
         for (auto& g : s->graphs) g.dirty = true;
         s->graphDirty = false;
     }
+    const hipStream_t st = caller ? *caller : s->joined();
     for (int k = 0; k < nsteps; ++k) {
         // the physical layout is re-sorted every layoutInterval steps; it never changes a result
         const bool keep = s->layoutPhase != 0;
         if (s->timing) {
-            enqueue_step(s, s->stream, S, true, false, keep);
+            enqueue_step(s, st, S, true, false, keep);
             collect_timing(s);
         } else if (s->useGraph) {
             auto& G = s->graphs[keep ? 1 : 0];
@@ -1041,9 +1065,9 @@ void run_steps(akua_solver* s, float dt, int nsteps) {
                 G.tuning = s->tuning;
                 G.dirty = false;
             }
-            HIP_CHECK(hipGraphLaunch(G.exec, s->stream));
+            HIP_CHECK(hipGraphLaunch(G.exec, st));
         } else {
-            enqueue_step(s, s->stream, S, false, false, keep);
+            enqueue_step(s, st, S, false, false, keep);
         }
         HIP_CHECK(hipGetLastError());
         s->layoutPhase = (s->layoutPhase + 1) % std::max(1, s->tuning.layoutInterval);
@@ -1059,7 +1083,7 @@ void run_density_probe(akua_solver* s) {
     if (!s->hasState) fail(AKUA_ERR_STATE, "set the particles first");
     upload_scenes(s);
     const StepParams S0{0.0f, {0.0f, 0.0f, 0.0f}};
-    hipStream_t st = s->stream;
+    hipStream_t st = s->joined();
     DeviceState d = s->devState();
     // the probe's own walk uses cells of h whatever search the steps use
     SphParams P0 = s->sph;
@@ -1128,7 +1152,7 @@ void upload_soa(akua_solver* s, const float* pos, const float* vel, const float*
         }
     }
     (void)n;
-    HIP_CHECK(hipStreamSynchronize(s->stream));
+    HIP_CHECK(hipStreamSynchronize(s->joined()));
     HIP_CHECK(hipMemcpy(s->X.p, X.data(), X.size() * sizeof(float4), hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(s->V.p, V.data(), V.size() * sizeof(float4), hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(s->VS.p, VS.data(), VS.size() * sizeof(float4), hipMemcpyHostToDevice));
@@ -1151,7 +1175,7 @@ void upload_soa(akua_solver* s, const float* pos, const float* vel, const float*
 template <class T>
 std::vector<T> download(akua_solver* s, const T* p, size_t n) {
     std::vector<T> h(n);
-    HIP_CHECK(hipStreamSynchronize(s->stream));
+    HIP_CHECK(hipStreamSynchronize(s->joined()));
     if (n) HIP_CHECK(hipMemcpy(h.data(), p, n * sizeof(T), hipMemcpyDeviceToHost));
     return h;
 }
@@ -1181,7 +1205,7 @@ void read_back(akua_solver* s, const std::vector<Readback>& pieces) {
     for (const Readback& r : pieces) total += r.bytes;
     if (!total) return;
     if (!s->staging.ensure(total)) {
-        HIP_CHECK(hipStreamSynchronize(s->stream));
+        HIP_CHECK(hipStreamSynchronize(s->joined()));
         for (const Readback& r : pieces) HIP_CHECK(hipMemcpy(r.to, r.from, r.bytes, hipMemcpyDeviceToHost));
         return;
     }
@@ -1193,15 +1217,15 @@ void read_back(akua_solver* s, const std::vector<Readback>& pieces) {
                              std::min(chunk, r.bytes - o)});
     const auto issue = [&](size_t k) {
         HIP_CHECK(hipMemcpyAsync(s->staging.chunk[k % ring], parts[k].from, parts[k].bytes, hipMemcpyDeviceToHost,
-                                 s->stream));
-        HIP_CHECK(hipEventRecord(s->staging.ready[k % ring], s->stream));
+                                 s->joined()));
+        HIP_CHECK(hipEventRecord(s->staging.ready[k % ring], s->joined()));
     };
     const auto empty = [&](size_t k) { std::memcpy(parts[k].to, s->staging.chunk[k % ring], parts[k].bytes); };
     // whatever happens, no copy into the chunks is left in flight
     struct Drain {
         hipStream_t st;
         ~Drain() { (void)hipStreamSynchronize(st); }
-    } drain{s->stream};
+    } drain{s->joined()};
 
     if (total <= kReadbackInline) {
         size_t issued = 0;
@@ -1327,7 +1351,7 @@ void take_snapshot(akua_solver* s, Snapshot& q) {
     q.X.alloc(n); q.V.alloc(n); q.W.alloc(n); q.VS.alloc(n); q.DP.alloc(n);
     q.dens.alloc(n); q.lam.alloc(n);
     q.id.alloc(n); q.lid.alloc(n);
-    hipStream_t st = s->stream;
+    hipStream_t st = s->joined();
     copy_dev(q.X.p, s->X.p, n, st); copy_dev(q.V.p, s->V.p, n, st); copy_dev(q.W.p, s->W.p, n, st);
     copy_dev(q.VS.p, s->VS.p, n, st); copy_dev(q.DP.p, s->DP.p, n, st);
     copy_dev(q.dens.p, s->dens.p, n, st); copy_dev(q.lam.p, s->lam.p, n, st);
@@ -1337,7 +1361,7 @@ void take_snapshot(akua_solver* s, Snapshot& q) {
 void restore_snapshot(akua_solver* s, const Snapshot& q) {
     const size_t n = s->nslots;
     s->layoutPhase = 0;
-    hipStream_t st = s->stream;
+    hipStream_t st = s->joined();
     copy_dev(s->X.p, q.X.p, n, st); copy_dev(s->V.p, q.V.p, n, st); copy_dev(s->W.p, q.W.p, n, st);
     copy_dev(s->VS.p, q.VS.p, n, st); copy_dev(s->DP.p, q.DP.p, n, st);
     copy_dev(s->dens.p, q.dens.p, n, st); copy_dev(s->lam.p, q.lam.p, n, st);
@@ -1357,9 +1381,9 @@ double time_trial(akua_solver* s, const Snapshot& q, float dt, int steps) {
     double best = 0.0;
     hipError_t e = hipSuccess;
     for (int r = 0; r < 2 && e == hipSuccess; ++r) {
-        HIP_CHECK(hipEventRecord(a, s->stream));
+        HIP_CHECK(hipEventRecord(a, s->joined()));
         run_steps(s, dt, steps);
-        HIP_CHECK(hipEventRecord(b, s->stream));
+        HIP_CHECK(hipEventRecord(b, s->joined()));
         HIP_CHECK(hipEventSynchronize(b));
         float ms = 0.0f;
         e = hipEventElapsedTime(&ms, a, b);
@@ -1500,7 +1524,7 @@ void check_network(const float* p) {
 void upload_network(akua_solver* s, const float* p) {
     check_network(p);
     ensure_learned(s);
-    HIP_CHECK(hipStreamSynchronize(s->stream));
+    HIP_CHECK(hipStreamSynchronize(s->joined()));
     HIP_CHECK(hipMemcpy(s->net.p, p, kMlpParams * sizeof(float), hipMemcpyHostToDevice));
     s->haveNet = true;
     reset_adam(s);
@@ -1600,7 +1624,7 @@ void train(akua_solver* s, float dt, const float* bmin, const float* bmax, int s
     ensure_train(s, B, perStep * (uint32_t)steps);
     ensure_balance(s);
     HIP_CHECK(hipMemset(s->lossBuf.p, 0, (size_t)perStep * steps * sizeof(float)));
-    hipStream_t st = s->stream;
+    hipStream_t st = s->joined();
     const StepParams S{dt, {s->cfg.gravity[0], s->cfg.gravity[1], s->cfg.gravity[2]}};
     MlpLossWeights lw{{c.lossWeights[0], c.lossWeights[1], c.lossWeights[2], c.lossWeights[3]}};
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -1720,7 +1744,7 @@ void autotune(akua_solver* s, float dt, const float* bmin, const float* bmax, in
                 apply_search(s, cells);
                 apply_tuning(s, tuning);
                 restore_snapshot(s, q);
-                (void)hipStreamSynchronize(s->stream);
+                (void)hipStreamSynchronize(s->joined());
             } catch (...) {
             }
         }
@@ -1782,7 +1806,7 @@ void autotune(akua_solver* s, float dt, const float* bmin, const float* bmax, in
     }
     apply_tuning(s, best);
     restore_snapshot(s, q);
-    HIP_CHECK(hipStreamSynchronize(s->stream));
+    HIP_CHECK(hipStreamSynchronize(s->joined()));
     guard.armed = false;
     s->timing = timing;
     s->useGraph = graph;
@@ -1913,6 +1937,7 @@ akua_status akua_batch_density_error(akua_solver* s, float* maxError, double* me
 akua_status akua_solver_destroy(akua_solver* s) {
     return guarded([&] {
         if (!s) return;
+        s->wait_for_caller();
         if (s->stream) (void)hipStreamSynchronize(s->stream);
         delete s;
     });
@@ -1956,7 +1981,7 @@ akua_status akua_solver_get_state(akua_solver* s, float* pos, float* vel, float*
         float* const rest = reinterpret_cast<float*>(s->XsC.p);
         const StateArrays out{reinterpret_cast<float*>(s->X0.p), reinterpret_cast<float*>(s->Vc.p), rest, rest + np,
                               rest + 2 * np, reinterpret_cast<uint32_t*>(rest + 3 * np)};
-        launch_export_state(s->stream, out, s->nparticles, s->nslots, s->dScenes.p, s->dChunkScene.p, s->X.p, s->V.p,
+        launch_export_state(s->joined(), out, s->nparticles, s->nslots, s->dScenes.p, s->dChunkScene.p, s->X.p, s->V.p,
                             s->dens.p, s->lam.p, s->id.p, s->lid.p);
         HIP_CHECK(hipGetLastError());
         std::vector<Readback> pieces;
@@ -1980,7 +2005,7 @@ akua_status akua_solver_get_particles(akua_solver* s, akua_particle* out, int32_
         if (s->scenes.size() != 1) fail(AKUA_ERR_UNSUPPORTED, "record export is per single-scene solver");
         if (s->aosStage.n < (size_t)n) s->aosStage.alloc((size_t)n);
         DeviceState ds = s->devState();
-        launch_export_aos(s->stream, s->aosStage.p, (uint32_t)n, s->X.p, s->V.p, s->VS.p, s->DP.p,
+        launch_export_aos(s->joined(), s->aosStage.p, (uint32_t)n, s->X.p, s->V.p, s->VS.p, s->DP.p,
                           s->dens.p, s->lam.p, s->id.p, s->lid.p, s->W.p, ds.skeys, s->color.p,
                           s->size.p);
         HIP_CHECK(hipGetLastError());
@@ -2019,27 +2044,58 @@ akua_status akua_solver_step_device(akua_solver* s, void* dParticles, int32_t n,
         // NULL is the null stream: the solver's own stream does not synchronise with it, so the
         // order is made explicit for every caller stream
         hipStream_t user = static_cast<hipStream_t>(stream);
-        if (!s->orderEvent) HIP_CHECK(hipEventCreateWithFlags(&s->orderEvent, hipEventDisableTiming));
-        hipEvent_t ev = s->orderEvent;
-        // the solver's stream waits for the caller's earlier work on the buffer
-        HIP_CHECK(hipEventRecord(ev, user));
-        HIP_CHECK(hipStreamWaitEvent(s->stream, ev, 0));
         auto* buf = static_cast<AosParticle*>(dParticles);
-        launch_import_aos(s->stream, buf, (uint32_t)n, s->X.p, s->V.p, s->VS.p, s->DP.p, s->dens.p,
-                          s->lam.p, s->id.p, s->lid.p, s->phys.p, s->color.p, s->size.p,
-                          s->blockMasses.p);
-        s->hasState = true;
-        s->layoutPhase = 0;
-        s->unitMass = false;  // the masses came from device memory: the kernels look at them
-        s->deviceMasses = true;
-        update_fast(s);
-        run_steps(s, dt, 1);
-        DeviceState ds = s->devState();
-        launch_export_aos(s->stream, buf, (uint32_t)n, s->X.p, s->V.p, s->VS.p, s->DP.p, s->dens.p,
-                          s->lam.p, s->id.p, s->lid.p, s->W.p, ds.skeys, s->color.p, s->size.p);
-        // the caller's later work on its stream waits for the written-back records
-        HIP_CHECK(hipEventRecord(ev, s->stream));
-        HIP_CHECK(hipStreamWaitEvent(user, ev, 0));
+        const auto step = [&](hipStream_t st, const hipStream_t* caller) {
+            launch_import_aos(st, buf, (uint32_t)n, s->X.p, s->V.p, s->VS.p, s->DP.p, s->dens.p,
+                              s->lam.p, s->id.p, s->lid.p, s->phys.p, s->color.p, s->size.p, s->blockMasses.p);
+            s->hasState = true;
+            s->layoutPhase = 0;
+            s->unitMass = false;  // the masses came from device memory: the kernels look at them
+            s->deviceMasses = true;
+            update_fast(s);
+            run_steps(s, dt, 1, caller);
+            DeviceState ds = s->devState();
+            launch_export_aos(st, buf, (uint32_t)n, s->X.p, s->V.p, s->VS.p, s->DP.p, s->dens.p,
+                              s->lam.p, s->id.p, s->lid.p, s->W.p, ds.skeys, s->color.p, s->size.p);
+        };
+        for (hipEvent_t* e : {&s->callerEvent, &s->orderEvent})
+            if (!*e) HIP_CHECK(hipEventCreateWithFlags(e, hipEventDisableTiming));
+        // The step runs on the caller's stream itself: between two streams every step waits for an event
+        // twice, some 40 us in which the chip is idle (1,000 particles: 111 us a step so, 71 here).  A
+        // stream that is being captured and timed steps keep to the solver's own.
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(user, &capture) != hipSuccess) {
+            (void)hipGetLastError();
+            capture = hipStreamCaptureStatusActive;
+        }
+        if (capture != hipStreamCaptureStatusNone || s->timing) {
+            // the solver's stream waits for the caller's earlier work on the buffer
+            HIP_CHECK(hipEventRecord(s->orderEvent, user));
+            HIP_CHECK(hipStreamWaitEvent(s->joined(), s->orderEvent, 0));
+            step(s->joined(), nullptr);
+            // the caller's later work on its stream waits for the written-back records
+            HIP_CHECK(hipEventRecord(s->orderEvent, s->joined()));
+            HIP_CHECK(hipStreamWaitEvent(user, s->orderEvent, 0));
+        } else {
+            if (s->ownPending) {  // behind the work on the solver's own stream
+                HIP_CHECK(hipEventRecord(s->orderEvent, s->stream));
+                HIP_CHECK(hipStreamWaitEvent(user, s->orderEvent, 0));
+            }
+            if (s->callerPending && s->callerStream != user)  // behind steps on another stream
+                HIP_CHECK(hipStreamWaitEvent(user, s->callerEvent, 0));
+            s->ownPending = false;
+            // whatever happens, what was enqueued is known to later work on the solver's own stream
+            struct Ended {
+                akua_solver* s;
+                hipStream_t user;
+                ~Ended() {
+                    s->callerPending = hipEventRecord(s->callerEvent, user) == hipSuccess;
+                    s->callerStream = user;
+                    if (!s->callerPending) (void)hipStreamSynchronize(user);
+                }
+            } ended{s, user};
+            step(user, &user);
+        }
         HIP_CHECK(hipGetLastError());
     });
 }
@@ -2056,7 +2112,7 @@ akua_status akua_solver_set_gravity(akua_solver* s, const float g[3]) {
 akua_status akua_solver_synchronize(akua_solver* s) {
     return guarded([&] {
         if (!s) fail(AKUA_ERR_INVALID_ARG, "NULL solver");
-        HIP_CHECK(hipStreamSynchronize(s->stream));
+        HIP_CHECK(hipStreamSynchronize(s->joined()));
     });
 }
 
@@ -2195,7 +2251,7 @@ akua_status akua_debug_boundary(akua_solver* s, float* pos, float* psi, int32_t 
         if (pos)
             for (uint32_t i = 0; i < k; ++i) boundary_position(B, i, pos + 3 * (size_t)i);
         if (psi && k) {
-            HIP_CHECK(hipStreamSynchronize(s->stream));
+            HIP_CHECK(hipStreamSynchronize(s->joined()));
             HIP_CHECK(hipMemcpy(psi, s->bndPsi.p, (size_t)k * sizeof(float), hipMemcpyDeviceToHost));
         }
     });
@@ -2278,11 +2334,11 @@ akua_status akua_render(akua_solver* s, const akua_camera* cam, int32_t width, i
         R.drawFloor = drawFloor ? 1 : 0;
         const size_t pixels = (size_t)width * (size_t)height;
         if (s->renderKeys.n < pixels || s->renderRgb.n < 3 * pixels) {
-            HIP_CHECK(hipStreamSynchronize(s->stream));
+            HIP_CHECK(hipStreamSynchronize(s->joined()));
             if (s->renderKeys.n < pixels) s->renderKeys.alloc(pixels);
             if (s->renderRgb.n < 3 * pixels) s->renderRgb.alloc(3 * pixels);
         }
-        launch_render(s->stream, s->X.p, s->color.p, s->size.p, s->id.p, s->lid.p, s->phys.p,
+        launch_render(s->joined(), s->X.p, s->color.p, s->size.p, s->id.p, s->lid.p, s->phys.p,
                       s->scenes[0].end, R, s->renderKeys.p, s->renderRgb.p);
         HIP_CHECK(hipGetLastError());
         read_back(s, {{rgb, s->renderRgb.p, 3 * pixels}});
@@ -2596,7 +2652,7 @@ akua_status akua_solver_mean_neighbours(akua_solver* s, double* mean) {
             *mean = 0.0;
             return;
         }
-        launch_count_sum(s->stream, s->devState(), s->nbrSum.p, kCountBlocks);
+        launch_count_sum(s->joined(), s->devState(), s->nbrSum.p, kCountBlocks);
         HIP_CHECK(hipGetLastError());
         auto v = download(s, s->nbrSum.p, kCountBlocks);
         unsigned long long t = 0;
