@@ -420,6 +420,16 @@ struct akua_solver {
 
 namespace {
 
+// The physical layout is left to the solver: every setting of it at its default.  Then super-cells are
+// single cells, whose layout keys sort in the hash sort's launches (1M dam break 1,344 -> 1,284 us a step,
+// with the learned warm start 1,096 -> 1,035, 64 scenes 2,524 -> 2,480 against super-cells of 2^3).
+bool layout_by_solver(const akua_solver* s) {
+    const akua_tuning& t = s->tuning;
+    return t.layoutLevel == kDefaultTuning.layoutLevel && t.hashDigitBits == kDefaultTuning.hashDigitBits &&
+           t.layoutDigitBits == kDefaultTuning.layoutDigitBits && t.layoutInterval == kDefaultTuning.layoutInterval;
+}
+int layout_level(const akua_solver* s) { return layout_by_solver(s) ? 0 : s->tuning.layoutLevel; }
+
 void update_layout(akua_solver* s);
 
 // The multiply-high modulo must agree with % for this divisor; checked on edge values and a
@@ -727,10 +737,7 @@ SweepLanes sweep_lanes(const akua_solver* s) {
 // Whether the step orders its particles by launch_order: a small single scene whose layout is left to
 // the solver, with the reference's search.
 bool small_order(const akua_solver* s) {
-    const akua_tuning& t = s->tuning;
-    return s->groups > 0 && s->sph.searchCells == 1 && t.layoutLevel == kDefaultTuning.layoutLevel &&
-           t.hashDigitBits == kDefaultTuning.hashDigitBits && t.layoutDigitBits == kDefaultTuning.layoutDigitBits &&
-           t.layoutInterval == kDefaultTuning.layoutInterval;
+    return s->groups > 0 && s->sph.searchCells == 1 && layout_by_solver(s);
 }
 
 void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool timed,
@@ -747,7 +754,7 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
     } else {
         // single-cell super-cells: the layout keys are sorted in the previous logical order, which
         // agrees with the new one within each key, so both sorts share their launches
-        const bool together = !keepLayout && s->tuning.layoutLevel == 0 && s->plan1.digitBits == s->plan2.digitBits;
+        const bool together = !keepLayout && layout_level(s) == 0 && s->plan1.digitBits == s->plan2.digitBits;
         // the prediction's launch also clears the cell table and, for paired look-back sorts, their
         // scratch
         const SortZeroSpans zero = together ? sort_both_zero_spans(s) : SortZeroSpans{};
@@ -909,7 +916,7 @@ constexpr int kLayoutMarginCells = 4;
 
 void update_layout(akua_solver* s) {
     int bits = 1;
-    const int L = s->tuning.layoutLevel;
+    const int L = layout_level(s);
     const float span = (float)(1 << L);
     const int margin = std::max(1, (kLayoutMarginCells + (1 << L) - 1) >> L);  // in super-cells
     for (SceneDev& sc : s->scenes) {
