@@ -40,6 +40,7 @@ namespace akua {
 
 struct DeviceState {
     uint32_t nslots;           // particle slots (all scenes, with alignment padding)
+    uint32_t nparticles;
     const SceneDev* scenes;
     const uint32_t* chunkScene;  // scene of each 256-slot chunk
     float4* X;
@@ -78,6 +79,12 @@ struct DeviceState {
     // SphParams::fast 2: per 256 imported records, whether a mass differs from 1; of all of them
     const uint32_t* blockMasses;
     uint32_t* massesDiffer;
+    // larger scenes (launch_tally): the particles of each group, then of each bin, and their prefix
+    uint32_t* tally;
+    uint32_t* tallyBase;       // tallyCount + 1 entries
+    uint32_t* tallyPart;       // per workgroup of the prefix
+    uint32_t tallyGroups, tallyCount;  // groups, groups and bins, of all scenes
+    uint4* tallied;            // (hash, previous logical index, place in its group, bin) of each slot
     uint32_t* skeysOut;        // skeys and perm1, for their writer
     uint32_t* perm1Out;
     uint32_t* keysM;           // super-cell Morton keys in logical order (second sort's input)
@@ -152,9 +159,14 @@ void launch_gather(hipStream_t st, const DeviceState& d, const SphParams& P, con
 // Physical start and contiguity of every bucket (after the gather).
 void launch_bucket_phys(hipStream_t st, const DeviceState& d);
 // phys[lid[p]] = p over every scene's slots.
+// Larger single scenes whose boxes have not many more cells than particles: the same in five launches,
+// with the cell order in memory.  kTallyBlock counters per workgroup of the prefix.
+constexpr uint32_t kTallyBlock = 8192;
+void launch_tally(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
+                  bool carryDelta);
 // Small single scenes: hashes, both orders (the physical is the logical), the cell table and the move,
 // instead of launch_predict_hash, the two sorts, launch_cell_keys, launch_gather and launch_bucket_phys.
-constexpr uint32_t kOrderMaxSlots = 1u << 17, kOrderMaxGroups = 1u << 13;
+constexpr uint32_t kOrderMaxSlots = 1u << 15, kOrderMaxGroups = 1u << 13;
 void launch_order(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
                   bool carryDelta);
 // The neighbour lists.  Below: bs is the workgroup size of the neighbour sweeps (128, 256 or 512;

@@ -19,9 +19,8 @@
 // launch-then-synchronise sequence, except XSPH, which reads a copy of the velocities instead of
 // racing on them.
 //
-// Kernels that walk neighbours map workgroups to XCDs by contiguous ranges of physical slots:
-// the hardware places workgroup b on XCD b % 8, so workgroup b takes chunk (b % 8) * (nb / 8) +
-// b / 8 and each XCD's L2 serves one spatially coherent eighth of the particles.
+// Kernels that walk neighbours map workgroups to XCDs by chunks of physical slots (xcd_block), so that
+// each XCD's L2 serves spatially coherent ranges of the particles.
 #include "pbf_kernels.h"
 
 #include <algorithm>
@@ -111,19 +110,30 @@ __device__ __forceinline__ T ld(const T* __restrict__ base, uint32_t j) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (uint32_t)(j * (uint32_t)sizeof(T)));
 }
 
-// Physical slot of this thread under the XCD-contiguous workgroup order (the grid is a multiple
-// of 8 workgroups of BS threads).
-template <int BS>
+// The work of workgroup b of nb (a multiple of 8), of `per` slots each: the hardware places b on XCD b % 8,
+// which takes every eighth chunk of kXcdChunk slots, and of the rest a contiguous eighth.  A chunk's data
+// and its surroundings stay in one XCD's L2; eighths of a whole scene differ in density, so that one XCD
+// works longest (us per step by launch_tally, one eighth / chunks of 32,768 / 4,096: 8M two columns 14,596 /
+// 11,370 / 11,213, sprayed 1M 1,394 / 1,257 / 1,281, learned 1M 959 / 942 / 938; 64 scenes 2,449 / 2,468 /
+// 2,461).
+constexpr uint32_t kXcdChunk = 32768u;
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb, uint32_t per) {
+    const uint32_t x = b % kXcds, j = b / kXcds, mine = nb / kXcds;
+    const uint32_t c = kXcdChunk / per, whole = mine / c * c;
+    return j < whole ? (j / c * kXcds + x) * c + j % c : whole * kXcds + x * (mine - whole) + (j - whole);
+}
+
+// Physical slot of this thread (with L lanes per slot: its lane's index among all slots' lanes).
+template <int BS, int L = 1>
 __device__ __forceinline__ uint32_t xcd_slot() {
-    const uint32_t nb = gridDim.x, b = blockIdx.x;
-    return ((b % kXcds) * (nb / kXcds) + b / kXcds) * BS + threadIdx.x;
+    return xcd_block(blockIdx.x, gridDim.x, BS / L) * BS + threadIdx.x;
 }
 
 // The same slot for virtual workgroup vb of nvb (a kernel that loops over virtual workgroups
 // with a smaller grid).
 template <int BS>
 __device__ __forceinline__ uint32_t xcd_slot_of(uint32_t vb, uint32_t nvb) {
-    return ((vb % kXcds) * (nvb / kXcds) + vb / kXcds) * BS + threadIdx.x;
+    return xcd_block(vb, nvb, BS) * BS + threadIdx.x;
 }
 
 __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t n, uint32_t v) {
@@ -333,10 +343,9 @@ __device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
 // Up to kOrderMaxSlots slots of a single scene take three launches where the two radix sorts, the cell
 // table and the move take thirteen, each at the launch's own cost (27,000 particles: 85 us of a 235 us
 // step before, 14 now; 1,000: 57 and 13).  The physical order is the logical order: the particles of a
-// cell are still neighbours in memory, and the arrays of such a scene fit the caches.  The sweeps lose
-// a little to it where they no longer do, which sets the limit: us per step against the (paired) sorts
-// and the cell order, 27,000 particles 107 / 139, 60,000 157 / 183, 100,000 221 / 243, 130,000 258 / 271
-// (sprayed 291 / 292).
+// cell are still neighbours in memory, and the arrays of such a scene fit the caches.  Larger scenes gain
+// more from the cell order than its two further launches cost (launch_tally; us per step so / there: 16,000
+// particles 87 / 90, 27,000 106 / 108, 32,000 sprayed 126 / 119, 40,000 134 / 124, 130,000 260 / 232).
 //   1. k_order_count: hashes; each particle takes a place in the group of its hash's upper bits;
 //   2. k_order_place: the groups' prefix (each workgroup its own, in LDS), hashes to their groups;
 //   3. k_order_rank: each particle's rank by (hash, previous logical index) among its group's few
@@ -479,6 +488,185 @@ __global__ __launch_bounds__(kBlock) void k_order_rank(DeviceState d, StepParams
     d.Tid[to] = id;
     d.lidT[to] = to;
     d.physT[to] = to;
+}
+
+// ---- larger scenes: both orders by counting, in five launches ----------------------------------------
+// The same idea where the cell order in memory is worth having: besides its group of hashes a particle is
+// counted in the bin of its cell, one prefix over groups and bins together gives the first place of each,
+// and the rank among its group's members also gives its place in the bin (a cell has one hash, so all its
+// particles are in one group).  Bins are the cells of the box and a few beyond, in cubes of 2^cubeLog2
+// cells with the Morton order inside; cells farther out share one bin per group.
+// Against the two radix sorts in shared launches, the cell table and the move (kernel time at 1M): 180 ->
+// 112 us in a settled flow, 266 -> 237 sprayed, where particles of a cell seldom lie side by side and the
+// counting (22 -> 92 us) and ranking (65 -> 110) slow down.
+
+// Bin of a cell within the scene; outside the range the group's.  The groups' bins lie behind blocks of
+// cells' bins, 2^binSpare to each: particles far out list slowly and sweep fast, so they are spread over
+// the scene (behind all cells they are one XCD's: list build of 8M sprayed particles 2.35 -> 3.32 ms).
+__device__ __forceinline__ uint32_t cell_bin(int cx, int cy, int cz, uint32_t group, const SceneDev& sc) {
+    const uint32_t u = (uint32_t)cx - (uint32_t)sc.binOrigin[0], v = (uint32_t)cy - (uint32_t)sc.binOrigin[1],
+                   w = (uint32_t)cz - (uint32_t)sc.binOrigin[2];
+    if (u >= sc.binCells[0] || v >= sc.binCells[1] || w >= sc.binCells[2])
+        return (((group >> sc.binSpare) + 1u) << sc.binBlock) + group;
+    const uint32_t c = sc.cubeLog2, low = (1u << c) - 1u;
+    const uint32_t cube = (u >> c) * sc.cubeStride[0] + (v >> c) * sc.cubeStride[1] + (w >> c) * sc.cubeStride[2];
+    const uint32_t b = (cube << (3u * c)) | spread3(u & low) | (spread3(v & low) << 1) | (spread3(w & low) << 2);
+    return b + ((b >> sc.binBlock) << sc.binSpare);
+}
+
+__global__ __launch_bounds__(kBlock) void k_tally_count(DeviceState d, SphParams P, StepParams S, uint32_t countBlocks) {
+    if (blockIdx.x == gridDim.x - 1u) {
+        gather_masses(d, P);
+        return;
+    }
+    if (blockIdx.x >= countBlocks) {
+        const uint32_t i = (blockIdx.x - countBlocks) * kBlock + threadIdx.x;
+        if (i < d.tableTotal) d.table[i] = make_uint4(kEmptyKey, kEmptyKey, kEmptyKey, kEmptyKey);
+        return;
+    }
+    const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    const SceneDev& sc = d.scenes[d.chunkScene[min(p, d.nslots - 1u) >> 8]];
+    const bool valid = p < d.nslots && p < sc.end;
+    uint32_t h = 0, k = 0, group = 0, bin = kEmptyKey;
+    if (valid) {
+        k = d.lid[p];
+        const f3 xs = predict_x(make3(d.X[p]), make3(d.V[p]), S);
+        int cx, cy, cz;
+        discretize(xs, P.cellHash, cx, cy, cz);
+        h = cell_hash(cx, cy, cz, sc);
+        group = h >> sc.groupShift;
+        bin = cell_bin(cx, cy, cz, group, sc) + sc.binBegin;
+        group += sc.groupBegin;
+    }
+    // by runs of one bin and group (particles of a cell mostly lie side by side; a wave is of one scene)
+    const uint32_t lane = __lane_id();
+    const uint32_t bin1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)bin, 0x138, 0xF, 0xF, false);  // wave_shr:1
+    const uint64_t heads = __ballot(lane == 0u || bin1 != bin);
+    const uint32_t head = 63u - (uint32_t)__builtin_clzll(heads & (~0ull >> (63u - lane)));
+    uint32_t place = 0;
+    if (valid && lane == head) {
+        const uint64_t after = lane == 63u ? 0ull : heads & (~0ull << (lane + 1u));
+        const uint32_t length = (after ? (uint32_t)__builtin_ctzll(after) : 64u) - lane;
+        place = atomicAdd(&d.tally[group], length);
+        atomicAdd(&d.tally[d.tallyGroups + bin], length);
+    }
+    place = (uint32_t)__shfl((int)place, (int)head, 64) + (lane - head);
+    if (valid) d.tallied[p] = make_uint4(h, k, place, bin);
+}
+
+// The prefix, kTallyBlock counters per workgroup, eight per thread: each workgroup's sum, then its prefix
+// behind the sums before it.  The counters are read for the last time there and are left empty.
+constexpr uint32_t kTallyThreads = kTallyBlock / 8u;
+
+__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* waves) {
+    const uint32_t inclusive = wave_prefix(v);
+    if (__lane_id() == 63u) waves[threadIdx.x >> 6] = inclusive;
+    __syncthreads();
+    uint32_t sum = 0;
+    for (uint32_t w = 0; w < kTallyThreads / 64u; ++w) sum += waves[w];
+    __syncthreads();
+    return sum;
+}
+
+__global__ __launch_bounds__(kTallyThreads) void k_tally_sum(DeviceState d) {
+    __shared__ uint32_t waves[kTallyThreads / 64u];
+    const uint4* const c = reinterpret_cast<const uint4*>(d.tally) + (size_t)blockIdx.x * (kTallyBlock / 4u) + 2u * threadIdx.x;
+    const uint4 a = c[0], b = c[1];
+    const uint32_t sum = block_sum(((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w)), waves);
+    if (threadIdx.x == 0) d.tallyPart[blockIdx.x] = sum;
+}
+
+__global__ __launch_bounds__(kTallyThreads) void k_tally_prefix(DeviceState d) {
+    __shared__ uint32_t waves[kTallyThreads / 64u];
+    uint4* const c = reinterpret_cast<uint4*>(d.tally) + (size_t)blockIdx.x * (kTallyBlock / 4u) + 2u * threadIdx.x;
+    const uint4 a = c[0], b = c[1];
+    uint32_t before = 0;
+    for (uint32_t k = threadIdx.x; k < blockIdx.x; k += kTallyThreads) before += d.tallyPart[k];
+    before = block_sum(before, waves);
+    const uint32_t sum = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
+    const uint32_t inclusive = wave_prefix(sum);
+    if (__lane_id() == 63u) waves[threadIdx.x >> 6] = inclusive;
+    __syncthreads();
+    uint32_t run = before + inclusive - sum;
+    for (uint32_t w = 0; w < (threadIdx.x >> 6); ++w) run += waves[w];
+    uint4 x, y;
+    x.x = run;       x.y = x.x + a.x; x.z = x.y + a.y; x.w = x.z + a.z;
+    y.x = x.w + a.w; y.y = y.x + b.x; y.z = y.y + b.y; y.w = y.z + b.z;
+    uint4* const out = reinterpret_cast<uint4*>(d.tallyBase) + (size_t)blockIdx.x * (kTallyBlock / 4u) + 2u * threadIdx.x;
+    out[0] = x;
+    out[1] = y;
+    c[0] = c[1] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+__global__ __launch_bounds__(kBlock) void k_tally_place(DeviceState d) {
+    const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    if (p >= d.nslots) return;
+    const SceneDev& sc = scene_of(d, p);
+    if (p >= sc.end) return;
+    const uint4 r = d.tallied[p];
+    const uint32_t q = d.tallyBase[sc.groupBegin + (r.x >> sc.groupShift)] + r.z;
+    if (q < d.nslots) d.placed[q] = make_uint4(r.x, r.y, p, r.w);
+}
+
+// kCarry, kCarryDelta: as in k_gather.
+template <bool kCarry, bool kCarryDelta>
+__global__ __launch_bounds__(kBlock) void k_tally_rank(DeviceState d, StepParams S, uint32_t nparticles) {
+    const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
+    if (q >= nparticles) return;
+    const uint4 me = d.placed[q];
+    const uint32_t h = me.x, k = me.y, src = me.z, bin = me.w;
+    if (src >= d.nslots) return;  // consistent counts never produce this
+    const SceneDev& sc = scene_of(d, src);
+    const uint32_t group = sc.groupBegin + (h >> sc.groupShift);
+    if (group >= d.tallyGroups || d.tallyGroups + bin >= d.tallyCount) return;  // nor this
+    const float4 x = d.X[src], v = d.V[src];
+    const uint32_t id = d.id[src];
+    const uint32_t b = d.tallyBase[group], e = min(d.tallyBase[group + 1u], nparticles);
+    const uint32_t binFirst = d.tallyBase[d.tallyGroups + bin] - nparticles;
+    // among the group: smaller hashes, the bucket, those of it before this particle, those of it in the same
+    // bin, and those in the same bin before this particle by hash and index
+    uint32_t smaller = 0, same = 0, sameBefore = 0, sameBin = 0, binBefore = 0;
+    constexpr uint32_t kBatch = 4;
+    for (uint32_t m0 = b; m0 < e; m0 += kBatch) {
+        uint4 o[kBatch];
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) o[u] = d.placed[min(m0 + u, e - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) {
+            const bool in = m0 + u < e, less = in && o[u].x < h, equal = in && o[u].x == h, mine = o[u].w == bin;
+            const bool before = equal && o[u].y < k;
+            smaller += less ? 1u : 0u;
+            same += equal ? 1u : 0u;
+            sameBefore += before ? 1u : 0u;
+            sameBin += equal && mine ? 1u : 0u;
+            binBefore += (less || before) && mine ? 1u : 0u;
+        }
+    }
+    const uint32_t shift = sc.begin - sc.first;  // slots of earlier scenes' padding
+    const uint32_t first = b + smaller + shift, to = first + sameBefore, p = binFirst + binBefore + shift;
+    if (to >= sc.end || p >= sc.end) return;  // consistent counts never produce this
+    if (sameBefore == 0u) {
+        const uint32_t slot = table_insert(d.table, sc, h);
+        if (slot != kEmptyKey) {
+            d.table[slot].y = first;
+            d.table[slot].z = first + same;
+            // one bin: the bucket's particles lie side by side in logical order (256 at most, as in k_bucket_phys)
+            d.table[slot].w = p | (sameBin == same && same <= 256u ? 0x80000000u : 0u);
+        }
+    }
+    d.skeysOut[to] = h;
+    d.perm1Out[to] = k;
+    d.physT[to] = p;
+    const f3 xs = predict_x(make3(x), make3(v), S);
+    d.X0[p] = x;
+    d.XsA[p] = make_float4(xs.x, xs.y, xs.z, x.w);
+    if (kCarry) {
+        d.Tdens[p] = d.dens[src];
+        d.Tlam[p] = d.lam[src];
+    }
+    if (kCarryDelta) d.TDP[p] = d.DP[src];
+    d.Tid[p] = id;
+    d.lidT[p] = to;
 }
 
 // Per bucket: where it starts in physical order and whether its particles occupy consecutive
@@ -732,8 +920,7 @@ __global__ __launch_bounds__(kWaveBuildBlock) void k_neighbours_wave(DeviceState
     extern __shared__ uint4 waveLds[];
     constexpr uint32_t kWaves = kWaveBuildBlock / 64;
     const uint32_t lane = __lane_id();
-    const uint32_t nb = gridDim.x, b = blockIdx.x;
-    const uint32_t block = (b % kXcds) * (nb / kXcds) + b / kXcds;
+    const uint32_t block = xcd_block(blockIdx.x, gridDim.x, kWaves * (uint32_t)S);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t base = (block * kWaves + wave) * (uint32_t)S;  // the wave's first slot
     if (base >= d.nslots) return;
@@ -1916,7 +2103,7 @@ constexpr int kGroupBlock = 256;
 
 template <int L>
 __device__ __forceinline__ LaneGroup<L> lane_group() {
-    const uint32_t T = xcd_slot<kGroupBlock>();
+    const uint32_t T = xcd_slot<kGroupBlock, L>();
     return {T / (uint32_t)L, T % (uint32_t)L, __lane_id() & ~(uint32_t)(L - 1)};
 }
 
@@ -2435,6 +2622,21 @@ void launch_order(hipStream_t st, const DeviceState& d, const SphParams& P, cons
         k_order_rank<true, false><<<count, kBlock, 0, st>>>(d, S);
     else
         k_order_rank<false, false><<<count, kBlock, 0, st>>>(d, S);
+}
+void launch_tally(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
+                  bool carryDelta) {
+    const uint32_t count = grid(d.nslots), prefix = d.tallyCount / kTallyBlock;
+    k_tally_count<<<count + grid(d.tableTotal) + 1u, kBlock, 0, st>>>(d, P, S, count);
+    k_tally_sum<<<prefix, kTallyThreads, 0, st>>>(d);
+    k_tally_prefix<<<prefix, kTallyThreads, 0, st>>>(d);
+    k_tally_place<<<count, kBlock, 0, st>>>(d);
+    const uint32_t rank = grid(d.nparticles);
+    if (carryDelta)
+        k_tally_rank<true, true><<<rank, kBlock, 0, st>>>(d, S, d.nparticles);
+    else if (carry)
+        k_tally_rank<true, false><<<rank, kBlock, 0, st>>>(d, S, d.nparticles);
+    else
+        k_tally_rank<false, false><<<rank, kBlock, 0, st>>>(d, S, d.nparticles);
 }
 void launch_bucket_phys(hipStream_t st, const DeviceState& d) {
     k_bucket_phys<<<grid(d.nslots), kBlock, 0, st>>>(d);

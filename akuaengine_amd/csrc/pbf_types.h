@@ -20,6 +20,14 @@ struct SceneDev {
     uint32_t modMagic;     // x % tableSize by multiply-high (fast_mod below)
     uint32_t modShift;
     uint32_t first;        // particles of the scenes before this one
+    // ordering by counting (launch_tally): the scene's groups of hashes and bins of cells, among all
+    uint32_t groupBegin, groupShift;
+    uint32_t binBegin;
+    uint32_t binBlock, binSpare;  // log2 of the cells' bins in a block, of the groups' bins behind it
+    int32_t binOrigin[3];      // cell coordinates of the range's lowest cell
+    uint32_t binCells[3];      // cells per axis, whole cubes of 2^cubeLog2
+    uint32_t cubeLog2;
+    uint32_t cubeStride[3];    // cubes from one cube to the next along each axis
     int32_t layoutOrigin[4];  // super-cell coordinates mapped to Morton coordinate 0
     float bmin[4];         // box (xyz) for the wall clamp and the velocity damping
     float bmax[4];

@@ -250,6 +250,10 @@ struct akua_solver {
     DevBuf<uint32_t> groupCount, groupBase;  // small scenes (launch_order); groupCount is zero between steps
     DevBuf<uint4> placed;
     uint32_t groups = 0;
+    // larger scenes (launch_tally): capacity and use of the counters (a multiple of kTallyBlock in use;
+    // 0: the boxes have too many cells), zero between steps
+    DevBuf<uint32_t> tally, tallyBase, tallyPart;
+    uint32_t tallyGroups = 0, tallyCount = 0;
     DevBuf<uint32_t> s1KA, s1VA, s1KB, s1VB, s2KA, s2VA, s2KB, s2VB, counts, totals, look, tickets;
     DevBuf<uint32_t> counts2, totals2, look2, tickets2;  // the layout sort's, beside the hash sort
     DevBuf<uint4> table;
@@ -348,6 +352,7 @@ struct akua_solver {
     DeviceState devState(bool keepLayout = false) {
         DeviceState d{};
         d.nslots = nslots;
+        d.nparticles = nparticles;
         d.scenes = dScenes.p;
         d.chunkScene = dChunkScene.p;
         d.X = X.p; d.V = V.p; d.dens = dens.p; d.lam = lam.p; d.id = id.p;
@@ -364,6 +369,11 @@ struct akua_solver {
         d.blockMasses = blockMasses.p; d.massesDiffer = massesDiffer.p;
         d.groupCount = groupCount.p; d.groupBase = groupBase.p; d.placed = placed.p;
         d.groups = groups;
+        d.tally = tally.p; d.tallyBase = tallyBase.p; d.tallyPart = tallyPart.p;
+        d.tallyGroups = tallyGroups; d.tallyCount = tallyCount;
+        // step scratch that nothing else uses before the sweeps
+        d.tallied = reinterpret_cast<uint4*>(XsC.p);
+        if (!groups) d.placed = reinterpret_cast<uint4*>(XsB.p);
         d.groupShift = (uint32_t)std::max(0, hashBits - (int)ceil_log2(groups));
         d.keysM = s2KA.p;
         d.perm2 = keepLayout ? perm2keep.p : (r2 ? s2VB.p : s2VA.p);
@@ -407,7 +417,7 @@ struct akua_solver {
         for (auto* b : {&dens, &lam, &Tdens, &Tlam, &size, &probeRho, &bndPsi, &net, &feat, &targ,
                         &lamHat, &adamM, &adamV, &part, &batchF, &batchT, &lossBuf})
             b->release();
-        for (auto* b : {&blockMasses, &massesDiffer, &id, &Tid, &lid, &phys, &lidT, &physT, &srcL, &bslot, &nbr, &cnt,
+        for (auto* b : {&tally, &tallyBase, &tallyPart, &blockMasses, &massesDiffer, &id, &Tid, &lid, &phys, &lidT, &physT, &srcL, &bslot, &nbr, &cnt,
                         &perm2keep, &s1KA, &s1VA, &s1KB, &s1VB, &s2KA, &s2VA, &s2KB, &s2VB, &counts,
                         &totals, &look, &tickets, &counts2, &totals2, &look2, &tickets2, &gate, &fallbacks, &work, &cntW, &nbrW, &qcost,
                         &queue, &qcount, &heads})
@@ -564,6 +574,24 @@ void setup(akua_solver* s, const std::vector<uint32_t>& counts) {
         s->groupBase.alloc(s->groups + 1);
         s->placed.alloc(ns);
         HIP_CHECK(hipMemset(s->groupCount.p, 0, s->groups * 4));
+    }
+    if (s->scenes.size() == 1 && s->nslots > kOrderMaxSlots) {
+        // groups of about four particles (cells hold more), and counters for four cells a slot
+        uint64_t g = 0;
+        for (SceneDev& sc : s->scenes) {
+            const uint32_t lg = std::max(6u, ceil_log2(((uint64_t)(sc.end - sc.begin) + 3u) / 4u));
+            sc.groupBegin = (uint32_t)g;
+            sc.groupShift = (uint32_t)std::max(0, (int)ceil_log2(sc.tableSize) - (int)lg);
+            g += 1ull << lg;
+        }
+        s->tallyGroups = (uint32_t)g;
+        const uint64_t room = (3ull * g + 4ull * ns + kTallyBlock - 1) / kTallyBlock * kTallyBlock;
+        if (room < (1ull << 31)) {
+            s->tally.alloc((size_t)room);
+            s->tallyBase.alloc((size_t)room);
+            s->tallyPart.alloc((size_t)(room / kTallyBlock));
+            HIP_CHECK(hipMemset(s->tally.p, 0, (size_t)room * 4));
+        }
     }
     s->table.alloc(s->tableTotal);
     s->bslot.alloc(ns);
@@ -722,7 +750,8 @@ uint32_t queue_passes(const akua_solver* s) { return 2u * (uint32_t)s->cfg.solve
 // 424 / 463 (uneven masses 547 / 516 / 505 / 538 / 574), 400,000 578 / 580 / 591 / 689 / 783.
 // In larger scenes the sweeps that wait for their gathers keep a few, those bound by arithmetic one;
 // us at 1M with 1 / 2 / 4 lanes: density and lambda 55 / 64 / 64, position delta 67 / 69 / 66, the
-// last one 83 / 78 / 83, vorticity 94 / 82 / 79, confinement 55 / 50 / 53, XSPH 92 / 75 / 72.
+// last one 83 / 78 / 83 (in 64 scenes of 2.6M 163 / 171), vorticity 94 / 82 / 79, confinement 55 / 50 / 53,
+// XSPH 92 / 75 / 72.
 struct SweepLanes {
     int jacobi, last, vorticity, confinement, xsph;
 };
@@ -731,13 +760,21 @@ SweepLanes sweep_lanes(const akua_solver* s) {
     if (s->tuning.laneGroup > 0) return all(s->tuning.laneGroup);
     if (s->nslots <= (1u << 15)) return all(16);
     if (s->nslots <= (1u << 18)) return all(4);
-    return SweepLanes{1, 2, 4, 2, 4};
+    return SweepLanes{1, s->scenes.size() == 1 ? 2 : 1, 4, 2, 4};
 }
 
 // Whether the step orders its particles by launch_order: a small single scene whose layout is left to
 // the solver, with the reference's search.
 bool small_order(const akua_solver* s) {
     return s->groups > 0 && s->sph.searchCells == 1 && layout_by_solver(s);
+}
+
+// Whether the step orders its particles by launch_tally: a larger single scene likewise, whose box has no
+// more than some four cells per particle.  Batches keep the sorts: their short scenes' bins and particles
+// far out cost more than the sorts' launches, which all scenes share (64 scenes of 2.6M, us per step: 2,449
+// with the sorts, 2,500 so).
+bool tally_order(const akua_solver* s) {
+    return s->tallyCount > 0 && s->sph.searchCells == 1 && layout_by_solver(s);
 }
 
 void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool timed,
@@ -750,6 +787,10 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
     if (small_order(s)) {
         L.before("order");
         launch_order(st, d, P, S, carry, carryDelta);
+        L.after("order");
+    } else if (tally_order(s)) {
+        L.before("order");
+        launch_tally(st, d, P, S, carry, carryDelta);
         L.after("order");
     } else {
         // single-cell super-cells: the layout keys are sorted in the previous logical order, which
@@ -914,6 +955,57 @@ SortPlan make_plan(int bits, int digitBits) {
 // the previous logical order it also splits their buckets (a key's cells then interleave).
 constexpr int kLayoutMarginCells = 4;
 
+// The scenes' bins of launch_tally: the cells of the box and kLayoutMarginCells beyond each wall, in cubes
+// of 16^3 cells (32,000 particles, whose data an XCD's cache holds; 8^3 in thin boxes), the longest axis slowest.
+void update_bins(akua_solver* s) {
+    uint64_t bins = 0;
+    for (SceneDev& sc : s->scenes) {
+        uint64_t cells[3];
+        int axis[3] = {0, 1, 2};
+        for (int a = 0; a < 3; ++a) {
+            const double lo = std::floor((double)sc.bmin[a] / s->sph.cellHash) - (double)kLayoutMarginCells;
+            const double hi = std::floor((double)sc.bmax[a] / s->sph.cellHash) + (double)kLayoutMarginCells;
+            sc.binOrigin[a] = (int32_t)std::min(std::max(lo, -1e9), 1e9);
+            cells[a] = (uint64_t)std::min(std::max(hi - lo + 1.0, 1.0), 1e9);
+        }
+        sc.cubeLog2 = std::min({cells[0], cells[1], cells[2]}) < 32 ? 3u : 4u;
+        std::sort(axis, axis + 3, [&](int a, int b) { return cells[a] < cells[b]; });
+        double cubes = 1.0;  // at most 2^90: compared as a double
+        uint64_t stride = 1;
+        for (int a : axis) {
+            const uint64_t c = (cells[a] + (1u << sc.cubeLog2) - 1u) >> sc.cubeLog2;
+            sc.binCells[a] = (uint32_t)(c << sc.cubeLog2);
+            sc.cubeStride[a] = (uint32_t)stride;
+            cubes *= (double)c;
+            stride *= c;
+            if (cubes > 1e9) stride = 0;
+        }
+        sc.binBegin = (uint32_t)bins;
+        // some 64 blocks of cells' bins, each with its share of the groups' bins behind it
+        const double b = cubes * (double)(1u << (3u * sc.cubeLog2));
+        if (b > 2e9) {
+            bins = UINT64_MAX;
+            break;
+        }
+        sc.binBlock = std::max(12u, ceil_log2(((uint64_t)b + 63u) / 64u));
+        const uint64_t blocks = (((uint64_t)b - 1u) >> sc.binBlock) + 1u;
+        const uint32_t groups = 1u << std::max(6u, ceil_log2(((uint64_t)(sc.end - sc.begin) + 3u) / 4u));
+        sc.binSpare = ceil_log2((groups + blocks - 1) / blocks);
+        bins += blocks * ((1ull << sc.binBlock) + (1ull << sc.binSpare));
+        if (bins > s->tally.n) {
+            bins = UINT64_MAX;
+            break;
+        }
+    }
+    uint32_t count = 0;
+    if (bins != UINT64_MAX) {
+        const uint64_t c = ((uint64_t)s->tallyGroups + bins + 1u + kTallyBlock - 1u) / kTallyBlock * kTallyBlock;
+        if (c <= s->tally.n) count = (uint32_t)c;
+    }
+    if (count != s->tallyCount) s->graphDirty = true;
+    s->tallyCount = count;
+}
+
 void update_layout(akua_solver* s) {
     int bits = 1;
     const int L = layout_level(s);
@@ -937,6 +1029,7 @@ void update_layout(akua_solver* s) {
         sc.layoutOrigin[3] = L;
     }
     for (SceneDev& sc : s->scenes) sc.layoutBits = (uint32_t)bits;
+    update_bins(s);
     s->plan1 = make_plan(s->plan1.bits, s->tuning.hashDigitBits);
     // single-cell super-cells with the layout digit width left to the solver: the hash sort's
     // width, so that the two sorts share their launches

@@ -1,4 +1,5 @@
-"""Ordering of small scenes by counting (one group of hash bits at a time) against the FP32 oracle: the
+"""Ordering of single scenes by counting (groups of hash bits, and bins of cells above 32,768 particles)
+against the FP32 oracle: the
 sorted hashes, the permutation, the buckets' ranges and the lists, over several steps, at the edges of
 waves, workgroups, group counts and of the largest such scene, with crowded and shared buckets, and
 where the layout setting changes between steps."""
@@ -77,3 +78,35 @@ def test_setting_changes_between_steps(gpu, oracle_mod, dam_params):
 
     s_default = gpu(1, cfg, corr).get_tuning()["layoutLevel"]
     _check(gpu, oracle_mod, cfg, corr, sc.pos, sc.box_min, sc.box_max, 7, between)
+
+
+@pytest.mark.parametrize("over", [dict(), dict(maxNeighbours=1), dict(maxNeighbours=2), dict(solverIterations=0)])
+def test_larger_scene_far_out_and_shared(gpu, oracle_mod, dam_params, over):
+    """Above 32,768 particles: a tenth of them far outside the box (bins per group), 900 in one cell,
+    tables of one and two entries per particle (cells of one bucket in several bins), no iterations, a box
+    that grows until its cells have no bins and shrinks again."""
+    cfg, corr = dam_params
+    rng = np.random.default_rng(8)
+    pos = np.concatenate([1.0 + rng.uniform(0.0, 0.099, (900, 3)), rng.uniform(-30.0, 40.0, (4000, 3)),
+                          rng.uniform(0.0, 4.0, (36000, 3))])
+    pos = rng.permutation(pos).astype(np.float32)
+    vel = rng.uniform(-0.5, 0.5, pos.shape).astype(np.float32)
+    cfg = dataclasses.replace(cfg, **over)
+    s = gpu(len(pos), cfg, corr)
+    o = oracle_mod.Oracle(len(pos), cfg, corr, 32)
+    s.set_state(pos, vel)
+    o.set_state(pos, vel)
+    for step, hi in enumerate((4.0, 4.0, 60.0, 5.0)):
+        print(f"[larger order] {over}, step {step}", flush=True)
+        s.step(DT, (0.0, 0.0, 0.0), (hi, 4.0, hi))
+        o.step(DT, (0.0, 0.0, 0.0), (hi, 4.0, hi))
+        t = o.taps()
+        np.testing.assert_array_equal(s.debug_hashes(), t["sorted_hash"])
+        np.testing.assert_array_equal(s.debug_permutation(), t["perm"])
+        assert np.array_equal(np.sort(s.debug_physical_order()), np.arange(len(pos)))
+        nbr, cnt = s.debug_neighbours()
+        np.testing.assert_array_equal(cnt, t["cnt"])
+        np.testing.assert_array_equal(nbr, t["nbr"])
+    g, r = s.get_state(), o.state()
+    for k in ("pos", "vel", "density", "lam", "ids"):
+        np.testing.assert_array_equal(g[k], r[k].astype(g[k].dtype), err_msg=k)
