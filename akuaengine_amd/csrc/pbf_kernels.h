@@ -186,6 +186,9 @@ void launch_count_sum(hipStream_t st, const DeviceState& d, unsigned long long* 
 // lanes (4, 8 or 16; 1: one thread per particle): a lane group per particle in the neighbour
 // sweeps, for scenes too small to fill the chip, with results identical to one lane per particle;
 // only for plain steps (residSlot -1, no gate), the physical order and no wall samples.
+// lanes of a sweep: one per particle, or one that shares the long lists of its wave (plain steps in the
+// physical order without wall samples), or a group of 2 to 16.
+constexpr int kLanesShared = 0;
 void launch_density_lambda(hipStream_t st, const DeviceState& d, const SphParams& P,
                            const float4* Xs, int bs, int residSlot = -1, bool gated = false,
                            int lanes = 1);

@@ -1936,6 +1936,182 @@ __global__ __launch_bounds__(BS) void k_xsph(DeviceState d, SphParams P) {
     xsph_slot(d, P, xcd_slot<BS>());
 }
 
+// ---- long lists shared by their wave -------------------------------------------------------------
+// In a sprayed scene the lists of a wave differ: 16 entries on average, 54 the longest (1M dam break after
+// 100 steps), and with one lane per list most lanes wait for a few.  Here each lane walks its list up to a
+// little over the wave's average; the chunks of four entries that are left are dealt to all lanes, which
+// compute their terms, and each list's own lane adds them from LDS in list order (a chunk's addition is
+// some seven instructions against sixty per entry's terms).  The same terms in the same order: the same
+// sums, with +0 in the place of entries past a list's end.
+// Where no list is more than kTailMin entries over the average (settled scenes), nothing is dealt.
+// Measured against one lane per list (the last delta: two): 50 steps of the 1M dam break 68 -> 61 us, the
+// last 77 -> 75, a settled 1M 56 -> 55 and 82 -> 70, 64 scenes of 2.6M 136 -> 127 and 163 -> 158.  The density
+// sweep, with five sums to pass through LDS and more waves per SIMD without them, gains nothing (55.9 us with
+// one lane, 57.5 so) and keeps one lane.
+constexpr uint32_t kTailMin = 8;
+
+// The largest value of the wave's 64 lanes.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+    for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off, 64));
+    return v;
+}
+// The largest value of this lane and those below it.
+__device__ __forceinline__ uint32_t wave_prefix_max(uint32_t v) {
+    int x = (int)v;
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false));  // row_shr:1
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false));  // row_shr:2
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false));  // row_shr:4
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false));  // row_shr:8
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));  // row_bcast:15 into rows 1 and 3
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)x;
+}
+
+// LDS of a wave: NA rows of 64 chunks' terms, and the lists' lanes by chunk.
+template <int NA>
+struct TailLds {
+    float4 terms[NA][64];
+    uint32_t owner[64];
+};
+
+// wave: chunk 0 of the list of the wave's lane 0; n: this lane's entries (0 without a particle);
+// own: what the terms need of the particle, as floats.  Every lane of the wave takes part.
+template <int NA, class T, int NO, class Load, class Term>
+__device__ __forceinline__ void walk_shared(const uint4* __restrict__ wave, uint32_t n, const float (&own)[NO],
+                                            Load load, Term term, float (&acc)[NA], TailLds<NA>& lds) {
+    const uint32_t lane = __lane_id();
+    const uint32_t longest = wave_max(n), mean = lane_u(wave_prefix(n), 63u) >> 6;
+    uint32_t until = (mean + mean / 8u + 3u) & ~3u;
+    if (longest <= until + kTailMin) until = longest;
+    const auto one = [&](const float (&o)[NO], const T& v, float (&t)[NA]) { term(o, v, t); };
+    walk_list<T>(wave + lane, min(n, until), load, [&](const T& v) {
+        float t[NA];
+        one(own, v, t);
+#pragma unroll
+        for (int c = 0; c < NA; ++c) acc[c] = acc[c] + t[c];
+    });
+    if (until == longest) return;
+    const uint32_t chunks = n > until ? (n - until + 3u) >> 2 : 0u;
+    const uint32_t end = wave_prefix(chunks), begin = end - chunks;
+    const uint32_t total = lane_u(end, 63u);
+    for (uint32_t q0 = 0; q0 < total; q0 += 64u) {
+        // whose chunk is q0 + lane: the last list that begins at or before it
+        wave_lds_order();
+        lds.owner[lane] = 0u;
+        wave_lds_order();
+        if (chunks != 0u && begin < q0 + 64u && end > q0) lds.owner[begin > q0 ? begin - q0 : 0u] = lane;
+        wave_lds_order();
+        const int who = (int)wave_prefix_max(lds.owner[lane]);
+        float o[NO];
+#pragma unroll
+        for (int k = 0; k < NO; ++k) o[k] = __shfl(own[k], who, 64);
+        const uint32_t first = (uint32_t)__shfl((int)begin, who, 64), entries = (uint32_t)__shfl((int)n, who, 64);
+        const bool in = q0 + lane < total;
+        const uint32_t k = in ? until + 4u * (q0 + lane - first) : 0u;  // the chunk's first entry; 0: some list's
+        float t[4][NA] = {};
+        if (in) {
+            const uint4 ch = wave[(size_t)(k >> 2) * 64u + (uint32_t)who];
+            const uint32_t e[4] = {ch.x, ch.y, ch.z, ch.w};
+            T v[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) v[u] = load(k + u < entries ? e[u] : e[0]);
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                float r[NA];
+                one(o, v[u], r);
+#pragma unroll
+                for (int c = 0; c < NA; ++c) t[u][c] = k + u < entries ? r[c] : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NA; ++c) lds.terms[c][lane] = make_float4(t[0][c], t[1][c], t[2][c], t[3][c]);
+        wave_lds_order();
+        const uint32_t from = max(begin, q0), to = min(end, q0 + 64u);
+        for (uint32_t q = from; q < to; ++q) {
+#pragma unroll
+            for (int c = 0; c < NA; ++c) {
+                const float4 x = lds.terms[c][q - q0];
+                acc[c] = (((acc[c] + x.x) + x.y) + x.z) + x.w;
+            }
+        }
+    }
+}
+
+constexpr int kTailBlock = 256;
+
+// The position delta and correction of a plain step (no work order, gate or wall samples).
+template <bool kFinal, bool kFast>
+__device__ __forceinline__ void delta_correct_tail(const DeviceState& d, const SphParams& P, const StepParams& S,
+                                                   const float4* __restrict__ XsIn, float4* __restrict__ XsOut,
+                                                   TailLds<3>* lds) {
+    const uint32_t i = xcd_slot<kTailBlock>(), i0 = i & ~63u;
+    if (i0 >= d.nslots) return;
+    const SceneDev& sc = scene_of(d, i0);
+    const bool valid = i < d.nslots && i < sc.end;
+    const float4 xi4 = valid ? XsIn[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const f3 xi = make3(xi4);
+    const float own[4] = {xi.x, xi.y, xi.z, valid ? d.lam[i] : 0.0f};
+    const Recip Rdq = recip(P.wdq);
+    float acc[3] = {0.0f, 0.0f, 0.0f};
+    const auto walk = [&](auto corrOn) {
+        constexpr bool kCorr = decltype(corrOn)::value;
+        walk_shared<3, XLam>(
+            d.nbr4 + list_base(i0, P.maxN), valid ? d.cnt[i] : 0u, own,
+            [&](uint32_t j) {
+                if (kFast) {
+                    const float4 a = ld(d.W, j);
+                    return XLam{a, a.w};
+                }
+                return XLam{ld(XsIn, j), ld(d.lam, j)};
+            },
+            [&](const float (&o)[4], const XLam& nb, float (&t)[3]) {
+                const f3 sep = f3{o[0], o[1], o[2]} - make3(nb.x);
+                const float d2 = dot3(sep, sep);
+                float coef = o[3] + nb.lam;
+                f3 g{0.0f, 0.0f, 0.0f};
+                if constexpr (kFast) {
+                    // the quotient of s_corr and the gradient's, with one test for the rare cases of all
+                    const float w = kCorr ? poly6_bounded(d2, P) : 1.0f;
+                    float q = kCorr ? div_by(w, Rdq.b, Rdq.r) : 0.0f;
+                    GradTerm G;
+                    const bool some = grad_term(sep, d2, P, G);
+                    if (__builtin_expect(some && (fminf(G.low, w) < kDivLowest || G.inexact), 0)) {
+                        if (kCorr) q = corr_by_division(w, q, Rdq);
+                        grad_by_division(G);
+                    }
+                    if (kCorr) coef = coef + P.negCorrK * corr_pow(q, P);
+                    if (some) g = G.g;
+                } else {
+                    if (kCorr) coef = coef + P.negCorrK * corr_pow(div_rn(poly6(d2, P), Rdq), P);
+                    grad_spiky_nonzero(sep, P, g);
+                }
+                const f3 u = (kFast ? coef : coef * nb.x.w) * g;  // m_j == 1 under kFast
+                t[0] = u.x; t[1] = u.y; t[2] = u.z;
+            },
+            acc, lds[threadIdx.x >> 6]);
+    };
+    if (P.corrOn)
+        walk(std::true_type{});
+    else
+        walk(std::false_type{});
+    if (!valid) return;
+    f3 dp{acc[0], acc[1], acc[2]};
+    const f3 q = correct_position(xi, dp, P, sc);
+    if (!kFinal) {
+        XsOut[i] = make_float4(q.x, q.y, q.z, xi4.w);
+        return;
+    }
+    finish_step<true>(d, S, sc, i, xi4, finish_in(d, i), q, dp);
+}
+
+template <bool kFinal, int kFast>
+__global__ __launch_bounds__(kTailBlock) void k_delta_correct_tail(DeviceState d, SphParams P, StepParams S,
+                                                                   const float4* __restrict__ XsIn,
+                                                                   float4* __restrict__ XsOut) {
+    __shared__ TailLds<3> lds[kTailBlock / 64];
+    by_masses<kFast>(d, [&](auto fast) { delta_correct_tail<kFinal, decltype(fast)::value>(d, P, S, XsIn, XsOut, lds); });
+}
+
 // ---- work queue: the sweeps as persistent kernels over 256-slot tiles, heaviest first -------
 // A batch of uneven scenes (and the uneven lists of one scene) leave each sweep's last waves
 // running on a few CUs.  With the work queue, the tiles of each XCD's contiguous range (the range
@@ -2761,6 +2937,14 @@ void launch_delta_correct(hipStream_t st, const DeviceState& d, const SphParams&
             if (final) AKUA_DCG(true, false); else AKUA_DCG(false, false);
         }
 #undef AKUA_DCG
+        return;
+    }
+    if (lanes == kLanesShared && applyDelta) {
+        const unsigned g = grid_xcd(d.nslots, kTailBlock);
+        if (final)
+            AKUA_BY_FAST((k_delta_correct_tail<true, K><<<g, kTailBlock, 0, st>>>(d, P, S, XsIn, XsOut)));
+        else
+            AKUA_BY_FAST((k_delta_correct_tail<false, K><<<g, kTailBlock, 0, st>>>(d, P, S, XsIn, XsOut)));
         return;
     }
     AKUA_BY_BLOCK(bs, (delta_correct_bs<BS>(st, d, P, S, XsIn, XsOut, final, applyDelta, gate,

@@ -748,19 +748,20 @@ uint32_t queue_passes(const akua_solver* s) { return 2u * (uint32_t)s->cfg.solve
 // 8 / 16 lanes: 4,000 particles 198 / 153 / 125 / 112 / 103, 27,000 203 / 163 / 138 / 142 / 138 (with
 // wall samples 297 / 265 / 201 / 189 / 172), 60,000 223 / 190 / 183 / 197 / 199, 200,000 385 / 378 / 381 /
 // 424 / 463 (uneven masses 547 / 516 / 505 / 538 / 574), 400,000 578 / 580 / 591 / 689 / 783.
-// In larger scenes the sweeps that wait for their gathers keep a few, those bound by arithmetic one;
+// In larger scenes the sweeps that wait for their gathers keep a few, the density sweep, bound by
+// arithmetic, one, and the position deltas one that shares the long lists of its wave (walk_shared);
 // us at 1M with 1 / 2 / 4 lanes: density and lambda 55 / 64 / 64, position delta 67 / 69 / 66, the
 // last one 83 / 78 / 83 (in 64 scenes of 2.6M 163 / 171), vorticity 94 / 82 / 79, confinement 55 / 50 / 53,
 // XSPH 92 / 75 / 72.
 struct SweepLanes {
-    int jacobi, last, vorticity, confinement, xsph;
+    int density, delta, last, vorticity, confinement, xsph;
 };
 SweepLanes sweep_lanes(const akua_solver* s) {
-    const auto all = [](int n) { return SweepLanes{n, n, n, n, n}; };
+    const auto all = [](int n) { return SweepLanes{n, n, n, n, n, n}; };
     if (s->tuning.laneGroup > 0) return all(s->tuning.laneGroup);
     if (s->nslots <= (1u << 15)) return all(16);
     if (s->nslots <= (1u << 18)) return all(4);
-    return SweepLanes{1, s->scenes.size() == 1 ? 2 : 1, 4, 2, 4};
+    return SweepLanes{1, kLanesShared, kLanesShared, 4, 2, 4};
 }
 
 // Whether the step orders its particles by launch_order: a small single scene whose layout is left to
@@ -827,12 +828,16 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
     // small scenes: lane groups in the sweeps of a plain step, and in those after the position update
     // of every step
     const bool plainOrder = !d.work && P.searchCells == 1;
-    SweepLanes lanes = plainOrder ? sweep_lanes(s) : SweepLanes{1, 1, 1, 1, 1};
+    SweepLanes lanes = plainOrder ? sweep_lanes(s) : SweepLanes{1, 1, 1, 1, 1, 1};
     // with the work queue too, the queue runs the Jacobi sweeps and confinement, and the lane groups run vorticity and XSPH (two gathered records per neighbour, whose latency
     // more lanes per particle hide better)
     const bool queueSet = s->tuning.workQueue > 0 && !learned && !record && s->queue.p &&
                           s->heads.n >= queue_heads_size(queue_passes(s));
-    if (queueSet || learned || record) lanes.jacobi = lanes.last = 1;
+    if (queueSet || learned || record) lanes.density = lanes.delta = lanes.last = 1;
+    if (P.bd.on) {  // the shared form has no wall samples
+        lanes.delta = std::max(1, lanes.delta);
+        lanes.last = std::max(1, lanes.last);
+    }
     // the sweeps of a plain step as persistent launches over each XCD's queue of tiles
     const bool queued = queueSet;
     uint32_t pass = 0;
@@ -894,7 +899,7 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
         if (queued)
             launch_density_lambda_queue(st, d, P, in, pass++);
         else
-            launch_density_lambda(st, d, P, in, bs, record && it == I - Jt ? 2 : -1, learned, lanes.jacobi);
+            launch_density_lambda(st, d, P, in, bs, record && it == I - Jt ? 2 : -1, learned, lanes.density);
         L.after(learned ? "density_lambda_fallback" : "density_lambda");
         if (record && it == I - Jt) {
             L.before("targets");
@@ -910,7 +915,7 @@ void enqueue_step(akua_solver* s, hipStream_t st, const StepParams& S, bool time
             launch_delta_correct_queue(st, d, P, S, in, out, last, pass++);
         else
             launch_delta_correct(st, d, P, S, in, out, last, true, bs, learned ? (last ? 2 : 1) : 0,
-                                 learned ? ws(J - 1) : nullptr, last ? lanes.last : lanes.jacobi);
+                                 learned ? ws(J - 1) : nullptr, last ? lanes.last : lanes.delta);
         L.after(name);
     }
     L.before("vorticity");

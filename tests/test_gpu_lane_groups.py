@@ -62,3 +62,23 @@ def test_default_group_by_size(gpu, oracle_mod, dam_params, n):
     sc = scenes.batched_scene(n, index=n % 5)
     print(f"[lane groups] n={n}", flush=True)
     _check(gpu, oracle_mod, cfg, corr, sc.pos, None, sc.box_min, sc.box_max, 0, 0, 2)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("cap", [30, 64, 91])
+def test_uneven_lists_in_large_scenes(gpu, oracle_mod, dam_params, cap, mixed):
+    """Above 262,144 particles a wave shares its long lists: dense blobs (about 95 neighbours) between
+    sparse particles in the same waves, lists of 0 to the cap, a last wave that is not full."""
+    from akuaengine_amd import scenes
+    cfg, corr = dam_params
+    cfg = dataclasses.replace(cfg, maxNeighbours=cap)
+    rng = np.random.default_rng(cap)
+    blob = scenes.lattice(7, 7, 7, 0.035, (0.0, 0.0, 0.0))
+    at = rng.uniform(0.5, 7.5, (300, 1, 3))
+    pos = np.concatenate([(blob[None] + at).reshape(-1, 3), rng.uniform(0.05, 7.95, (160001, 3))])
+    pos = (pos + rng.uniform(-0.004, 0.004, pos.shape)).astype(np.float32)
+    assert len(pos) > 1 << 18 and len(pos) % 64
+    mass = rng.uniform(0.5, 1.5, len(pos)).astype(np.float32) if mixed else None
+    print(f"[lane groups] uneven lists, cap {cap}, masses {mixed}", flush=True)
+    longest = _check(gpu, oracle_mod, cfg, corr, pos, mass, (0.0, 0.0, 0.0), (8.0, 8.0, 8.0), 0, 0, 2)
+    assert longest == cap
