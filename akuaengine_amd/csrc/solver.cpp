@@ -247,13 +247,17 @@ struct akua_solver {
     DevBuf<float> dens, lam, Tdens, Tlam, size;
     DevBuf<uint32_t> id, Tid, lid, phys, lidT, physT, srcL, bslot, nbr, cnt, perm2keep;
     DevBuf<uint2> layPhys;
-    DevBuf<uint32_t> groupCount, groupBase;  // small scenes (launch_order); groupCount is zero between steps
-    DevBuf<uint4> placed;
-    uint32_t groups = 0;
+    // Single scenes, in one allocation: the record masses' words (massesDiffer, then blockMasses), and the
+    // counters of launch_order (groupCount, groupBase) or launch_tally (tally, tallyBase, tallyPart), of
+    // which groupCount and tally are zero between steps.
+    DevBuf<uint32_t> counters;
+    uint32_t *massesDiffer = nullptr, *blockMasses = nullptr;
+    uint32_t *groupCount = nullptr, *groupBase = nullptr;
+    uint32_t groups = 0;       // small scenes
     // larger scenes (launch_tally): capacity and use of the counters (a multiple of kTallyBlock in use;
     // 0: the boxes have too many cells), zero between steps
-    DevBuf<uint32_t> tally, tallyBase, tallyPart;
-    uint32_t tallyGroups = 0, tallyCount = 0;
+    uint32_t *tally = nullptr, *tallyBase = nullptr, *tallyPart = nullptr;
+    uint32_t tallyRoom = 0, tallyGroups = 0, tallyCount = 0;
     DevBuf<uint32_t> s1KA, s1VA, s1KB, s1VB, s2KA, s2VA, s2KB, s2VB, counts, totals, look, tickets;
     DevBuf<uint32_t> counts2, totals2, look2, tickets2;  // the layout sort's, beside the hash sort
     DevBuf<uint4> table;
@@ -269,7 +273,6 @@ struct akua_solver {
     bool exact = true;             // the autotuner keeps the reference's search (akua_solver_set_exact)
     bool unitMass = false;         // every particle's mass is exactly 1 (known from the upload)
     bool deviceMasses = false;     // the masses came from device memory (akua_solver_step_device)
-    DevBuf<uint32_t> blockMasses, massesDiffer;  // what the device found in them
     bool boundedQuotients = false; // quotients_bounded(sph)
 
     // learned warm start
@@ -366,14 +369,14 @@ struct akua_solver {
         d.keysL = s1KA.p;
         d.skeys = d.skeysOut = r1 ? s1KB.p : s1KA.p;
         d.perm1 = d.perm1Out = r1 ? s1VB.p : s1VA.p;
-        d.blockMasses = blockMasses.p; d.massesDiffer = massesDiffer.p;
-        d.groupCount = groupCount.p; d.groupBase = groupBase.p; d.placed = placed.p;
+        d.blockMasses = blockMasses; d.massesDiffer = massesDiffer;
+        d.groupCount = groupCount; d.groupBase = groupBase;
         d.groups = groups;
-        d.tally = tally.p; d.tallyBase = tallyBase.p; d.tallyPart = tallyPart.p;
+        d.tally = tally; d.tallyBase = tallyBase; d.tallyPart = tallyPart;
         d.tallyGroups = tallyGroups; d.tallyCount = tallyCount;
         // step scratch that nothing else uses before the sweeps
         d.tallied = reinterpret_cast<uint4*>(XsC.p);
-        if (!groups) d.placed = reinterpret_cast<uint4*>(XsB.p);
+        d.placed = reinterpret_cast<uint4*>(XsB.p);
         d.groupShift = (uint32_t)std::max(0, hashBits - (int)ceil_log2(groups));
         d.keysM = s2KA.p;
         d.perm2 = keepLayout ? perm2keep.p : (r2 ? s2VB.p : s2VA.p);
@@ -417,12 +420,12 @@ struct akua_solver {
         for (auto* b : {&dens, &lam, &Tdens, &Tlam, &size, &probeRho, &bndPsi, &net, &feat, &targ,
                         &lamHat, &adamM, &adamV, &part, &batchF, &batchT, &lossBuf})
             b->release();
-        for (auto* b : {&tally, &tallyBase, &tallyPart, &blockMasses, &massesDiffer, &id, &Tid, &lid, &phys, &lidT, &physT, &srcL, &bslot, &nbr, &cnt,
+        for (auto* b : {&counters, &id, &Tid, &lid, &phys, &lidT, &physT, &srcL, &bslot, &nbr, &cnt,
                         &perm2keep, &s1KA, &s1VA, &s1KB, &s1VB, &s2KA, &s2VA, &s2KB, &s2VB, &counts,
                         &totals, &look, &tickets, &counts2, &totals2, &look2, &tickets2, &gate, &fallbacks, &work, &cntW, &nbrW, &qcost,
                         &queue, &qcount, &heads})
             b->release();
-        layPhys.release(); groupCount.release(); groupBase.release(); placed.release(); table.release(); dTiles.release(); dSortScenes.release(); nbrSum.release();
+        layPhys.release(); table.release(); dTiles.release(); dSortScenes.release(); nbrSum.release();
         probeMax.release(); probeSum.release(); renderKeys.release(); renderRgb.release();
         resid.release(); residPart.release(); residBlk.release(); aosStage.release();
     }
@@ -563,34 +566,38 @@ void setup(akua_solver* s, const std::vector<uint32_t>& counts) {
         for (auto* l : {&s->look, &s->look2}) l->alloc((size_t)2 * s->numTiles * (1u << kMaxDigitBits));
         for (auto* t : {&s->tickets, &s->tickets2}) t->alloc((size_t)kMaxPasses);
     }
-    if (s->scenes.size() == 1) {  // record stepping is per single-scene solver
-        s->massesDiffer.alloc(1);
-        s->blockMasses.alloc((ns + 255) / 256);
-    }
-    if (s->scenes.size() == 1 && s->nslots <= kOrderMaxSlots) {
-        // about four particles a group: cells hold more, so that most groups are one cell
-        s->groups = std::min(kOrderMaxGroups, std::max(256u, 1u << ceil_log2((s->nslots + 3u) / 4u)));
-        s->groupCount.alloc(s->groups);
-        s->groupBase.alloc(s->groups + 1);
-        s->placed.alloc(ns);
-        HIP_CHECK(hipMemset(s->groupCount.p, 0, s->groups * 4));
-    }
-    if (s->scenes.size() == 1 && s->nslots > kOrderMaxSlots) {
-        // groups of about four particles (cells hold more), and counters for four cells a slot
-        uint64_t g = 0;
-        for (SceneDev& sc : s->scenes) {
-            const uint32_t lg = std::max(6u, ceil_log2(((uint64_t)(sc.end - sc.begin) + 3u) / 4u));
-            sc.groupBegin = (uint32_t)g;
+    if (s->scenes.size() == 1) {
+        const size_t masses = (1 + (ns + 255) / 256 + 3) / 4 * 4;  // the counters are read four at a time
+        size_t words = masses;
+        if (s->nslots <= kOrderMaxSlots) {
+            // about four particles a group: cells hold more, so that most groups are one cell
+            s->groups = std::min(kOrderMaxGroups, std::max(256u, 1u << ceil_log2((s->nslots + 3u) / 4u)));
+            words += 2 * (size_t)s->groups + 1;
+        } else {
+            // groups likewise, and counters for four cells a slot
+            SceneDev& sc = s->scenes[0];
+            const uint32_t lg = std::max(6u, ceil_log2(((uint64_t)ns + 3u) / 4u));
+            sc.groupBegin = 0;
             sc.groupShift = (uint32_t)std::max(0, (int)ceil_log2(sc.tableSize) - (int)lg);
-            g += 1ull << lg;
+            s->tallyGroups = 1u << lg;
+            const uint64_t room = (3ull * s->tallyGroups + 4ull * ns + kTallyBlock - 1) / kTallyBlock * kTallyBlock;
+            if (room < (1ull << 31)) {
+                s->tallyRoom = (uint32_t)room;
+                words += 2 * (size_t)room + room / kTallyBlock;
+            }
         }
-        s->tallyGroups = (uint32_t)g;
-        const uint64_t room = (3ull * g + 4ull * ns + kTallyBlock - 1) / kTallyBlock * kTallyBlock;
-        if (room < (1ull << 31)) {
-            s->tally.alloc((size_t)room);
-            s->tallyBase.alloc((size_t)room);
-            s->tallyPart.alloc((size_t)(room / kTallyBlock));
-            HIP_CHECK(hipMemset(s->tally.p, 0, (size_t)room * 4));
+        s->counters.alloc(words);
+        HIP_CHECK(hipMemset(s->counters.p, 0, words * 4));
+        s->massesDiffer = s->counters.p;
+        s->blockMasses = s->counters.p + 1;
+        uint32_t* const c = s->counters.p + masses;
+        if (s->groups) {
+            s->groupCount = c;
+            s->groupBase = c + s->groups;
+        } else if (s->tallyRoom) {
+            s->tally = c;
+            s->tallyBase = c + s->tallyRoom;
+            s->tallyPart = s->tallyBase + s->tallyRoom;
         }
     }
     s->table.alloc(s->tableTotal);
@@ -997,7 +1004,7 @@ void update_bins(akua_solver* s) {
         const uint32_t groups = 1u << std::max(6u, ceil_log2(((uint64_t)(sc.end - sc.begin) + 3u) / 4u));
         sc.binSpare = ceil_log2((groups + blocks - 1) / blocks);
         bins += blocks * ((1ull << sc.binBlock) + (1ull << sc.binSpare));
-        if (bins > s->tally.n) {
+        if (bins > s->tallyRoom) {
             bins = UINT64_MAX;
             break;
         }
@@ -1005,7 +1012,7 @@ void update_bins(akua_solver* s) {
     uint32_t count = 0;
     if (bins != UINT64_MAX) {
         const uint64_t c = ((uint64_t)s->tallyGroups + bins + 1u + kTallyBlock - 1u) / kTallyBlock * kTallyBlock;
-        if (c <= s->tally.n) count = (uint32_t)c;
+        if (c <= s->tallyRoom) count = (uint32_t)c;
     }
     if (count != s->tallyCount) s->graphDirty = true;
     s->tallyCount = count;
@@ -2152,7 +2159,7 @@ akua_status akua_solver_step_device(akua_solver* s, void* dParticles, int32_t n,
         auto* buf = static_cast<AosParticle*>(dParticles);
         const auto step = [&](hipStream_t st, const hipStream_t* caller) {
             launch_import_aos(st, buf, (uint32_t)n, s->X.p, s->V.p, s->VS.p, s->DP.p, s->dens.p,
-                              s->lam.p, s->id.p, s->lid.p, s->phys.p, s->color.p, s->size.p, s->blockMasses.p);
+                              s->lam.p, s->id.p, s->lid.p, s->phys.p, s->color.p, s->size.p, s->blockMasses);
             s->hasState = true;
             s->layoutPhase = 0;
             s->unitMass = false;  // the masses came from device memory: the kernels look at them
