@@ -67,6 +67,7 @@ BYTES = {
     "confinement": lambda nb: 56 + 4 * nb,
     "xsph": lambda nb: 44 + 4 * nb,
     "predict_hash": lambda nb: 44,
+    "order": lambda nb: 116,  # predict/hash and move together (launch_order, launch_tally)
     "gather": lambda nb: 72,
     "rs_hist": lambda nb: 4,
     "rs_scan": lambda nb: 0,
