@@ -252,8 +252,9 @@ void launch_render(hipStream_t st, const float4* X, const float4* color, const f
     const uint32_t pixels = (uint32_t)(R.width * R.height);
     k_render_clear<<<(std::max(pixels, n) + 255) / 256, 256, 0, st>>>(zbuf, pixels, lid, phys, n);
     if (n) {
-        // n * kSplatLanes stays below 2^32: slots number at most 2^28
-        k_render_splat<<<(n * kSplatLanes + 255) / 256, 256, 0, st>>>(X, size, id, lid, n, R, zbuf);
+        // at most 2^28 slots: the lanes number at most 2^32, the last of them 2^32 - 1
+        const uint32_t blocks = (uint32_t)(((uint64_t)n * kSplatLanes + 255u) / 256u);
+        k_render_splat<<<blocks, 256, 0, st>>>(X, size, id, lid, n, R, zbuf);
     }
     k_render_resolve<<<(pixels + 255) / 256, 256, 0, st>>>(X, color, size, id, phys, R, zbuf, rgb);
 }
