@@ -322,7 +322,6 @@ struct akua_solver {
     // stream (joined()) waits for before its next work, and whether that stream has had work since
     // step_device last waited for it (events created on first use)
     hipEvent_t callerEvent = nullptr, orderEvent = nullptr;
-    hipStream_t callerStream = nullptr;
     bool callerPending = false, ownPending = false;
 
     // The solver's own stream, behind the steps on the caller's.
@@ -331,7 +330,6 @@ struct akua_solver {
             const hipError_t e = hipStreamWaitEvent(stream, callerEvent, 0);
             if (e != hipSuccess) throw std::runtime_error(std::string("hipStreamWaitEvent: ") + hipGetErrorString(e));
             callerPending = false;
-            callerStream = nullptr;
         }
         ownPending = true;
         return stream;
@@ -2193,8 +2191,9 @@ akua_status akua_solver_step_device(akua_solver* s, void* dParticles, int32_t n,
                 HIP_CHECK(hipEventRecord(s->orderEvent, s->stream));
                 HIP_CHECK(hipStreamWaitEvent(user, s->orderEvent, 0));
             }
-            if (s->callerPending && s->callerStream != user)  // behind steps on another stream
-                HIP_CHECK(hipStreamWaitEvent(user, s->callerEvent, 0));
+            // behind the last such step, whatever its stream was: an equal handle need not be the same
+            // stream (hipStreamPerThread is each host thread's own; a destroyed stream's may come again)
+            if (s->callerPending) HIP_CHECK(hipStreamWaitEvent(user, s->callerEvent, 0));
             s->ownPending = false;
             // whatever happens, what was enqueued is known to later work on the solver's own stream
             struct Ended {
@@ -2202,7 +2201,6 @@ akua_status akua_solver_step_device(akua_solver* s, void* dParticles, int32_t n,
                 hipStream_t user;
                 ~Ended() {
                     s->callerPending = hipEventRecord(s->callerEvent, user) == hipSuccess;
-                    s->callerStream = user;
                     if (!s->callerPending) (void)hipStreamSynchronize(user);
                 }
             } ended{s, user};
