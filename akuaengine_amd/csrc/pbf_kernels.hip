@@ -339,6 +339,30 @@ __device__ __forceinline__ uint32_t wave_prefix(uint32_t v) {
     return (uint32_t)x;
 }
 
+// The largest value of this lane and those below it.
+__device__ __forceinline__ uint32_t wave_prefix_max(uint32_t v) {
+    int x = (int)v;
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false));  // row_shr:1
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false));  // row_shr:2
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false));  // row_shr:4
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false));  // row_shr:8
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));  // row_bcast:15 into rows 1 and 3
+    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)x;
+}
+
+// LDS written by some lanes of a wave and read by others: LDS instructions of one wave complete in
+// issue order, so only the compiler has to be kept from moving accesses across this point.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 // ---- small scenes: both orders from one counting pass ----------------------------------------------
 // Up to kOrderMaxSlots slots of a single scene take three launches where the two radix sorts, the cell
 // table and the move take thirteen, each at the launch's own cost (27,000 particles: 85 us of a 235 us
@@ -436,12 +460,230 @@ __global__ __launch_bounds__(kOrderBlock) void k_order_place(DeviceState d) {
     if (q < d.nslots) d.placed[q] = make_uint4(h, k, r.y, 0u);
 }
 
-// kCarry, kCarryDelta: as in k_gather.
+// ---- crowded groups of the orderings by counting -----------------------------------------------------
+// k_order_rank and k_tally_rank rank a particle by going through its group, a handful of members where the
+// particles spread over the cells.  In a group of more than kCrowd (thousands in one cell, or coincident, or
+// not finite, which all hash to one cell) that would be quadratic; such a group is sorted instead, by one of
+// the workgroups that the rank launch has in front for this: by digits of eight bits, stable, its 16-byte
+// records going to and fro between placed and tallied, which is free then.  Passes in which all digits are
+// equal fall away, so a group that is one crowded cell takes the two or three of the index.
+// Measured: 1M with clumps of up to 4,800 in a cell, rank launch 474 us unsorted, and with groups sorted from
+// 128 / 256 / 512 / 1,024 members on 286 / 208 / 208 / 216; 100,000 particles at one point 7.5 -> 0.44 ms a step
+// (0.49 by radix sorts), a million, one workgroup's work, 20 ms (2.2 by radix sorts).  Scenes without crowds: 1M
+// 110.5 us both ways, 27,000 particles 7.4 -> 7.7.
+constexpr uint32_t kCrowd = 512;
+constexpr uint32_t kCrowdPer = 4;  // records of a thread between the barriers of a pass
+constexpr uint32_t kMaxCrowdBlocks = 256;
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+struct CrowdLds {
+    uint32_t first[kBlock];              // next place of each digit
+    uint32_t wave[kBlock / 64][kBlock];  // digits of a tile by wave
+    uint32_t sums[kBlock / 64];
+    uint32_t crowds[kBlock], ncrowds;    // crowded groups of 256
+};
+// One for all the rank kernels: one in each would take its room in all of them.
+__device__ __forceinline__ CrowdLds& crowd_lds() {
+    __shared__ CrowdLds lds;
+    return lds;
+}
+
+__device__ __forceinline__ uint32_t bits_below(uint32_t n) { return n > 1u ? 32u - (uint32_t)__builtin_clz(n - 1u) : 0u; }
+
+// Sorts a[0, m) by the low bits of field kField, to and fro with b; a is where the records end up.  Every thread of
+// the workgroup, with the same arguments.
+template <char kField>
+__device__ __forceinline__ void crowd_sort(u32x4*& a, u32x4*& b, uint32_t m, uint32_t bits, CrowdLds& L) {
+    const auto key = [](u32x4 r) { return kField == 'x' ? r.x : kField == 'y' ? r.y : r.w; };
+    static_assert(kBlock == 256, "a thread per digit");
+    const uint32_t t = threadIdx.x, lane = __lane_id(), wave = t >> 6;
+    for (uint32_t shift = 0; shift < bits; shift += 8u) {
+        L.first[t] = 0u;
+#pragma unroll
+        for (uint32_t w = 0; w < kBlock / 64; ++w) L.wave[w][t] = 0u;
+        __syncthreads();
+        for (uint32_t i0 = 0; i0 < m; i0 += kBlock * 8u) {  // eight loads in flight
+            uint32_t k[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u) k[u] = key(a[min(i0 + u * kBlock + t, m - 1u)]);
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u)
+                if (i0 + u * kBlock + t < m) atomicAdd(&L.first[(k[u] >> shift) & 255u], 1u);
+        }
+        __syncthreads();
+        const uint32_t count = L.first[t];
+        if (__syncthreads_or(count == m)) continue;  // one digit
+        const uint32_t inclusive = wave_prefix(count);
+        if (lane == 63u) L.sums[wave] = inclusive;
+        __syncthreads();
+        uint32_t before = inclusive - count;
+        for (uint32_t w = 0; w < wave; ++w) before += L.sums[w];
+        L.first[t] = before;
+        __syncthreads();
+        for (uint32_t t0 = 0; t0 < m; t0 += kBlock * kCrowdPer) {
+            u32x4 r[kCrowdPer];
+            uint32_t rank[kCrowdPer];
+            const uint32_t mine = t0 + wave * (64u * kCrowdPer) + lane;
+#pragma unroll
+            for (uint32_t u = 0; u < kCrowdPer; ++u) r[u] = a[min(mine + 64u * u, m - 1u)];
+#pragma unroll
+            for (uint32_t u = 0; u < kCrowdPer; ++u) {
+                const bool in = mine + 64u * u < m;
+                const uint32_t digit = (key(r[u]) >> shift) & 255u;
+                uint64_t peers = __ballot(in);
+#pragma unroll
+                for (uint32_t k = 0; k < 8u; ++k) {
+                    const bool one = ((digit >> k) & 1u) != 0u;
+                    const uint64_t ones = __ballot(one);
+                    peers &= one ? ones : ~ones;
+                }
+                const uint32_t below = lanes_below(peers), prior = L.wave[wave][digit];
+                wave_lds_order();
+                if (in && below == 0u) L.wave[wave][digit] = prior + (uint32_t)__builtin_popcountll(peers);
+                wave_lds_order();
+                rank[u] = prior + below;
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t u = 0; u < kCrowdPer; ++u) {
+                const uint32_t digit = (key(r[u]) >> shift) & 255u;
+                uint32_t at = L.first[digit] + rank[u];
+                for (uint32_t w = 0; w < wave; ++w) at += L.wave[w][digit];
+                if (mine + 64u * u < m && at < m) b[at] = r[u];
+            }
+            __syncthreads();
+            uint32_t sum = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < kBlock / 64; ++w) {
+                sum += L.wave[w][t];
+                L.wave[w][t] = 0u;
+            }
+            L.first[t] += sum;
+            __syncthreads();
+        }
+        u32x4* const x = a;
+        a = b;
+        b = x;
+    }
+}
+
+// The move of a particle from slot src to slot p, logical index to.  kCarry, kCarryDelta: as in k_gather.
 template <bool kCarry, bool kCarryDelta>
-__global__ __launch_bounds__(kBlock) void k_order_rank(DeviceState d, StepParams S) {
-    const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
+__device__ __forceinline__ void order_move(const DeviceState& d, const StepParams& S, uint32_t src, uint32_t to,
+                                           uint32_t p, float4 x, float4 v, uint32_t id) {
+    const f3 xs = predict_x(make3(x), make3(v), S);
+    d.physT[to] = p;
+    d.X0[p] = x;
+    d.XsA[p] = make_float4(xs.x, xs.y, xs.z, x.w);
+    if (kCarry) {
+        d.Tdens[p] = d.dens[src];
+        d.Tlam[p] = d.lam[src];
+    }
+    if (kCarryDelta) d.TDP[p] = d.DP[src];
+    d.Tid[p] = id;
+    d.lidT[p] = to;
+}
+
+// The group of records [b, e): orders, table entries and moves.  kBins: with bins (k_tally_rank); else the
+// physical order is the logical order.  Records keep their hash in x throughout: the rank launch's other
+// threads read it to see that their group is not theirs.
+template <bool kCarry, bool kCarryDelta, bool kBins>
+__device__ __forceinline__ void crowd_place(const DeviceState& d, const StepParams& S, uint32_t b, uint32_t e, CrowdLds& L) {
+    const SceneDev& sc = d.scenes[0];
+    const uint32_t t = threadIdx.x, lane = __lane_id(), wave = t >> 6, m = e - b;
+    u32x4 *a = reinterpret_cast<u32x4*>(d.placed + b), *o = reinterpret_cast<u32x4*>(d.tallied + b);
+    crowd_sort<'y'>(a, o, m, bits_below(d.nslots), L);
+    crowd_sort<'x'>(a, o, m, kBins ? sc.groupShift : d.groupShift, L);
+    // logical order: (hash, logical index and in the top bit whether the hash begins there, slot, bin)
+    for (uint32_t i = t; i < m; i += kBlock) {
+        const u32x4 r = a[i];
+        const bool head = i == 0u || a[i - 1u].x != r.x;
+        d.skeysOut[b + i] = r.x;
+        d.perm1Out[b + i] = r.y;
+        o[i] = u32x4{r.x, (b + i) | (head ? 0x80000000u : 0u), r.z, r.w};
+    }
+    __syncthreads();
+    u32x4* const ordered = o;
+    o = a;
+    a = ordered;
+    if (kBins) crowd_sort<'w'>(a, o, m, bits_below(d.tallyCount), L);
+    uint32_t carry = 0;  // where the bin begins that the records before are in
+    for (uint32_t t0 = 0; t0 < m; t0 += kBlock) {
+        const uint32_t i = t0 + t;
+        const u32x4 r = a[min(i, m - 1u)];
+        const uint32_t h = r.x, to = r.y & 0x7FFFFFFFu, src = r.z, bin = r.w;
+        uint32_t p = to;
+        if (kBins) {
+            const uint32_t begins = wave_prefix_max(i < m && i != 0u && a[i - 1u].w != bin ? i : 0u);
+            if (lane == 63u) L.sums[wave] = begins;
+            __syncthreads();
+            uint32_t begin = max(carry, begins);
+            for (uint32_t w = 0; w < kBlock / 64; ++w) {
+                if (w < wave) begin = max(begin, L.sums[w]);
+                carry = max(carry, L.sums[w]);
+            }
+            __syncthreads();
+            if (d.tallyGroups + bin >= d.tallyCount) continue;  // consistent counts never produce this
+            p = d.tallyBase[d.tallyGroups + bin] - d.nparticles + (i - begin);
+        }
+        if (i >= m || src >= d.nslots || to >= sc.end || p >= sc.end) continue;
+        if ((r.y >> 31) != 0u) {
+            uint32_t last = to + 1u, end = e;  // the hash's end: the first place of another
+            while (last < end) {
+                const uint32_t mid = (last + end) >> 1;
+                if (d.skeysOut[mid] == h) last = mid + 1u;
+                else end = mid;
+            }
+            const uint32_t same = last - to;
+            bool together = same <= 256u;  // as in k_bucket_phys
+            if (kBins && together) {  // in one bin: its last member stands same - 1 records on
+                together = same <= m - i;
+                const u32x4 z = a[together ? i + same - 1u : i];
+                together = together && z.w == bin && (z.y & 0x7FFFFFFFu) == to + same - 1u;
+            }
+            const uint32_t slot = table_insert(d.table, sc, h);
+            if (slot != kEmptyKey) {
+                d.table[slot].y = to;
+                d.table[slot].z = to + same;
+                d.table[slot].w = p | (together ? 0x80000000u : 0u);
+            }
+        }
+        order_move<kCarry, kCarryDelta>(d, S, src, to, p, d.X[src], d.V[src], d.id[src]);
+    }
+    __syncthreads();
+}
+
+// The crowded ones of the groups, which begin at base[0, groups], by workgroup blockIdx.x of crowdBlocks.
+template <bool kCarry, bool kCarryDelta, bool kBins>
+__device__ __forceinline__ void crowd_groups(const DeviceState& d, const StepParams& S, const uint32_t* __restrict__ base,
+                                             uint32_t groups, uint32_t end, uint32_t crowdBlocks, CrowdLds& L) {
+    for (uint32_t g0 = blockIdx.x * kBlock; g0 < groups; g0 += crowdBlocks * kBlock) {
+        const uint32_t g = g0 + threadIdx.x;
+        const bool crowd = g < groups && min(base[g + 1u], end) - base[g] > kCrowd;
+        if (!__syncthreads_or(crowd)) continue;
+        if (threadIdx.x == 0) L.ncrowds = 0u;
+        __syncthreads();
+        if (crowd) L.crowds[atomicAdd(&L.ncrowds, 1u)] = g;
+        __syncthreads();
+        for (uint32_t k = 0; k < L.ncrowds; ++k) {
+            const uint32_t c = L.crowds[k];
+            crowd_place<kCarry, kCarryDelta, kBins>(d, S, base[c], min(base[c + 1u], end), L);
+        }
+        __syncthreads();
+    }
+}
+
+// kCarry, kCarryDelta: as in k_gather.  The first crowdBlocks workgroups take the crowded groups.
+template <bool kCarry, bool kCarryDelta>
+__global__ __launch_bounds__(kBlock) void k_order_rank(DeviceState d, StepParams S, uint32_t crowdBlocks) {
+    if (blockIdx.x < crowdBlocks) {
+        crowd_groups<kCarry, kCarryDelta, false>(d, S, d.groupBase, d.groups, d.nslots, crowdBlocks, crowd_lds());
+        return;
+    }
+    const uint32_t q = (blockIdx.x - crowdBlocks) * kBlock + threadIdx.x;
     // the counts were read by the launch before: empty for the next step
-    for (uint32_t g = q; g < d.groups; g += gridDim.x * kBlock) d.groupCount[g] = 0u;
+    for (uint32_t g = q; g < d.groups; g += (gridDim.x - crowdBlocks) * kBlock) d.groupCount[g] = 0u;
     if (q >= d.nslots) return;
     const SceneDev& sc = d.scenes[0];
     const uint4 me = d.placed[q];
@@ -450,6 +692,7 @@ __global__ __launch_bounds__(kBlock) void k_order_rank(DeviceState d, StepParams
     const float4 x = d.X[src], v = d.V[src];
     const uint32_t id = d.id[src];
     const uint32_t b = d.groupBase[group], e = min(d.groupBase[group + 1u], d.nslots);
+    if (e - b > kCrowd) return;
     uint32_t smaller = 0, same = 0, sameBefore = 0;
     constexpr uint32_t kBatch = 8;
     for (uint32_t m0 = b; m0 < e; m0 += kBatch) {
@@ -477,17 +720,7 @@ __global__ __launch_bounds__(kBlock) void k_order_rank(DeviceState d, StepParams
     }
     d.skeysOut[to] = h;
     d.perm1Out[to] = k;
-    const f3 xs = predict_x(make3(x), make3(v), S);
-    d.X0[to] = x;
-    d.XsA[to] = make_float4(xs.x, xs.y, xs.z, x.w);
-    if (kCarry) {
-        d.Tdens[to] = d.dens[src];
-        d.Tlam[to] = d.lam[src];
-    }
-    if (kCarryDelta) d.TDP[to] = d.DP[src];
-    d.Tid[to] = id;
-    d.lidT[to] = to;
-    d.physT[to] = to;
+    order_move<kCarry, kCarryDelta>(d, S, src, to, to, x, v, id);
 }
 
 // ---- larger scenes: both orders by counting, in five launches ----------------------------------------
@@ -608,10 +841,14 @@ __global__ __launch_bounds__(kBlock) void k_tally_place(DeviceState d) {
     if (q < d.nslots) d.placed[q] = make_uint4(r.x, r.y, p, r.w);
 }
 
-// kCarry, kCarryDelta: as in k_gather.
+// kCarry, kCarryDelta: as in k_gather.  The first crowdBlocks workgroups take the crowded groups.
 template <bool kCarry, bool kCarryDelta>
-__global__ __launch_bounds__(kBlock) void k_tally_rank(DeviceState d, StepParams S, uint32_t nparticles) {
-    const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
+__global__ __launch_bounds__(kBlock) void k_tally_rank(DeviceState d, StepParams S, uint32_t nparticles, uint32_t crowdBlocks) {
+    if (blockIdx.x < crowdBlocks) {
+        crowd_groups<kCarry, kCarryDelta, true>(d, S, d.tallyBase, d.tallyGroups, nparticles, crowdBlocks, crowd_lds());
+        return;
+    }
+    const uint32_t q = (blockIdx.x - crowdBlocks) * kBlock + threadIdx.x;
     if (q >= nparticles) return;
     const uint4 me = d.placed[q];
     const uint32_t h = me.x, k = me.y, src = me.z, bin = me.w;
@@ -622,6 +859,7 @@ __global__ __launch_bounds__(kBlock) void k_tally_rank(DeviceState d, StepParams
     const float4 x = d.X[src], v = d.V[src];
     const uint32_t id = d.id[src];
     const uint32_t b = d.tallyBase[group], e = min(d.tallyBase[group + 1u], nparticles);
+    if (e - b > kCrowd) return;
     const uint32_t binFirst = d.tallyBase[d.tallyGroups + bin] - nparticles;
     // among the group: smaller hashes, the bucket, those of it before this particle, those of it in the same
     // bin, and those in the same bin before this particle by hash and index
@@ -656,17 +894,7 @@ __global__ __launch_bounds__(kBlock) void k_tally_rank(DeviceState d, StepParams
     }
     d.skeysOut[to] = h;
     d.perm1Out[to] = k;
-    d.physT[to] = p;
-    const f3 xs = predict_x(make3(x), make3(v), S);
-    d.X0[p] = x;
-    d.XsA[p] = make_float4(xs.x, xs.y, xs.z, x.w);
-    if (kCarry) {
-        d.Tdens[p] = d.dens[src];
-        d.Tlam[p] = d.lam[src];
-    }
-    if (kCarryDelta) d.TDP[p] = d.DP[src];
-    d.Tid[p] = id;
-    d.lidT[p] = to;
+    order_move<kCarry, kCarryDelta>(d, S, src, to, p, x, v, id);
 }
 
 // Per bucket: where it starts in physical order and whether its particles occupy consecutive
@@ -886,18 +1114,6 @@ __host__ __device__ __forceinline__ uint32_t wave_row_words(int maxN) {
 template <uint32_t kWaveRows>
 __host__ __device__ __forceinline__ uint32_t wave_build_words(int maxN) {
     return kWaveRows * wave_row_words(maxN) + kWaveWindow / 32u + (2u * kWaveRuns * 27u + 3u) / 4u * 4u + 64u;
-}
-
-// LDS written by some lanes of a wave and read by others: LDS instructions of one wave complete in
-// issue order, so only the compiler has to be kept from moving accesses across this point.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
 __device__ __forceinline__ uint32_t lane_u(uint32_t v, uint32_t lane) {
@@ -1985,17 +2201,6 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v) {
     for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off, 64));
     return v;
 }
-// The largest value of this lane and those below it.
-__device__ __forceinline__ uint32_t wave_prefix_max(uint32_t v) {
-    int x = (int)v;
-    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false));  // row_shr:1
-    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false));  // row_shr:2
-    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false));  // row_shr:4
-    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false));  // row_shr:8
-    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));  // row_bcast:15 into rows 1 and 3
-    x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));  // row_bcast:31 into rows 2 and 3
-    return (uint32_t)x;
-}
 
 // LDS of a wave: NA rows of 64 chunks' terms, and the lists' lanes by chunk.
 template <int NA>
@@ -2817,17 +3022,22 @@ void launch_gather(hipStream_t st, const DeviceState& d, const SphParams& P, con
     else
         k_gather<false, false><<<grid(d.nslots), kBlock, 0, st>>>(d, P, S, layoutPrev);
 }
+namespace {
+// Workgroups for the crowded groups: each looks at 256 groups at least.
+inline uint32_t crowd_blocks(uint32_t groups) { return std::min((groups + kBlock - 1u) / kBlock, kMaxCrowdBlocks); }
+}  // namespace
 void launch_order(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
                   bool carryDelta) {
     const uint32_t count = grid(d.nslots);
     k_order_count<<<count + grid(d.tableTotal) + 1u, kBlock, 0, st>>>(d, P, S, count);
     k_order_place<<<(d.nslots + kOrderBlock - 1) / kOrderBlock, kOrderBlock, 0, st>>>(d);
+    const uint32_t crowd = crowd_blocks(d.groups);
     if (carryDelta)
-        k_order_rank<true, true><<<count, kBlock, 0, st>>>(d, S);
+        k_order_rank<true, true><<<crowd + count, kBlock, 0, st>>>(d, S, crowd);
     else if (carry)
-        k_order_rank<true, false><<<count, kBlock, 0, st>>>(d, S);
+        k_order_rank<true, false><<<crowd + count, kBlock, 0, st>>>(d, S, crowd);
     else
-        k_order_rank<false, false><<<count, kBlock, 0, st>>>(d, S);
+        k_order_rank<false, false><<<crowd + count, kBlock, 0, st>>>(d, S, crowd);
 }
 void launch_tally(hipStream_t st, const DeviceState& d, const SphParams& P, const StepParams& S, bool carry,
                   bool carryDelta) {
@@ -2836,13 +3046,13 @@ void launch_tally(hipStream_t st, const DeviceState& d, const SphParams& P, cons
     k_tally_sum<<<prefix, kTallyThreads, 0, st>>>(d);
     k_tally_prefix<<<prefix, kTallyThreads, 0, st>>>(d);
     k_tally_place<<<count, kBlock, 0, st>>>(d);
-    const uint32_t rank = grid(d.nparticles);
+    const uint32_t rank = grid(d.nparticles), crowd = crowd_blocks(d.tallyGroups);
     if (carryDelta)
-        k_tally_rank<true, true><<<rank, kBlock, 0, st>>>(d, S, d.nparticles);
+        k_tally_rank<true, true><<<crowd + rank, kBlock, 0, st>>>(d, S, d.nparticles, crowd);
     else if (carry)
-        k_tally_rank<true, false><<<rank, kBlock, 0, st>>>(d, S, d.nparticles);
+        k_tally_rank<true, false><<<crowd + rank, kBlock, 0, st>>>(d, S, d.nparticles, crowd);
     else
-        k_tally_rank<false, false><<<rank, kBlock, 0, st>>>(d, S, d.nparticles);
+        k_tally_rank<false, false><<<crowd + rank, kBlock, 0, st>>>(d, S, d.nparticles, crowd);
 }
 void launch_bucket_phys(hipStream_t st, const DeviceState& d) {
     k_bucket_phys<<<grid(d.nslots), kBlock, 0, st>>>(d);
