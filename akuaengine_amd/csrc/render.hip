@@ -72,53 +72,99 @@ __device__ __forceinline__ float sprite_d2(const Sprite& sp, int fx, int fy) {
     return ox * ox + oy * oy;
 }
 
-// kSplatLanes lanes per particle share its sprite's fragments: at the reference's point size a sprite
-// has some 80, and one thread per particle left the chip to a few waves of long serial loops.  A key that
-// the pixel already undercuts needs no atomic (keys only fall, so an old value read decides the same):
-// sprites overlap many deep.  Measured at 27,000 particles, 1280 x 720: 79 us with one thread, 36 with
-// eight lanes, 28 with their keys read four at a time, 25 with sixteen (300,000: 188 and 158).
-constexpr uint32_t kSplatLanes = 16, kSplatBatch = 4;
-
-__global__ __launch_bounds__(256) void k_render_splat(const float4* __restrict__ X, const float* __restrict__ size,
-                                                      const uint32_t* __restrict__ id,
-                                                      const uint32_t* __restrict__ lid, uint32_t n, RenderParams R,
-                                                      unsigned long long* zbuf) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t i = t / kSplatLanes;
-    if (i >= n) return;
-    const float4 x = X[i];
-    const uint32_t draw = lid[i];
-    const float sz = R.pointSize > 0.0f ? R.pointSize : size[id[i]];
+// A sprite's fragments on the screen: the rectangle's first column and row, its width and size, and the key
+// (depth, then draw order) that its pixels take the smallest of.
+struct Splat {
     Sprite sp;
-    if (!sprite_of(R, x.x, x.y, x.z, sz, sp)) return;
-    const float x0 = sp.xw - 0.5f * sp.s, y0 = sp.yw - 0.5f * sp.s;
+    int fx0, fy0;
+    uint32_t w, count;  // count 0: nothing to draw
+    unsigned long long key;
+};
+
+__device__ __forceinline__ Splat splat_of(const RenderParams& R, float4 x, float size, uint32_t draw) {
+    Splat s;
+    s.count = 0u;
+    if (!sprite_of(R, x.x, x.y, x.z, size, s.sp)) return s;
+    const float x0 = s.sp.xw - 0.5f * s.sp.s, y0 = s.sp.yw - 0.5f * s.sp.s;
     // fragments whose centres f + 0.5 lie in [x0, x0 + s)
-    int fx0 = (int)ceilf(x0 - 0.5f), fx1 = (int)ceilf(x0 + sp.s - 0.5f) - 1;
-    int fy0 = (int)ceilf(y0 - 0.5f), fy1 = (int)ceilf(y0 + sp.s - 0.5f) - 1;
+    int fx0 = (int)ceilf(x0 - 0.5f), fx1 = (int)ceilf(x0 + s.sp.s - 0.5f) - 1;
+    int fy0 = (int)ceilf(y0 - 0.5f), fy1 = (int)ceilf(y0 + s.sp.s - 0.5f) - 1;
     fx0 = max(fx0, 0);
     fy0 = max(fy0, 0);
     fx1 = min(fx1, R.width - 1);
     fy1 = min(fy1, R.height - 1);
-    if (fx1 < fx0 || fy1 < fy0) return;
-    const unsigned long long key = ((unsigned long long)__float_as_uint(sp.zw) << 32) | (unsigned long long)draw;
-    // fragments of the rectangle row by row (at most 257 x 257), kSplatBatch of this lane's at a time:
-    // their pixels' keys are read together
-    const uint32_t w = (uint32_t)(fx1 - fx0 + 1), count = w * (uint32_t)(fy1 - fy0 + 1);
-    uint32_t row = (t % kSplatLanes) / w, column = t % kSplatLanes - row * w;
-    for (uint32_t f = t % kSplatLanes; f < count; f += kSplatLanes * kSplatBatch) {
+    if (fx1 < fx0 || fy1 < fy0) return s;
+    s.fx0 = fx0;
+    s.fy0 = fy0;
+    s.w = (uint32_t)(fx1 - fx0 + 1);
+    s.count = s.w * (uint32_t)(fy1 - fy0 + 1);  // at most 257 x 257
+    s.key = ((unsigned long long)__float_as_uint(s.sp.zw) << 32) | (unsigned long long)draw;
+    return s;
+}
+
+// Fragments first, first + kStride, ... of the rectangle row by row, kSplatBatch at a time: their pixels' keys are
+// read together.  A key that the pixel already undercuts needs no atomic (keys only fall, so an old value
+// read decides the same): sprites overlap many deep.
+constexpr uint32_t kSplatBatch = 4;
+template <uint32_t kStride>
+__device__ __forceinline__ void splat_draw(const RenderParams& R, const Splat& s, uint32_t first, unsigned long long* zbuf) {
+    uint32_t row = first / s.w, column = first - row * s.w;
+    for (uint32_t f = first; f < s.count; f += kStride * kSplatBatch) {
         unsigned long long* at[kSplatBatch];
         unsigned long long old[kSplatBatch];
 #pragma unroll
         for (uint32_t u = 0; u < kSplatBatch; ++u) {
-            const int fx = fx0 + (int)column, fy = fy0 + (int)row;
-            const bool in = f + u * kSplatLanes < count && !(sprite_d2(sp, fx, fy) > 0.25f);
+            const int fx = s.fx0 + (int)column, fy = s.fy0 + (int)row;
+            const bool in = f + u * kStride < s.count && !(sprite_d2(s.sp, fx, fy) > 0.25f);
             at[u] = in ? &zbuf[(size_t)(R.height - 1 - fy) * (size_t)R.width + (size_t)fx] : nullptr;
             old[u] = in ? __hip_atomic_load(at[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0ull;
-            for (column += kSplatLanes; column >= w; column -= w) ++row;
+            for (column += kStride; column >= s.w; column -= s.w) ++row;
         }
 #pragma unroll
         for (uint32_t u = 0; u < kSplatBatch; ++u)
-            if (old[u] > key) atomicMin(at[u], key);
+            if (old[u] > s.key) atomicMin(at[u], s.key);
+    }
+}
+
+// A wave projects kPer particles, one per lane.  A sprite of a few fragments is drawn by its lane, a
+// larger one by sixteen, four sprites at a time: at the reference's point size a near sprite has some 80
+// fragments, a serial chain for one lane, and a distant one a few, for which sixteen lanes are idle.  Measured at
+// 1280 x 720, us with one lane per sprite / with sixteen / so: 27,000 particles 269 / 54 / 54, in sprites of about
+// one pixel 2.5 / 8.1 / 4.7; a million over the image 454 / 261 / 123, of 3-5 pixels 34 / 147 / 37; eight million
+// 509 / 1,170 / 507 and 296 / 1,112 / 293.
+constexpr uint32_t kSplatLanes = 16;
+
+template <uint32_t kPer>
+__global__ __launch_bounds__(256) void k_render_splat(const float4* __restrict__ X, const float* __restrict__ size,
+                                                      const uint32_t* __restrict__ id,
+                                                      const uint32_t* __restrict__ lid, uint32_t n, RenderParams R,
+                                                      unsigned long long* zbuf) {
+    constexpr uint32_t kOwn = kPer == 4u ? 4u : 8u;  // with four particles all of them have their lanes at once
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t i = (blockIdx.x * (256u / 64u) + (threadIdx.x >> 6)) * kPer + lane;
+    Splat mine;
+    mine.count = 0u;
+    if (lane < kPer && i < n) mine = splat_of(R, X[i], R.pointSize > 0.0f ? R.pointSize : size[id[i]], lid[i]);
+    if (mine.count != 0u && mine.count <= kOwn) splat_draw<1u>(R, mine, 0u, zbuf);
+    for (unsigned long long large = __ballot(mine.count > kOwn); large != 0ull;) {
+        // the next four: this lane's sixteen take the (lane / 16)th
+        uint32_t from = 64u;
+#pragma unroll
+        for (uint32_t g = 0; g < 64u / kSplatLanes; ++g) {
+            if (g == lane / kSplatLanes && large != 0ull) from = (uint32_t)__builtin_ctzll(large);
+            large &= large - 1ull;
+        }
+        const int of = (int)(from & 63u);
+        Splat s;
+        s.sp.xw = __shfl(mine.sp.xw, of, 64);
+        s.sp.yw = __shfl(mine.sp.yw, of, 64);
+        s.sp.s = __shfl(mine.sp.s, of, 64);
+        s.fx0 = __shfl(mine.fx0, of, 64);
+        s.fy0 = __shfl(mine.fy0, of, 64);
+        s.w = (uint32_t)__shfl((int)mine.w, of, 64);
+        s.count = (uint32_t)__shfl((int)mine.count, of, 64);
+        s.key = (unsigned long long)__shfl((long long)mine.key, of, 64);
+        if (from < 64u) splat_draw<kSplatLanes>(R, s, lane % kSplatLanes, zbuf);
     }
 }
 
@@ -251,11 +297,17 @@ void launch_render(hipStream_t st, const float4* X, const float4* color, const f
                    const RenderParams& R, unsigned long long* zbuf, unsigned char* rgb) {
     const uint32_t pixels = (uint32_t)(R.width * R.height);
     k_render_clear<<<(std::max(pixels, n) + 255) / 256, 256, 0, st>>>(zbuf, pixels, lid, phys, n);
-    if (n) {
-        // at most 2^28 slots: the lanes number at most 2^32, the last of them 2^32 - 1
-        const uint32_t blocks = (uint32_t)(((uint64_t)n * kSplatLanes + 255u) / 256u);
-        k_render_splat<<<blocks, 256, 0, st>>>(X, size, id, lid, n, R, zbuf);
-    }
+    // fewer particles per wave where few waves would draw them all
+    const auto splat = [&](auto kernel, uint32_t per) {
+        const uint32_t waves = (n + per - 1u) / per;
+        kernel<<<(waves + 3u) / 4u, 256, 0, st>>>(X, size, id, lid, n, R, zbuf);
+    };
+    if (n > (1u << 17))
+        splat(k_render_splat<64>, 64u);
+    else if (n > (1u << 15))
+        splat(k_render_splat<16>, 16u);
+    else if (n)
+        splat(k_render_splat<4>, 4u);
     k_render_resolve<<<(pixels + 255) / 256, 256, 0, st>>>(X, color, size, id, phys, R, zbuf, rgb);
 }
 
