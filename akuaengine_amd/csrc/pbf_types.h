@@ -123,6 +123,12 @@ constexpr uint32_t kSlotAlign = 256;
 // Most slots of a solver: per-slot arrays of up to 16-byte elements are then addressed by 32-bit
 // byte offsets in the kernels.
 constexpr uint32_t kMaxSlots = 1u << 28;
+// Lanes per slot (a power of two) that one launch can have: fewer than asked for where its work items, up to
+// 2,048 slots more than there are (whole workgroups, on every XCD), would reach 2^32.
+constexpr int launch_lanes(uint32_t nslots, int lanes) {
+    while (lanes > 1 && ((uint64_t)nslots + 2048u) * (uint64_t)lanes >= (1ull << 32)) lanes /= 2;
+    return lanes;
+}
 constexpr uint32_t kEmptyKey = 0xFFFFFFFFu;  // never a hash: hashes are < tableSize <= 2^32 - 1
 
 }  // namespace akua

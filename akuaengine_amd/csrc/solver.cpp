@@ -763,7 +763,7 @@ struct SweepLanes {
 };
 SweepLanes sweep_lanes(const akua_solver* s) {
     const auto all = [](int n) { return SweepLanes{n, n, n, n, n, n}; };
-    if (s->tuning.laneGroup > 0) return all(s->tuning.laneGroup);
+    if (s->tuning.laneGroup > 0) return all(launch_lanes(s->nslots, s->tuning.laneGroup));
     if (s->nslots <= (1u << 15)) return all(16);
     if (s->nslots <= (1u << 18)) return all(4);
     return SweepLanes{1, kLanesShared, kLanesShared, 4, 2, 4};
