@@ -23,9 +23,9 @@ void camera_setup(const float position[3], float yawDeg, float pitchDeg, float f
 
 // Slots 0..n-1 of one scene: X (physical order), colour and size by particle id, the logical
 // (draw) index of each slot and the slot of each logical index.  zbuf: width * height keys;
-// rgb: width * height * 3 bytes (device memory).
+// rgb: width * height * 3 bytes (device memory).  huge: n + 1 words of scratch.
 void launch_render(hipStream_t st, const float4* X, const float4* color, const float* size,
                    const uint32_t* id, const uint32_t* lid, uint32_t* phys, uint32_t n,
-                   const RenderParams& R, unsigned long long* zbuf, unsigned char* rgb);
+                   const RenderParams& R, unsigned long long* zbuf, unsigned char* rgb, uint32_t* huge);
 
 }  // namespace akua

@@ -26,10 +26,11 @@ constexpr float kMaxPointSize = 256.0f;  // GL clamps sprites to an implementati
 constexpr float kFloorY = -0.02f;        // FLOOR_LEVEL (Application.cpp:16)
 constexpr float kFloorExtent = 100.0f;   // floor quad x, z in [0, 100] (Application.cpp:130-135)
 
-// Empties the pixels' keys and inverts the draw order: phys[k], the slot drawn k-th.
+// Empties the pixels' keys and the list of huge sprites and inverts the draw order: phys[k], the slot drawn k-th.
 __global__ void k_render_clear(unsigned long long* __restrict__ z, uint32_t pixels, const uint32_t* __restrict__ lid,
-                               uint32_t* __restrict__ phys, uint32_t n) {
+                               uint32_t* __restrict__ phys, uint32_t n, uint32_t* __restrict__ huge) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0u) huge[0] = 0u;
     if (i < pixels) z[i] = ~0ull;
     if (i < n) {
         const uint32_t k = lid[i];
@@ -128,17 +129,19 @@ __device__ __forceinline__ void splat_draw(const RenderParams& R, const Splat& s
 
 // A wave projects kPer particles, one per lane.  A sprite of a few fragments is drawn by its lane, a
 // larger one by sixteen, four sprites at a time: at the reference's point size a near sprite has some 80
-// fragments, a serial chain for one lane, and a distant one a few, for which sixteen lanes are idle.  Measured at
-// 1280 x 720, us with one lane per sprite / with sixteen / so: 27,000 particles 269 / 54 / 54, in sprites of about
-// one pixel 2.5 / 8.1 / 4.7; a million over the image 454 / 261 / 123, of 3-5 pixels 34 / 147 / 37; eight million
-// 509 / 1,170 / 507 and 296 / 1,112 / 293.
-constexpr uint32_t kSplatLanes = 16;
+// fragments, a serial chain for one lane, and a distant one a few, for which sixteen lanes are idle.  Sprites of
+// more than kSplatHuge fragments, close to the camera, are listed for a launch of their own (kList): those of one
+// wave would keep it busy long after the others.  Measured at 1280 x 720, us with one lane per sprite / with
+// sixteen / so: 27,000 particles in the default view 267 / 53 / 53, in sprites of about one pixel 3 / 7 / 4; 1M from
+// (5, 4, 16) 459 / 249 / 176, in sprites of 1-5 pixels 34 / 148 / 58, from within 6,602 / 1,658 / 286; 8M 526 / 1,166
+// / 517 and 300 / 1,182 / 307.
+constexpr uint32_t kSplatLanes = 16, kSplatHuge = 1024;
 
-template <uint32_t kPer>
+template <uint32_t kPer, bool kList>
 __global__ __launch_bounds__(256) void k_render_splat(const float4* __restrict__ X, const float* __restrict__ size,
                                                       const uint32_t* __restrict__ id,
                                                       const uint32_t* __restrict__ lid, uint32_t n, RenderParams R,
-                                                      unsigned long long* zbuf) {
+                                                      unsigned long long* zbuf, uint32_t* __restrict__ huge) {
     constexpr uint32_t kOwn = kPer == 4u ? 4u : 8u;  // with four particles all of them have their lanes at once
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t i = (blockIdx.x * (256u / 64u) + (threadIdx.x >> 6)) * kPer + lane;
@@ -146,6 +149,19 @@ __global__ __launch_bounds__(256) void k_render_splat(const float4* __restrict__
     mine.count = 0u;
     if (lane < kPer && i < n) mine = splat_of(R, X[i], R.pointSize > 0.0f ? R.pointSize : size[id[i]], lid[i]);
     if (mine.count != 0u && mine.count <= kOwn) splat_draw<1u>(R, mine, 0u, zbuf);
+    if (kList) {
+        const bool listed = mine.count > kSplatHuge;
+        const unsigned long long all = __ballot(listed);
+        if (all != 0ull) {
+            uint32_t at = 0;
+            if (lane == 0u) at = atomicAdd(huge, (uint32_t)__builtin_popcountll(all));
+            at = (uint32_t)__shfl((int)at, 0, 64) + (uint32_t)__builtin_popcountll(all & ~(~0ull << lane));
+            if (listed) {
+                huge[1u + at] = i;
+                mine.count = 0u;
+            }
+        }
+    }
     for (unsigned long long large = __ballot(mine.count > kOwn); large != 0ull;) {
         // the next four: this lane's sixteen take the (lane / 16)th
         uint32_t from = 64u;
@@ -165,6 +181,20 @@ __global__ __launch_bounds__(256) void k_render_splat(const float4* __restrict__
         s.count = (uint32_t)__shfl((int)mine.count, of, 64);
         s.key = (unsigned long long)__shfl((long long)mine.key, of, 64);
         if (from < 64u) splat_draw<kSplatLanes>(R, s, lane % kSplatLanes, zbuf);
+    }
+}
+
+// The listed sprites, a workgroup each.
+constexpr uint32_t kHugeBlock = 256, kHugeBlocks = 2048;
+__global__ __launch_bounds__(kHugeBlock) void k_render_huge(const float4* __restrict__ X, const float* __restrict__ size,
+                                                            const uint32_t* __restrict__ id,
+                                                            const uint32_t* __restrict__ lid, uint32_t n, RenderParams R,
+                                                            unsigned long long* zbuf, const uint32_t* __restrict__ huge) {
+    const uint32_t count = min(huge[0], n);
+    for (uint32_t q = blockIdx.x; q < count; q += gridDim.x) {
+        const uint32_t i = min(huge[1u + q], n - 1u);
+        const Splat s = splat_of(R, X[i], R.pointSize > 0.0f ? R.pointSize : size[id[i]], lid[i]);
+        if (s.count != 0u) splat_draw<kHugeBlock>(R, s, threadIdx.x, zbuf);
     }
 }
 
@@ -294,20 +324,23 @@ void camera_setup(const float position[3], float yawDeg, float pitchDeg, float f
 
 void launch_render(hipStream_t st, const float4* X, const float4* color, const float* size,
                    const uint32_t* id, const uint32_t* lid, uint32_t* phys, uint32_t n,
-                   const RenderParams& R, unsigned long long* zbuf, unsigned char* rgb) {
+                   const RenderParams& R, unsigned long long* zbuf, unsigned char* rgb, uint32_t* huge) {
     const uint32_t pixels = (uint32_t)(R.width * R.height);
-    k_render_clear<<<(std::max(pixels, n) + 255) / 256, 256, 0, st>>>(zbuf, pixels, lid, phys, n);
-    // fewer particles per wave where few waves would draw them all
+    k_render_clear<<<(std::max(pixels, n) + 255) / 256, 256, 0, st>>>(zbuf, pixels, lid, phys, n, huge);
+    // Particles per wave: fewer where few waves would draw them all, and up to 2^21 no more than sixteen, as the
+    // sprites of a wave lie side by side and one near the camera is at work for longest (1M from (3, 2, 6) after 30
+    // steps, us with one lane per sprite / sixteen / so with 64 / so with 16: 896 / 191 / 485 / 205).
     const auto splat = [&](auto kernel, uint32_t per) {
         const uint32_t waves = (n + per - 1u) / per;
-        kernel<<<(waves + 3u) / 4u, 256, 0, st>>>(X, size, id, lid, n, R, zbuf);
+        kernel<<<(waves + 3u) / 4u, 256, 0, st>>>(X, size, id, lid, n, R, zbuf, huge);
     };
-    if (n > (1u << 17))
-        splat(k_render_splat<64>, 64u);
+    if (n > (1u << 21))
+        splat(k_render_splat<64, true>, 64u);
     else if (n > (1u << 15))
-        splat(k_render_splat<16>, 16u);
+        splat(k_render_splat<16, true>, 16u);
     else if (n)
-        splat(k_render_splat<4>, 4u);
+        splat(k_render_splat<4, false>, 4u);
+    if (n > (1u << 15)) k_render_huge<<<kHugeBlocks, kHugeBlock, 0, st>>>(X, size, id, lid, n, R, zbuf, huge);
     k_render_resolve<<<(pixels + 255) / 256, 256, 0, st>>>(X, color, size, id, phys, R, zbuf, rgb);
 }
 

@@ -2449,7 +2449,8 @@ akua_status akua_render(akua_solver* s, const akua_camera* cam, int32_t width, i
             if (s->renderRgb.n < 3 * pixels) s->renderRgb.alloc(3 * pixels);
         }
         launch_render(s->joined(), s->X.p, s->color.p, s->size.p, s->id.p, s->lid.p, s->phys.p,
-                      s->scenes[0].end, R, s->renderKeys.p, s->renderRgb.p);
+                      s->scenes[0].end, R, s->renderKeys.p, s->renderRgb.p,
+                      reinterpret_cast<uint32_t*>(s->XsC.p));  // which every step writes before it reads it
         HIP_CHECK(hipGetLastError());
         read_back(s, {{rgb, s->renderRgb.p, 3 * pixels}});
     });

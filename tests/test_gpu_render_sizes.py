@@ -26,7 +26,8 @@ def _scene(n, rng):
     return vis, pos, col, size
 
 
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 32767, 32768, 32769, 32785, 131071, 131072, 131073, 131137])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 32767, 32768, 32769, 32785, 131071, 131072, 131073, 131137,
+                               (1 << 21) - 1, (1 << 21) + 1])
 def test_image_does_not_depend_on_the_number_of_particles(n):
     import torch
     if torch.cuda.device_count() < 1:
