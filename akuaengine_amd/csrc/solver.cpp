@@ -167,50 +167,19 @@ struct TimedLaunch {
     hipEvent_t a, b;
 };
 
-// Pinned host chunks that device memory passes through on its way to the caller's pageable memory,
-// each with the event of its last copy.  At most kStageChunks chunks, made when first used and kept
-// with the solver.
-constexpr size_t kStageChunk = 1u << 20, kStageChunks = 16;
-
-struct Staging {
-    std::vector<char*> chunk;
-    std::vector<hipEvent_t> ready;
-    size_t bytes = 0;  // of each chunk
-    Staging() = default;
-    Staging(const Staging&) = delete;
-    Staging& operator=(const Staging&) = delete;
-    // Chunks for `total` bytes: at least one, or false where the host has no pinned memory left.
-    bool ensure(size_t total) {
-        const size_t want = std::min(kStageChunk, (total + 65535) / 65536 * 65536);
-        if (want > bytes) {
-            release();
-            bytes = want;
-        }
-        const size_t count = std::min(kStageChunks, (total + bytes - 1) / bytes);
-        while (chunk.size() < count) {
-            if (ready.size() == chunk.size()) {
-                hipEvent_t e = nullptr;
-                HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-                ready.push_back(e);
-            }
-            void* p = nullptr;
-            if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
-                (void)hipGetLastError();
-                break;
-            }
-            chunk.push_back(static_cast<char*>(p));
-        }
-        return !chunk.empty();
-    }
-    void release() {
-        for (auto e : ready) (void)hipEventDestroy(e);
-        for (auto p : chunk) (void)hipHostFree(p);
-        ready.clear();
-        chunk.clear();
-        bytes = 0;
-    }
-    ~Staging() { release(); }
+// Pinned host memory that device memory passes through on its way to the caller's pageable memory: one ring of
+// chunks for all solvers, of kRingSmall bytes or, once more than kReadbackInline are read at a time, kRingLarge; used
+// by one read-back at a time (another at the same time copies without it) and freed with the last solver that has
+// used it.  One allocation for all its chunks: each one costs up to 0.3 ms.
+constexpr size_t kRingSmall = 2u << 20, kRingLarge = 16u << 20;
+constexpr size_t kChunkSmall = 512u << 10, kChunkLarge = 1u << 20;
+struct PinnedRing {
+    std::mutex use;
+    char* p = nullptr;
+    size_t bytes = 0;
+    int solvers = 0;
 };
+PinnedRing g_ring;
 
 }  // namespace
 
@@ -340,7 +309,10 @@ struct akua_solver {
     }
     // record export staging (get_particles), allocated on first use
     DevBuf<AosParticle> aosStage;
-    Staging staging;  // pinned chunks of get_state and get_particles, allocated on first use
+    // the read-backs of get_state, get_particles and render: whether this solver counts among g_ring's, an event
+    // for each chunk's last copy, and whether there has been a small read-back
+    bool usesRing = false, readBefore = false;
+    std::vector<hipEvent_t> chunkReady;
 
     // timing
     bool timing = false;
@@ -402,7 +374,15 @@ struct akua_solver {
         wait_for_caller();
         if (stream) (void)hipStreamSynchronize(stream);
         release_buffers();
-        staging.release();
+        for (auto e : chunkReady) (void)hipEventDestroy(e);
+        if (usesRing) {
+            std::lock_guard<std::mutex> lock(g_ring.use);
+            if (--g_ring.solvers == 0) {
+                (void)hipHostFree(g_ring.p);
+                g_ring.p = nullptr;
+                g_ring.bytes = 0;
+            }
+        }
         for (auto& g : graphs)
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
         for (auto e : eventPool) (void)hipEventDestroy(e);
@@ -1305,6 +1285,36 @@ struct Readback {
 constexpr size_t kReadbackInline = 4u << 20, kReadbackPerThread = 2u << 20;
 constexpr unsigned kReadbackThreads = 8;
 
+// Whether this read-back passes through the ring, whose lock the caller holds.  A solver's first small one
+// does not make the ring: a program that reads or draws once would only pay for it (27,000 particles: 0.19 ms
+// without, 0.17 with the ring and 0.3 for making it).
+bool take_ring(akua_solver* s, size_t total) {
+    const bool first = !s->readBefore;
+    s->readBefore = true;
+    const size_t want = total <= kReadbackInline ? kRingSmall : kRingLarge;
+    if (g_ring.bytes < want) {
+        if (first && total <= kReadbackInline) return false;
+        void* p = nullptr;
+        if (hipHostMalloc(&p, want, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (g_ring.p) (void)hipHostFree(g_ring.p);
+        g_ring.p = static_cast<char*>(p);
+        g_ring.bytes = want;
+    }
+    if (!s->usesRing) {
+        s->usesRing = true;
+        ++g_ring.solvers;
+    }
+    while (s->chunkReady.size() < g_ring.bytes / kChunkSmall) {
+        hipEvent_t e = nullptr;
+        HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        s->chunkReady.push_back(e);
+    }
+    return true;
+}
+
 void read_back(akua_solver* s, const std::vector<Readback>& pieces) {
     struct Part {
         char* to;
@@ -1314,23 +1324,25 @@ void read_back(akua_solver* s, const std::vector<Readback>& pieces) {
     size_t total = 0;
     for (const Readback& r : pieces) total += r.bytes;
     if (!total) return;
-    if (!s->staging.ensure(total)) {
+    std::unique_lock<std::mutex> ringLock(g_ring.use, std::try_to_lock);
+    if (!ringLock.owns_lock() || !take_ring(s, total)) {
+        if (ringLock.owns_lock()) ringLock.unlock();
         HIP_CHECK(hipStreamSynchronize(s->joined()));
         for (const Readback& r : pieces) HIP_CHECK(hipMemcpy(r.to, r.from, r.bytes, hipMemcpyDeviceToHost));
         return;
     }
-    const size_t chunk = s->staging.bytes, ring = s->staging.chunk.size();
+    const size_t chunk = total <= kReadbackInline ? kChunkSmall : kChunkLarge, ring = g_ring.bytes / chunk;
+    const auto chunk_of = [&](size_t k) { return g_ring.p + k % ring * chunk; };
     std::vector<Part> parts;
     for (const Readback& r : pieces)
         for (size_t o = 0; o < r.bytes; o += chunk)
             parts.push_back({static_cast<char*>(r.to) + o, static_cast<const char*>(r.from) + o,
                              std::min(chunk, r.bytes - o)});
     const auto issue = [&](size_t k) {
-        HIP_CHECK(hipMemcpyAsync(s->staging.chunk[k % ring], parts[k].from, parts[k].bytes, hipMemcpyDeviceToHost,
-                                 s->joined()));
-        HIP_CHECK(hipEventRecord(s->staging.ready[k % ring], s->joined()));
+        HIP_CHECK(hipMemcpyAsync(chunk_of(k), parts[k].from, parts[k].bytes, hipMemcpyDeviceToHost, s->joined()));
+        HIP_CHECK(hipEventRecord(s->chunkReady[k % ring], s->joined()));
     };
-    const auto empty = [&](size_t k) { std::memcpy(parts[k].to, s->staging.chunk[k % ring], parts[k].bytes); };
+    const auto empty = [&](size_t k) { std::memcpy(parts[k].to, chunk_of(k), parts[k].bytes); };
     // whatever happens, no copy into the chunks is left in flight
     struct Drain {
         hipStream_t st;
@@ -1341,7 +1353,7 @@ void read_back(akua_solver* s, const std::vector<Readback>& pieces) {
         size_t issued = 0;
         for (size_t k = 0; k < parts.size(); ++k) {
             for (; issued < parts.size() && issued < k + ring; ++issued) issue(issued);
-            HIP_CHECK(hipEventSynchronize(s->staging.ready[k % ring]));
+            HIP_CHECK(hipEventSynchronize(s->chunkReady[k % ring]));
             empty(k);
         }
         return;
@@ -1399,7 +1411,7 @@ void read_back(akua_solver* s, const std::vector<Readback>& pieces) {
             }
             issue(issued);
         }
-        HIP_CHECK(hipEventSynchronize(s->staging.ready[k % ring]));
+        HIP_CHECK(hipEventSynchronize(s->chunkReady[k % ring]));
         if (alone) {
             empty(k);
             done[k] = 1;
