@@ -1517,6 +1517,8 @@ double time_trial(akua_solver* s, const Snapshot& q, float dt, int steps) {
     return best / steps;
 }
 
+// Part of the key: raised when the kernels change so much that settings measured before no longer hold.
+constexpr int kTunedKernels = 2;
 std::string tuning_key(akua_solver* s) {
     hipDeviceProp_t prop{};
     HIP_CHECK(hipGetDeviceProperties(&prop, s->device));
@@ -1526,7 +1528,7 @@ std::string tuning_key(akua_solver* s) {
     std::ostringstream k;
     k << arch << " n2^" << ceil_log2(std::max<uint64_t>(1, s->nparticles)) << " scenes2^"
       << ceil_log2(std::max<uint64_t>(1, s->scenes.size())) << " cap" << s->cfg.maxNeighbours
-      << " it" << s->cfg.solverIterations << (s->exact ? "" : " inexact");
+      << " it" << s->cfg.solverIterations << " kernels" << kTunedKernels << (s->exact ? "" : " inexact");
     return k.str();
 }
 

@@ -205,11 +205,14 @@ akua_status akua_solver_set_exact(akua_solver* s, int32_t exact);
 akua_status akua_solver_get_tuning(const akua_solver* s, akua_tuning* t);
 /* Times short trials of candidate settings by coordinate descent (block, then layout level, then
  * the two digit widths, then the layout interval and the balance tile, then the lane group and the
- * work queue together) and keeps the fastest.  Each trial restarts from a copy of the current particle state, which is restored afterwards, so the call leaves the state as it found it.
+ * work queue together) and keeps the fastest.  Each trial restarts from a copy of the current
+ * particle state, which is restored afterwards, so the call leaves the state as it found it.
  * boxMin/boxMax: the box the trials step in (NULL: each scene's current box).  trialSteps: timed
- * steps per candidate (1..1000), run twice; the faster run counts.  cachePath (NULL: no cache): a text file of earlier results keyed
- * by device architecture, log2 of the particle count, log2 of the scene count, neighbour cap and
- * iteration count; a hit applies the cached setting without trials, a miss appends the result.
+ * steps per candidate (1..1000), run twice; the faster run counts.  cachePath (NULL: no cache): a
+ * text file of earlier results keyed by device architecture, log2 of the particle count, log2 of
+ * the scene count, neighbour cap, iteration count and a number for the library's kernels (results
+ * measured with others are left in the file and not applied); a hit applies the cached setting
+ * without trials, a miss appends the result.
  * best (may be NULL) receives the setting now in use. */
 akua_status akua_solver_autotune(akua_solver* s, float deltaTime, const float boxMin[3],
                                  const float boxMax[3], int32_t trialSteps, const char* cachePath,
