@@ -40,7 +40,6 @@ namespace akua {
 
 struct DeviceState {
     uint32_t nslots;           // particle slots (all scenes, with alignment padding)
-    uint32_t nparticles;
     const SceneDev* scenes;
     const uint32_t* chunkScene;  // scene of each 256-slot chunk
     float4* X;
@@ -83,7 +82,7 @@ struct DeviceState {
     uint32_t* tally;
     uint32_t* tallyBase;       // tallyCount + 1 entries
     uint32_t* tallyPart;       // per workgroup of the prefix
-    uint32_t tallyGroups, tallyCount;  // groups, groups and bins, of all scenes
+    uint32_t tallyGroups, tallyCount;  // groups, groups and bins
     uint4* tallied;            // (hash, previous logical index, place in its group, bin) of each slot
     uint32_t* skeysOut;        // skeys and perm1, for their writer
     uint32_t* perm1Out;

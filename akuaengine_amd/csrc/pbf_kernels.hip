@@ -625,7 +625,7 @@ __device__ __forceinline__ void crowd_place(const DeviceState& d, const StepPara
             }
             __syncthreads();
             if (d.tallyGroups + bin >= d.tallyCount) continue;  // consistent counts never produce this
-            p = d.tallyBase[d.tallyGroups + bin] - d.nparticles + (i - begin);
+            p = d.tallyBase[d.tallyGroups + bin] - d.nslots + (i - begin);
         }
         if (i >= m || src >= d.nslots || to >= sc.end || p >= sc.end) continue;
         if ((r.y >> 31) != 0u) {
@@ -733,7 +733,7 @@ __global__ __launch_bounds__(kBlock) void k_order_rank(DeviceState d, StepParams
 // 112 us in a settled flow, 266 -> 237 sprayed, where particles of a cell seldom lie side by side and the
 // counting (22 -> 92 us) and ranking (65 -> 110) slow down.
 
-// Bin of a cell within the scene; outside the range the group's.  The groups' bins lie behind blocks of
+// Bin of a cell; outside the range the group's.  The groups' bins lie behind blocks of
 // cells' bins, 2^binSpare to each: particles far out list slowly and sweep fast, so they are spread over
 // the scene (behind all cells they are one XCD's: list build of 8M sprayed particles 2.35 -> 3.32 ms).
 __device__ __forceinline__ uint32_t cell_bin(int cx, int cy, int cz, uint32_t group, const SceneDev& sc) {
@@ -758,8 +758,8 @@ __global__ __launch_bounds__(kBlock) void k_tally_count(DeviceState d, SphParams
         return;
     }
     const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
-    const SceneDev& sc = d.scenes[d.chunkScene[min(p, d.nslots - 1u) >> 8]];
-    const bool valid = p < d.nslots && p < sc.end;
+    const SceneDev& sc = d.scenes[0];
+    const bool valid = p < d.nslots;
     uint32_t h = 0, k = 0, group = 0, bin = kEmptyKey;
     if (valid) {
         k = d.lid[p];
@@ -768,10 +768,9 @@ __global__ __launch_bounds__(kBlock) void k_tally_count(DeviceState d, SphParams
         discretize(xs, P.cellHash, cx, cy, cz);
         h = cell_hash(cx, cy, cz, sc);
         group = h >> sc.groupShift;
-        bin = cell_bin(cx, cy, cz, group, sc) + sc.binBegin;
-        group += sc.groupBegin;
+        bin = cell_bin(cx, cy, cz, group, sc);
     }
-    // by runs of one bin and group (particles of a cell mostly lie side by side; a wave is of one scene)
+    // by runs of one bin and group (particles of a cell mostly lie side by side)
     const uint32_t lane = __lane_id();
     const uint32_t bin1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)bin, 0x138, 0xF, 0xF, false);  // wave_shr:1
     const uint64_t heads = __ballot(lane == 0u || bin1 != bin);
@@ -834,33 +833,31 @@ __global__ __launch_bounds__(kTallyThreads) void k_tally_prefix(DeviceState d) {
 __global__ __launch_bounds__(kBlock) void k_tally_place(DeviceState d) {
     const uint32_t p = blockIdx.x * kBlock + threadIdx.x;
     if (p >= d.nslots) return;
-    const SceneDev& sc = scene_of(d, p);
-    if (p >= sc.end) return;
     const uint4 r = d.tallied[p];
-    const uint32_t q = d.tallyBase[sc.groupBegin + (r.x >> sc.groupShift)] + r.z;
+    const uint32_t q = d.tallyBase[r.x >> d.scenes[0].groupShift] + r.z;
     if (q < d.nslots) d.placed[q] = make_uint4(r.x, r.y, p, r.w);
 }
 
 // kCarry, kCarryDelta: as in k_gather.  The first crowdBlocks workgroups take the crowded groups.
 template <bool kCarry, bool kCarryDelta>
-__global__ __launch_bounds__(kBlock) void k_tally_rank(DeviceState d, StepParams S, uint32_t nparticles, uint32_t crowdBlocks) {
+__global__ __launch_bounds__(kBlock) void k_tally_rank(DeviceState d, StepParams S, uint32_t crowdBlocks) {
     if (blockIdx.x < crowdBlocks) {
-        crowd_groups<kCarry, kCarryDelta, true>(d, S, d.tallyBase, d.tallyGroups, nparticles, crowdBlocks, crowd_lds());
+        crowd_groups<kCarry, kCarryDelta, true>(d, S, d.tallyBase, d.tallyGroups, d.nslots, crowdBlocks, crowd_lds());
         return;
     }
     const uint32_t q = (blockIdx.x - crowdBlocks) * kBlock + threadIdx.x;
-    if (q >= nparticles) return;
+    if (q >= d.nslots) return;
     const uint4 me = d.placed[q];
     const uint32_t h = me.x, k = me.y, src = me.z, bin = me.w;
     if (src >= d.nslots) return;  // consistent counts never produce this
-    const SceneDev& sc = scene_of(d, src);
-    const uint32_t group = sc.groupBegin + (h >> sc.groupShift);
+    const SceneDev& sc = d.scenes[0];
+    const uint32_t group = h >> sc.groupShift;
     if (group >= d.tallyGroups || d.tallyGroups + bin >= d.tallyCount) return;  // nor this
     const float4 x = d.X[src], v = d.V[src];
     const uint32_t id = d.id[src];
-    const uint32_t b = d.tallyBase[group], e = min(d.tallyBase[group + 1u], nparticles);
+    const uint32_t b = d.tallyBase[group], e = min(d.tallyBase[group + 1u], d.nslots);
     if (e - b > kCrowd) return;
-    const uint32_t binFirst = d.tallyBase[d.tallyGroups + bin] - nparticles;
+    const uint32_t binFirst = d.tallyBase[d.tallyGroups + bin] - d.nslots;
     // among the group: smaller hashes, the bucket, those of it before this particle, those of it in the same
     // bin, and those in the same bin before this particle by hash and index
     uint32_t smaller = 0, same = 0, sameBefore = 0, sameBin = 0, binBefore = 0;
@@ -880,8 +877,7 @@ __global__ __launch_bounds__(kBlock) void k_tally_rank(DeviceState d, StepParams
             binBefore += (less || before) && mine ? 1u : 0u;
         }
     }
-    const uint32_t shift = sc.begin - sc.first;  // slots of earlier scenes' padding
-    const uint32_t first = b + smaller + shift, to = first + sameBefore, p = binFirst + binBefore + shift;
+    const uint32_t first = b + smaller, to = first + sameBefore, p = binFirst + binBefore;
     if (to >= sc.end || p >= sc.end) return;  // consistent counts never produce this
     if (sameBefore == 0u) {
         const uint32_t slot = table_insert(d.table, sc, h);
@@ -3046,13 +3042,13 @@ void launch_tally(hipStream_t st, const DeviceState& d, const SphParams& P, cons
     k_tally_sum<<<prefix, kTallyThreads, 0, st>>>(d);
     k_tally_prefix<<<prefix, kTallyThreads, 0, st>>>(d);
     k_tally_place<<<count, kBlock, 0, st>>>(d);
-    const uint32_t rank = grid(d.nparticles), crowd = crowd_blocks(d.tallyGroups);
+    const uint32_t crowd = crowd_blocks(d.tallyGroups);
     if (carryDelta)
-        k_tally_rank<true, true><<<crowd + rank, kBlock, 0, st>>>(d, S, d.nparticles, crowd);
+        k_tally_rank<true, true><<<crowd + count, kBlock, 0, st>>>(d, S, crowd);
     else if (carry)
-        k_tally_rank<true, false><<<crowd + rank, kBlock, 0, st>>>(d, S, d.nparticles, crowd);
+        k_tally_rank<true, false><<<crowd + count, kBlock, 0, st>>>(d, S, crowd);
     else
-        k_tally_rank<false, false><<<crowd + rank, kBlock, 0, st>>>(d, S, d.nparticles, crowd);
+        k_tally_rank<false, false><<<crowd + count, kBlock, 0, st>>>(d, S, crowd);
 }
 void launch_bucket_phys(hipStream_t st, const DeviceState& d) {
     k_bucket_phys<<<grid(d.nslots), kBlock, 0, st>>>(d);

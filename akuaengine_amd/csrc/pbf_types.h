@@ -20,9 +20,8 @@ struct SceneDev {
     uint32_t modMagic;     // x % tableSize by multiply-high (fast_mod below)
     uint32_t modShift;
     uint32_t first;        // particles of the scenes before this one
-    // ordering by counting (launch_tally): the scene's groups of hashes and bins of cells, among all
-    uint32_t groupBegin, groupShift;
-    uint32_t binBegin;
+    // ordering of a single scene by counting (launch_tally): its groups of hashes and bins of cells
+    uint32_t groupShift;
     uint32_t binBlock, binSpare;  // log2 of the cells' bins in a block, of the groups' bins behind it
     int32_t binOrigin[3];      // cell coordinates of the range's lowest cell
     uint32_t binCells[3];      // cells per axis, whole cubes of 2^cubeLog2

@@ -325,7 +325,6 @@ struct akua_solver {
     DeviceState devState(bool keepLayout = false) {
         DeviceState d{};
         d.nslots = nslots;
-        d.nparticles = nparticles;
         d.scenes = dScenes.p;
         d.chunkScene = dChunkScene.p;
         d.X = X.p; d.V = V.p; d.dens = dens.p; d.lam = lam.p; d.id = id.p;
@@ -555,7 +554,6 @@ void setup(akua_solver* s, const std::vector<uint32_t>& counts) {
             // groups likewise, and counters for four cells a slot
             SceneDev& sc = s->scenes[0];
             const uint32_t lg = std::max(6u, ceil_log2(((uint64_t)ns + 3u) / 4u));
-            sc.groupBegin = 0;
             sc.groupShift = (uint32_t)std::max(0, (int)ceil_log2(sc.tableSize) - (int)lg);
             s->tallyGroups = 1u << lg;
             const uint64_t room = (3ull * s->tallyGroups + 4ull * ns + kTallyBlock - 1) / kTallyBlock * kTallyBlock;
@@ -945,50 +943,39 @@ SortPlan make_plan(int bits, int digitBits) {
 // the previous logical order it also splits their buckets (a key's cells then interleave).
 constexpr int kLayoutMarginCells = 4;
 
-// The scenes' bins of launch_tally: the cells of the box and kLayoutMarginCells beyond each wall, in cubes
+// The bins of launch_tally: the cells of the box and kLayoutMarginCells beyond each wall, in cubes
 // of 16^3 cells (32,000 particles, whose data an XCD's cache holds; 8^3 in thin boxes), the longest axis slowest.
 void update_bins(akua_solver* s) {
-    uint64_t bins = 0;
-    for (SceneDev& sc : s->scenes) {
-        uint64_t cells[3];
-        int axis[3] = {0, 1, 2};
-        for (int a = 0; a < 3; ++a) {
-            const double lo = std::floor((double)sc.bmin[a] / s->sph.cellHash) - (double)kLayoutMarginCells;
-            const double hi = std::floor((double)sc.bmax[a] / s->sph.cellHash) + (double)kLayoutMarginCells;
-            sc.binOrigin[a] = (int32_t)std::min(std::max(lo, -1e9), 1e9);
-            cells[a] = (uint64_t)std::min(std::max(hi - lo + 1.0, 1.0), 1e9);
-        }
-        sc.cubeLog2 = std::min({cells[0], cells[1], cells[2]}) < 32 ? 3u : 4u;
-        std::sort(axis, axis + 3, [&](int a, int b) { return cells[a] < cells[b]; });
-        double cubes = 1.0;  // at most 2^90: compared as a double
-        uint64_t stride = 1;
-        for (int a : axis) {
-            const uint64_t c = (cells[a] + (1u << sc.cubeLog2) - 1u) >> sc.cubeLog2;
-            sc.binCells[a] = (uint32_t)(c << sc.cubeLog2);
-            sc.cubeStride[a] = (uint32_t)stride;
-            cubes *= (double)c;
-            stride *= c;
-            if (cubes > 1e9) stride = 0;
-        }
-        sc.binBegin = (uint32_t)bins;
-        // some 64 blocks of cells' bins, each with its share of the groups' bins behind it
-        const double b = cubes * (double)(1u << (3u * sc.cubeLog2));
-        if (b > 2e9) {
-            bins = UINT64_MAX;
-            break;
-        }
+    if (s->tallyRoom == 0) return;
+    SceneDev& sc = s->scenes[0];
+    uint64_t cells[3];
+    int axis[3] = {0, 1, 2};
+    for (int a = 0; a < 3; ++a) {
+        const double lo = std::floor((double)sc.bmin[a] / s->sph.cellHash) - (double)kLayoutMarginCells;
+        const double hi = std::floor((double)sc.bmax[a] / s->sph.cellHash) + (double)kLayoutMarginCells;
+        sc.binOrigin[a] = (int32_t)std::min(std::max(lo, -1e9), 1e9);
+        cells[a] = (uint64_t)std::min(std::max(hi - lo + 1.0, 1.0), 1e9);
+    }
+    sc.cubeLog2 = std::min({cells[0], cells[1], cells[2]}) < 32 ? 3u : 4u;
+    std::sort(axis, axis + 3, [&](int a, int b) { return cells[a] < cells[b]; });
+    double cubes = 1.0;  // at most 2^90: compared as a double
+    uint64_t stride = 1;
+    for (int a : axis) {
+        const uint64_t c = (cells[a] + (1u << sc.cubeLog2) - 1u) >> sc.cubeLog2;
+        sc.binCells[a] = (uint32_t)(c << sc.cubeLog2);
+        sc.cubeStride[a] = (uint32_t)stride;
+        cubes *= (double)c;
+        stride *= c;
+        if (cubes > 1e9) stride = 0;
+    }
+    // some 64 blocks of cells' bins, each with its share of the groups' bins behind it
+    uint32_t count = 0;
+    const double b = cubes * (double)(1u << (3u * sc.cubeLog2));
+    if (b <= 2e9) {
         sc.binBlock = std::max(12u, ceil_log2(((uint64_t)b + 63u) / 64u));
         const uint64_t blocks = (((uint64_t)b - 1u) >> sc.binBlock) + 1u;
-        const uint32_t groups = 1u << std::max(6u, ceil_log2(((uint64_t)(sc.end - sc.begin) + 3u) / 4u));
-        sc.binSpare = ceil_log2((groups + blocks - 1) / blocks);
-        bins += blocks * ((1ull << sc.binBlock) + (1ull << sc.binSpare));
-        if (bins > s->tallyRoom) {
-            bins = UINT64_MAX;
-            break;
-        }
-    }
-    uint32_t count = 0;
-    if (bins != UINT64_MAX) {
+        sc.binSpare = ceil_log2((s->tallyGroups + blocks - 1) / blocks);
+        const uint64_t bins = blocks * ((1ull << sc.binBlock) + (1ull << sc.binSpare));
         const uint64_t c = ((uint64_t)s->tallyGroups + bins + 1u + kTallyBlock - 1u) / kTallyBlock * kTallyBlock;
         if (c <= s->tallyRoom) count = (uint32_t)c;
     }
