@@ -210,6 +210,8 @@ struct alignas(16) GradLds {
 };
 static_assert(sizeof(GradLds) <= 65536, "one workgroup's LDS");
 
+typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
+
 __device__ __forceinline__ bf16x4 lds4(const uint16_t* p) { return *reinterpret_cast<const bf16x4*>(p); }
 
 __device__ __forceinline__ f32x4 mma(bf16x4 a, bf16x4 b, f32x4 c) {
@@ -305,7 +307,10 @@ __global__ __launch_bounds__(64 * kMlpGradWaves) void k_mlp_grad(const float* __
         float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f), tg = f;
         if (row < n) {
             f = *reinterpret_cast<const float4*>(feat + (size_t)row * kMlpIn + 4 * g);
-            if (g == 0) tg = *reinterpret_cast<const float4*>(targ + (size_t)row * kMlpOut);
+            if (g == 0) {  // the caller's array, of which only a float's alignment is asked
+                const f32x4a4 v = *reinterpret_cast<const f32x4a4*>(targ + (size_t)row * kMlpOut);
+                tg = make_float4(v[0], v[1], v[2], v[3]);
+            }
         }
         __syncthreads();  // the weights are in LDS; the round before has read its rows
         const bf16x4 x = row < n ? pack_bf16((f.x - mean[0]) * inv[0], (f.y - mean[1]) * inv[1],

@@ -323,10 +323,11 @@ akua_status akua_mlp_adam_step(float* params, float* m, float* v, int64_t t, flo
  * for callers that cannot allocate device memory (code under HIP graph capture, tight training or
  * serving loops).  params, m, v, features, targets (n rows) and loss are device pointers, updated
  * as akua_mlp_adam_step updates them; lossWeights is host memory read during the call.  The work
- * is enqueued on `stream` (NULL: the null stream) and the call returns without waiting.  The
- * gradient partials live in one fixed array of the library per device, 256 x 5509 floats
- * (5.64 MB, held until the process ends), whatever n is, so no n is refused for its size; every
- * call rewrites all of it, and calls that overlap on one device race on it. */
+ * is enqueued on `stream` (NULL: the null stream) and the call returns without waiting.  features
+ * begin at a multiple of 16 bytes, the other arrays at any float.  The gradient partials live in
+ * one fixed array of the library per device, 256 x 5509 floats (5.64 MB, held until the process
+ * ends), whatever n is, so no n is refused for its size; a call writes the rows that it reads (one
+ * per 64 rows of features, at most 256), and calls that overlap on one device race on them. */
 akua_status akua_mlp_adam_step_device(float* params, float* m, float* v, int64_t t,
                                       float learningRate, const float* features,
                                       const float* targets, int32_t n, const float lossWeights[4],
