@@ -157,7 +157,6 @@ void launch_gather(hipStream_t st, const DeviceState& d, const SphParams& P, con
                    bool carry, bool carryDelta, bool layoutPrev);
 // Physical start and contiguity of every bucket (after the gather).
 void launch_bucket_phys(hipStream_t st, const DeviceState& d);
-// phys[lid[p]] = p over every scene's slots.
 // Larger single scenes whose boxes have not many more cells than particles: the same in five launches,
 // with the cell order in memory.  kTallyBlock counters per workgroup of the prefix.
 constexpr uint32_t kTallyBlock = 8192;
@@ -182,11 +181,10 @@ void launch_balance(hipStream_t st, const DeviceState& d, const SphParams& P, ui
 void launch_count_sum(hipStream_t st, const DeviceState& d, unsigned long long* part, uint32_t blocks);
 // residSlot >= 0: also the per-scene max and sum of max(0, C) into check residSlot of d.resid.
 // gated: only scenes whose d.gate is set run (the fallback's iterations).
-// lanes (4, 8 or 16; 1: one thread per particle): a lane group per particle in the neighbour
-// sweeps, for scenes too small to fill the chip, with results identical to one lane per particle;
-// only for plain steps (residSlot -1, no gate), the physical order and no wall samples.
-// lanes of a sweep: one per particle, or one that shares the long lists of its wave (plain steps in the
-// physical order without wall samples), or a group of 2 to 16.
+// lanes of a sweep: one per particle (1), or a group of 2 to 16 per particle, for scenes too small to fill the
+// chip (plain steps, residSlot -1 and no gate, in the physical order, with or without wall samples), or, in the
+// position deltas, one that shares the long lists of its wave (kLanesShared; such steps without wall samples).
+// The results are the same.
 constexpr int kLanesShared = 0;
 void launch_density_lambda(hipStream_t st, const DeviceState& d, const SphParams& P,
                            const float4* Xs, int bs, int residSlot = -1, bool gated = false,

@@ -964,8 +964,8 @@ __device__ __forceinline__ bool table_find(const uint4* __restrict__ table, cons
 }
 
 // kernel_find_neighbours (NeighbourSearchCUDA.cu:72-130), one thread per particle: for lists too long
-// for k_neighbours_wave's rows.  Stencil cells in (dx, dy, dz) order, each bucket walked in logical order, self skipped, r^2 < h^2 kept, at most maxNeighbours.  A
-// bucket reached from two stencil cells with equal hashes is walked twice, as in the reference.
+// for k_neighbours_wave's rows.  Stencil cells in (dx, dy, dz) order, each bucket walked in logical
+// order, self skipped, r^2 < h^2 kept, at most maxNeighbours.  A bucket reached from two stencil cells with equal hashes is walked twice, as in the reference.
 // The list stores physical slots.
 //
 // The walk is latency-bound, so memory requests are issued in batches: the nine table probes of
@@ -1082,7 +1082,8 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(DeviceState d, SphParams 
 //      each particle of the run (its position in scalar registers) is tested against all 64 at once:
 //      the accepted lanes' ranks in the ballot are their positions behind the particle's entries so
 //      far, in stream order;
-//   3. entries gather in LDS, one row per particle, and leave as whole 16-byte chunks.
+//   3. entries gather in LDS, one row per particle, and leave as whole 16-byte chunks;
+//   4. once all lists of a run are full, the stream goes on at the next run's first candidates.
 // With one thread per particle a wave walks 27 buckets per lane, for as long as its lane with most
 // candidates, and appends under eight masks per batch; here probes and candidate loads are made once
 // per run, every lane of a test does work, and lists of uneven length cost no idle lanes.
@@ -1096,7 +1097,8 @@ __global__ __launch_bounds__(kBlock) void k_neighbours(DeviceState d, SphParams 
 constexpr uint32_t kWaveRuns = 4;              // runs probed together
 constexpr uint32_t kWaveWindow = 2048;         // stream positions per bitmap
 constexpr int kWaveBuildBlock = 256;
-// Longest lists of which eight, or two, rows per wave fit in a workgroup's 64 KB of LDS.
+// Longest lists that are built with eight, or two, rows per wave: 47 KB of LDS a workgroup at 320, so that
+// three share a CU's 160 KB, and 63 of the 64 KB that a workgroup can have at 1,792.
 constexpr int kWaveBuildMaxN8 = 320, kWaveBuildMaxN2 = 1792;
 
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
@@ -2345,9 +2347,8 @@ __global__ __launch_bounds__(kTailBlock) void k_delta_correct_tail(DeviceState d
 
 // ---- work queue: the sweeps as persistent kernels over 256-slot tiles, heaviest first -------
 // A batch of uneven scenes (and the uneven lists of one scene) leave each sweep's last waves
-// running on a few CUs.  With the work queue, the tiles of each XCD's contiguous range (the range
-// xcd_slot gives it) are ordered by the sum of their neighbour counts, heaviest first, once per
-// step after the list build; each sweep then runs a resident grid whose workgroups take tiles of
+// running on a few CUs.  With the work queue, each XCD has a contiguous eighth of the tiles, ordered by
+// the sum of their neighbour counts, heaviest first, once per step after the list build; each sweep then runs a resident grid whose workgroups take tiles of
 // their XCD's queue until it is empty: in the dynamic mode the next free position (through
 // counters), in the static mode every R-th position from their own rank (R resident workgroups
 // per XCD).  Which workgroup runs which tile decides nothing: every slot is computed as in the

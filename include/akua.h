@@ -8,9 +8,12 @@
  * Here the solver owns its device memory, runs headless, and every call returns an akua_status.
  * No C++ exception crosses the ABI.  Signatures use only plain C types and pointers.
  *
- * Threading: one solver runs on one HIP stream.  Calls on one solver must be serialised by the
- * caller; different solvers may be used from different threads.  akua_solver_step() is
- * asynchronous with respect to the host; every get/debug call synchronises the solver's stream.
+ * Threading: a solver's work is in the order of the calls.  It runs on a HIP stream of the solver's
+ * own, except for akua_solver_step_device, which runs on the caller's stream, behind the solver's
+ * earlier work on any stream.  Calls on one solver must be serialised by the caller, from whichever
+ * threads; different solvers may be used from different threads at the same time.
+ * akua_solver_step() is asynchronous with respect to the host; every get/debug call waits for the
+ * solver's work.
  */
 #ifndef AKUA_H
 #define AKUA_H

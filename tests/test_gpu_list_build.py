@@ -35,7 +35,7 @@ def _check(gpu, oracle_mod, cfg, corr, pos, lo, hi):
     return cnt
 
 
-# wave sizes change at 2^16, 2^17 and 2^19 slots
+# wave sizes change at 2^13 (below), 2^17 and 2^19 slots
 @pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 63, 65, 257, 4099, 65535, 65537, 131071, 131073, 524287, 524289])
 def test_counts_around_the_wave_sizes(gpu, oracle_mod, dam_params, n):
     from akuaengine_amd import scenes
@@ -70,3 +70,13 @@ def test_shared_buckets_and_search_cells(gpu, oracle_mod, dam_params):
     for over in (dict(maxNeighbours=1), dict(maxNeighbours=2), dict(spatialHashCellSize=0.13),
                  dict(spatialHashCellSize=0.07, maxNeighbours=40)):
         _check(gpu, oracle_mod, dataclasses.replace(cfg, **over), corr, pos, (0.0, 0.0, 0.0), (2.0, 2.0, 2.0))
+
+
+@pytest.mark.parametrize("n", [8191, 8192, 8193])
+def test_counts_around_the_smallest_waves(gpu, oracle_mod, dam_params, n):
+    """Waves of four slots below 2^13, of eight from there on."""
+    from akuaengine_amd import scenes
+    cfg, corr = dam_params
+    sc = scenes.batched_scene(n, index=n % 7)
+    print(f"[list build] n={n}", flush=True)
+    _check(gpu, oracle_mod, cfg, corr, sc.pos, sc.box_min, sc.box_max)
