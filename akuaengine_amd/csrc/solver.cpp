@@ -177,6 +177,7 @@ struct PinnedRing {
     std::mutex use;
     char* p = nullptr;
     size_t bytes = 0;
+    bool made = false;  // at some time
     int solvers = 0;
 };
 PinnedRing g_ring;
@@ -310,7 +311,7 @@ struct akua_solver {
     // record export staging (get_particles), allocated on first use
     DevBuf<AosParticle> aosStage;
     // the read-backs of get_state, get_particles and render: whether this solver counts among g_ring's, an event
-    // for each chunk's last copy, and whether there has been a small read-back
+    // for each chunk's last copy, and whether there has been a read-back that wanted a ring
     bool usesRing = false, readBefore = false;
     std::vector<hipEvent_t> chunkReady;
 
@@ -1272,15 +1273,17 @@ struct Readback {
 constexpr size_t kReadbackInline = 4u << 20, kReadbackPerThread = 2u << 20;
 constexpr unsigned kReadbackThreads = 8;
 
-// Whether this read-back passes through the ring, whose lock the caller holds.  A solver's first small one
-// does not make the ring: a program that reads or draws once would only pay for it (27,000 particles: 0.19 ms
-// without, 0.17 with the ring and 0.3 for making it).
+// Whether this read-back passes through the ring, whose lock the caller holds.  The process's first one makes it
+// (whatever comes first waits some 7 ms for the copy engine).  After the last solver has given it back, a solver's
+// first one of up to kReadbackInline bytes does without: a program that reads or draws once per solver would pay
+// 0.45 ms and more for it.  Later ones are worth it: a state of 1.1 MB takes 0.17 ms with the ring and 0.13 to 0.67
+// without, by where the caller's memory comes from.
 bool take_ring(akua_solver* s, size_t total) {
-    const bool first = !s->readBefore;
-    s->readBefore = true;
     const size_t want = total <= kReadbackInline ? kRingSmall : kRingLarge;
     if (g_ring.bytes < want) {
-        if (first && total <= kReadbackInline) return false;
+        const bool first = !s->readBefore;
+        s->readBefore = true;
+        if (g_ring.made && first && total <= kReadbackInline) return false;
         void* p = nullptr;
         if (hipHostMalloc(&p, want, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
@@ -1289,6 +1292,7 @@ bool take_ring(akua_solver* s, size_t total) {
         if (g_ring.p) (void)hipHostFree(g_ring.p);
         g_ring.p = static_cast<char*>(p);
         g_ring.bytes = want;
+        g_ring.made = true;
     }
     if (!s->usesRing) {
         s->usesRing = true;
