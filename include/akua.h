@@ -153,7 +153,7 @@ typedef struct akua_tuning {
     int32_t layoutLevel;      /* physical layout: super-cells of 2^level hash cells per axis, 0..3.
                                  1 (the default) with the next three at their defaults too leaves the
                                  layout to the solver: the logical order in small single scenes, else
-                                 single cells */
+                                 single cells; with any of them set, 1 is super-cells of 2^3 cells */
     int32_t hashDigitBits;    /* radix digit width of the hash sort: 0 (balanced) or 5..8 */
     int32_t layoutDigitBits;  /* radix digit width of the layout sort: 0 (balanced) or 5..8 */
     int32_t layoutInterval;   /* the physical layout is re-sorted every layoutInterval steps (1..8);
