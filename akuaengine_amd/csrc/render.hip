@@ -4,12 +4,13 @@
 // fluidParticle.vert: gl_PointSize = size / |world - camera|; fluidParticle.frag: discard where
 // |gl_PointCoord - 0.5| > 0.5, colour * exp(-3 d^2)) over a floor mesh (floor.frag: checker of
 // floor(x) + floor(z)), depth test GL_LESS, particles in buffer order.  Here:
-//   k_render_clear   every pixel key to the maximum (no sprite);
-//   k_render_splat   one thread per particle: the clip-volume test of a GL point, the sprite
-//                    square, and for each fragment centre inside the disc an atomic minimum of
-//                    (window depth bits << 32 | draw index) -- the smallest depth wins and, at
-//                    equal depth, the earlier particle in buffer order, which is what GL_LESS
-//                    keeps when the sprites are drawn in that order;
+//   k_render_clear   every pixel key to the maximum (no sprite), and the draw order's inverse;
+//   k_render_splat   one lane per particle: the clip-volume test of a GL point, the sprite
+//                    square, and by one or more lanes for each fragment centre inside the disc an
+//                    atomic minimum of (window depth bits << 32 | draw index) -- the smallest depth
+//                    wins and, at equal depth, the earlier particle in buffer order, which is what
+//                    GL_LESS keeps when the sprites are drawn in that order;
+//   k_render_huge    the same for the sprites that k_render_splat lists as too large for a wave;
 //   k_render_resolve one thread per pixel: the winning sprite's colour at this fragment, or the
 //                    floor where a ray through the pixel centre meets it nearer, or the clear
 //                    colour; written as RGB8 rows from the top.
